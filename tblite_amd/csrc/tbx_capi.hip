@@ -22,6 +22,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include "../../include/tbx.h"
+#include "tbx_eigen.h"
 #include "tbx_tables.h"
 
 // Default row atoms per band of the unit builders (build_units_list, the
@@ -63,6 +64,9 @@ extern "C" hipError_t tbx_launch_density(const TbxMols *mol, const double *C, co
 extern "C" hipError_t tbx_launch_fermi(const TbxMols *mol, const double *nel, double kt,
                                        const double *emo, double *occ, double *efermi,
                                        hipStream_t stream);
+extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, int nmol,
+                                       const EigWork *wk, double *H, const double *S, double *ev,
+                                       int *info, hipStream_t s);
 extern "C" hipError_t tbx_launch_ncoord(const TbxMols *mol, const double *rcov, double ka,
                                         double kb, double rshift, double cutoff,
                                         const double *xyz, double *cn, hipStream_t stream);
@@ -953,6 +957,15 @@ static std::vector<char> species_bytes(const tbx_basis *bas, const tbx_h0par *h0
     return r;
 }
 
+// Molecules of the batched eigensolver in descending order of size, cut into
+// launches whose matrices fit the workspace.
+struct EigPlan {
+    std::vector<EigMol> mols;
+    std::vector<int> n, first;   // sizes; first molecule of each launch, and the end
+    std::vector<int> large;      // molecules beyond TBX_EIG_MAXN
+    long long elems = -1;        // workspace elements per matrix (-1: no plan yet)
+};
+
 struct tbx_batch {
     tbx_context *ctx = nullptr;
     HostSpecies hs;
@@ -963,9 +976,11 @@ struct tbx_batch {
     DevBuf flag, dse_tmp;
     hipEvent_t ev[16] = {};  // pairs (start, end): forward, -, gradient, adjoint, 4 SCF kernels
     bool timed = false;
-    // generalized eigensolver (rocSOLVER): handle, copy of S, workspace, info
+    // generalized eigensolver: workspace, info, the molecules in descending
+    // order of size (host and device); handle of rocSOLVER for the others
     rocblas_handle solver = nullptr;
-    DevBuf sy_b, sy_e, sy_info;
+    DevBuf sy_b, sy_e, sy_info, sy_mols;
+    EigPlan eig;
     // coordination number: covalent radii per species (device) and constants
     DevBuf rcov;
     bool cn_set = false;
@@ -1425,7 +1440,7 @@ static int batch_create(tbx_context *ctx, const tbx_batch_desc *desc, const int 
     b->ctx = ctx;
     b->cutoff = desc->cutoff;
     for (DevBuf *d : {&b->tab.species, &b->tab.mols, &b->flag, &b->dse_tmp, &b->rcov, &b->sy_b,
-                      &b->sy_e, &b->sy_info})
+                      &b->sy_e, &b->sy_info, &b->sy_mols})
         d->budget = &ctx->budget;
     int st = build_species(desc->bas, desc->h0, b->hs);
     if (!st) st = build_mols(b->hs, desc->nmol, desc->mol_nat, desc->id, b->hm);
@@ -1746,6 +1761,7 @@ extern "C" void tbx_batch_delete(tbx_batch *b)
     b->sy_b.release();
     b->sy_e.release();
     b->sy_info.release();
+    b->sy_mols.release();
     if (b->solver) (void)rocblas_destroy_handle(b->solver);
     for (auto &ev : b->ev)
         if (ev) (void)hipEventDestroy(ev);
@@ -1979,43 +1995,168 @@ extern "C" int tbx_batch_ncoord_gradient(tbx_batch *b, const double *d_xyz,
     return TBX_OK;
 }
 
-// Density matrices of the SCF (scf/diag.f90:62-166, wavefunction/fermi.f90):
-// the generalized eigenproblem per molecule (rocSOLVER dsygvd, as the
-// reference's lapack/sygvd.f90 calls LAPACK's), the Fermi filling and the
-// density products on the device.
+// The eigenproblem of molecules that the batched kernels do not take, one
+// rocSOLVER call each (S is overwritten by its Cholesky factor: on a copy).
+static int sygvd_library(tbx_batch *b, const std::vector<int> &which, double *d_H,
+                         const double *d_S, double *d_eval, hipStream_t s)
+{
+    if (!b->solver && rocblas_create_handle(&b->solver) != rocblas_status_success)
+        return fail(TBX_ERR_DEVICE, "rocblas_create_handle failed");
+    if (rocblas_set_stream(b->solver, s) != rocblas_status_success)
+        return fail(TBX_ERR_DEVICE, "rocblas_set_stream failed");
+    size_t nn = 1;
+    for (int m : which) nn = std::max(nn, (size_t)b->hm.mol_nao[m] * b->hm.mol_nao[m]);
+    HIP_TRY(b->sy_b.reserve(sizeof(double) * nn));
+    HIP_TRY(b->sy_e.reserve(sizeof(double) * (size_t)std::max(1, b->hm.nao)));
+    for (int m : which) {
+        const int n = b->hm.mol_nao[m];
+        const long long d0 = b->hm.mol_dense[m];
+        const int a0 = b->hm.mol_ao[m];
+        HIP_TRY(hipMemcpyAsync(b->sy_b.p, d_S + d0, sizeof(double) * (size_t)n * n,
+                               hipMemcpyDeviceToDevice, s));
+        const rocblas_status st = rocsolver_dsygvd(
+            b->solver, rocblas_eform_ax, rocblas_evect_original, rocblas_fill_upper, n, d_H + d0,
+            n, b->sy_b.as<double>(), n, d_eval + a0, b->sy_e.as<double>() + a0,
+            b->sy_info.as<rocblas_int>() + m);
+        if (st != rocblas_status_success)
+            return fail(TBX_ERR_DEVICE, "rocsolver_dsygvd (molecule %d): status %d", m, (int)st);
+    }
+    return TBX_OK;
+}
+
+// Launches of the batched eigensolver: the molecules in descending order of
+// size, consecutive ones together while their matrices fit `elems` elements.
+static void eig_plan(const HostMols &hm, long long elems, EigPlan &p)
+{
+    p = EigPlan{};
+    p.elems = elems;
+    std::vector<int> order(hm.nmol);
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int a, int c) { return hm.mol_nao[a] > hm.mol_nao[c]; });
+    long long w = 0;
+    for (int m : order) {
+        const int n = hm.mol_nao[m];
+        if (n > TBX_EIG_MAXN) {
+            p.large.push_back(m);
+            continue;
+        }
+        const long long nn = (long long)n * n;
+        // a launch takes up to 32768 molecules (grid dimension)
+        if (p.first.empty() || w + nn > elems || (int)p.mols.size() - p.first.back() >= 32768) {
+            p.first.push_back((int)p.mols.size());
+            w = 0;
+        }
+        p.mols.push_back(EigMol{n, m, hm.mol_ao[m], hm.nao, w, hm.mol_dense[m]});
+        p.n.push_back(n);
+        w += nn;
+    }
+    p.first.push_back((int)p.mols.size());
+}
+
+// Workspace of the batched eigensolver.  A matrix of the workspace holds at
+// most 2^24 elements (128 MB; four of them), or the largest molecule: launches
+// over more molecules at a time gained nothing.  Less where the context's
+// memory limit asks for it; false: not even one molecule at a time fits.
+static bool eig_workspace(tbx_batch *b, EigWork &wk, hipError_t &err)
+{
+    const HostMols &hm = b->hm;
+    long long big = 1, sum = 0;
+    for (int n : hm.mol_nao)
+        if (n <= TBX_EIG_MAXN) {
+            big = std::max(big, (long long)n * n);
+            sum += (long long)n * n;
+        }
+    const size_t nao = (size_t)std::max(1, hm.nao);
+    const size_t vec = sizeof(double) * (14 * nao + hm.nmol) + sizeof(int) * 4 * nao;
+    long long want = std::max(big, std::min(sum, 1LL << 24));
+    err = hipSuccess;
+    for (;; want = std::max(big, want / 8)) {
+        const size_t bytes = sizeof(double) * 4 * (size_t)want + vec;
+        if (b->eig.elems == want && b->sy_b.cap >= bytes) break;
+        err = b->sy_b.reserve(bytes);
+        if (err == hipSuccess) break;
+        if (err != hipErrorOutOfMemory || want == big) return false;
+        (void)hipGetLastError();
+    }
+    if (b->eig.elems != want) {
+        eig_plan(hm, want, b->eig);
+        const size_t bytes = sizeof(EigMol) * std::max<size_t>(b->eig.mols.size(), 1);
+        err = b->sy_mols.reserve(bytes);
+        if (err == hipSuccess && !b->eig.mols.empty())
+            err = hipMemcpy(b->sy_mols.p, b->eig.mols.data(), sizeof(EigMol) * b->eig.mols.size(),
+                            hipMemcpyHostToDevice);
+        if (err != hipSuccess) {
+            b->eig.elems = -1;
+            return false;
+        }
+    }
+    double *p = b->sy_b.as<double>();
+    for (double *&m : wk.m) {
+        m = p;
+        p += want;
+    }
+    auto take = [&](size_t k) {
+        double *q = p;
+        p += k;
+        return q;
+    };
+    wk.d = take(nao);
+    wk.e = take(nao);
+    wk.tau = take(nao);
+    wk.p = take(2 * nao);
+    wk.ev = take(2 * nao);
+    for (double *&v : wk.v) v = take(nao);
+    wk.anorm = take(hm.nmol);
+    int *q = reinterpret_cast<int *>(p);
+    for (int *&v : wk.iv) {
+        v = q;
+        q += nao;
+    }
+    wk.stride = hm.nao;
+    return true;
+}
+
+// The generalized eigenproblem of every molecule (lapack/sygvd.f90,
+// scf/diag.f90:62-108): the batched kernels of tbx_eigen.hip for molecules of
+// up to TBX_EIG_MAXN orbitals (a strip of 16 columns has to fit LDS),
+// rocSOLVER's dsygvd molecule by molecule for larger ones, and for all where
+// the context's memory limit leaves no room for the kernels' workspace.
 extern "C" int tbx_batch_sygvd(tbx_batch *b, double *d_H, const double *d_S, double *d_eval,
                                void *stream)
 {
     if (!b || !d_H || !d_S || !d_eval) return fail(TBX_ERR_ARG, "null argument");
     hipStream_t s = pick_stream(b, stream);
     HIP_TRY(hipSetDevice(b->ctx->device));
-    if (!b->solver && rocblas_create_handle(&b->solver) != rocblas_status_success)
-        return fail(TBX_ERR_DEVICE, "rocblas_create_handle failed");
-    if (rocblas_set_stream(b->solver, s) != rocblas_status_success)
-        return fail(TBX_ERR_DEVICE, "rocblas_set_stream failed");
-    // S is overwritten by its Cholesky factor: solve on a copy
-    HIP_TRY(b->sy_b.reserve(sizeof(double) * (size_t)b->hm.ndense));
-    HIP_TRY(b->sy_e.reserve(sizeof(double) * (size_t)std::max(1, b->hm.nao)));
     HIP_TRY(b->sy_info.reserve(sizeof(rocblas_int) * (size_t)b->hm.nmol));
-    HIP_TRY(hipMemcpyAsync(b->sy_b.p, d_S, sizeof(double) * (size_t)b->hm.ndense,
-                           hipMemcpyDeviceToDevice, s));
-    for (int m = 0; m < b->hm.nmol; ++m) {
-        const int n = b->hm.mol_nao[m];
-        const long long d0 = b->hm.mol_dense[m];
-        const int a0 = b->hm.mol_ao[m];
-        const rocblas_status st = rocsolver_dsygvd(
-            b->solver, rocblas_eform_ax, rocblas_evect_original, rocblas_fill_upper, n, d_H + d0,
-            n, b->sy_b.as<double>() + d0, n, d_eval + a0, b->sy_e.as<double>() + a0,
-            b->sy_info.as<rocblas_int>() + m);
-        if (st != rocblas_status_success)
-            return fail(TBX_ERR_DEVICE, "rocsolver_dsygvd (molecule %d): status %d", m, (int)st);
+    EigWork wk{};
+    hipError_t err = hipSuccess;
+    std::vector<int> library;
+    if (eig_workspace(b, wk, err)) {
+        const EigPlan &p = b->eig;
+        for (size_t k = 0; k + 1 < p.first.size(); ++k) {
+            const int m0 = p.first[k];
+            HIP_TRY(tbx_launch_eigen(b->sy_mols.as<EigMol>() + m0, p.n.data() + m0,
+                                     p.first[k + 1] - m0, &wk, d_H, d_S, d_eval,
+                                     b->sy_info.as<int>(), s));
+        }
+        library = p.large;
+        // the copy of S of a large molecule needs the buffer the kernels use
+        if (!library.empty()) HIP_TRY(hipStreamSynchronize(s));
+    } else {
+        if (err != hipErrorOutOfMemory) HIP_TRY(err);
+        (void)hipGetLastError();
+        library.resize(b->hm.nmol);
+        std::iota(library.begin(), library.end(), 0);
     }
+    if (!library.empty())
+        if (int st = sygvd_library(b, library, d_H, d_S, d_eval, s)) return st;
     std::vector<rocblas_int> info(b->hm.nmol);
     HIP_TRY(hipMemcpyAsync(info.data(), b->sy_info.p, sizeof(rocblas_int) * info.size(),
                            hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     for (int m = 0; m < b->hm.nmol; ++m)
-        if (info[m] != 0)
+        if (info[m] != 0 && info[m] != TBX_EIG_NONFINITE)
             return fail(TBX_ERR_ARG, "sygvd failed for molecule %d (info %d): S not positive "
                                      "definite or no convergence", m, (int)info[m]);
     return TBX_OK;
