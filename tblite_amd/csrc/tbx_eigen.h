@@ -4,7 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #define TBX_EIG_MAXN 1024  /* most orbitals: a 16-column strip of the matrix fits LDS */
-#define TBX_TRD_LDS 128    /* trailing columns of the tridiagonal form held in LDS */
+#define TBX_TRD_TAIL 128   /* trailing columns of the tridiagonal form held in registers */
 #define TBX_EIG_NONFINITE (-1) /* info: H holds an infinity or NaN, the results are NaN */
 #define TBX_DC_LEAF 64     /* rows of a divide-and-conquer leaf */
 

@@ -9,8 +9,8 @@
 //                 L are kept as their inverses
 //   k_eig_trsm    Y = L^-1 H, then A = L^-1 Y^T: strips of 16 columns in LDS,
 //                 FP64 MFMA products with the 64 x 64 blocks of L
-//   k_trd_step    one Householder column of A per launch (n > TBX_TRD_LDS)
-//   k_trd_lds     the last TBX_TRD_LDS columns, the whole rest of A in LDS
+//   k_trd_step    one Householder column of A per launch (n > TBX_TRD_TAIL)
+//   k_trd_tail    the last TBX_TRD_TAIL columns, the whole rest of A in registers
 //   k_dc_leaf     eigenpairs of tridiagonal blocks of at most 64 rows by divide
 //                 and conquer from single rows, in LDS
 //   k_dc_prep, k_dc_secular, k_dc_zhat, k_dc_norm, k_dc_gemm
@@ -23,6 +23,8 @@
 // Matrices are column-major n x n at EigMol::w0 of the workspace buffers,
 // vectors at the molecule's first orbital a0.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 
 #include "tbx_eigen.h"
 
@@ -68,23 +70,66 @@ __device__ __forceinline__ double wsum(double v)
     return lane63(v);
 }
 
-// sums (and a product) over groups of LPR = 4 or 8 consecutive lanes, on all
-// of them: quad permutations, then the mirror of the half row
-template <int LPR>
-__device__ __forceinline__ double gsum(double v)
+// a and b folded into one register: lanes 0..31 hold the sum of the two halves
+// of a, lanes 32..63 that of b (fold32); rows 0 / 1 and 2 / 3 of 16 lanes
+// likewise (fold16)
+__device__ __forceinline__ double fold32(double a, double b)
+{
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32),
+                                                     false, false);
+    return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) +
+           __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+__device__ __forceinline__ double fold16(double a, double b)
+{
+    const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)y, false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(y >> 32),
+                                                     false, false);
+    return __longlong_as_double(((long long)hi[0] << 32) | lo[0]) +
+           __longlong_as_double(((long long)hi[1] << 32) | lo[1]);
+}
+
+__device__ __forceinline__ double lane_of(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_readlane((int)b, l);
+    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+// the four sums over the wavefront at once (a third of the instructions of
+// four wsum): after the folds each row of 16 lanes belongs to one of them
+__device__ __forceinline__ void wsum4(double s[4])
+{
+    double v = fold16(fold32(s[0], s[1]), fold32(s[2], s[3]));  // rows: s0, s2, s1, s3
+    v += dpp<0x128, 0xf>(v);  // rotations within the row
+    v += dpp<0x124, 0xf>(v);
+    v += dpp<0x122, 0xf>(v);
+    v += dpp<0x121, 0xf>(v);
+    s[0] = lane_of(v, 0);
+    s[2] = lane_of(v, 16);
+    s[1] = lane_of(v, 32);
+    s[3] = lane_of(v, 48);
+}
+
+// sums and a product over the four lanes of a quad, on all of them
+__device__ __forceinline__ double qsum(double v)
 {
     v += dpp<0xB1, 0xf>(v);
-    v += dpp<0x4E, 0xf>(v);
-    if (LPR == 8) v += dpp<0x141, 0xf>(v);
-    return v;
+    return v + dpp<0x4E, 0xf>(v);
 }
-template <int LPR>
-__device__ __forceinline__ double gprod(double v)
+__device__ __forceinline__ double qprod(double v)
 {
     v *= dpp<0xB1, 0xf>(v);
-    v *= dpp<0x4E, 0xf>(v);
-    if (LPR == 8) v *= dpp<0x141, 0xf>(v);
-    return v;
+    return v * dpp<0x4E, 0xf>(v);
+}
+__device__ __forceinline__ double qmax(double v)
+{
+    v = fmax(v, dpp<0xB1, 0xf>(v));
+    return fmax(v, dpp<0x4E, 0xf>(v));
 }
 
 // reciprocal to about one unit in the last place (finite, nonzero arguments)
@@ -134,13 +179,21 @@ __global__ void __launch_bounds__(256) k_eig_symm(const EigMol *mols, const doub
 constexpr int NB = 64;
 constexpr int PR = NB + 16;  // LDS row length (doubles), as in the density kernel
 
+// element (r, c) of an n x n matrix, zero outside
+__device__ __forceinline__ double ldg(const double *M, int n, int r, int c)
+{
+    return (r < n && c < n) ? M[r + (long long)c * n] : 0.0;
+}
+
 // Tile T[k][r] = M(r0 + r, c0 + k), zero outside n
 __device__ __forceinline__ void tile_load(double (*T)[PR], const double *M, int n, int r0, int c0)
 {
-    for (int e = threadIdx.x; e < NB * NB; e += 256) {
-        const int r = e & (NB - 1), k = e / NB;
-        T[k][r] = (r0 + r < n && c0 + k < n) ? M[(r0 + r) + (long long)(c0 + k) * n] : 0.0;
-    }
+    const int r = threadIdx.x & (NB - 1), k = threadIdx.x / NB;
+    double v[NB / 4];  // every load is under way before the first is stored
+#pragma unroll
+    for (int q = 0; q < NB / 4; ++q) v[q] = ldg(M, n, r0 + r, c0 + k + 4 * q);
+#pragma unroll
+    for (int q = 0; q < NB / 4; ++q) T[k + 4 * q][r] = v[q];
 }
 
 // D(r, c) = sum_k A(r, k) B(c, k) of 64 x 64 tiles T[k][row]: each of the four
@@ -187,8 +240,8 @@ __device__ __forceinline__ void tile_put(double (*T)[PR], int sr, int sc, const 
 // one broadcast of the pivot's column and row through LDS and one barrier.
 // Writes inv(L) (zero above the diagonal) to Linv (column-major, ld n) and
 // returns false if a pivot is not positive.
-__device__ bool factor_inverse(double (*T)[PR], double (*buf)[2 * NB], int nv, double *Linv,
-                               int n)
+__device__ bool factor_inverse(double (*T)[PR], double (*buf)[2 * NB], double *pivot, int nv,
+                               double *Linv, int n)
 {
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     double t[4][4], x[4][4];
@@ -201,7 +254,9 @@ __device__ bool factor_inverse(double (*T)[PR], double (*buf)[2 * NB], int nv, d
             x[a][b] = i == j ? 1.0 : 0.0;
         }
     bool ok = true;
-    double rs[4] = {1.0, 1.0, 1.0, 1.0};  // pivots of the rows ty + 16 a
+    if (tid < NB) pivot[tid] = 1.0;
+    // step k = 16 kb + kk changes the rows below k only: the columns from the
+    // block kb on in T (those before k are no longer used), up to it in X
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb)
         for (int kk = 0; kk < 16; ++kk) {
@@ -210,33 +265,38 @@ __device__ bool factor_inverse(double (*T)[PR], double (*buf)[2 * NB], int nv, d
             double *col = buf[k & 1], *row = buf[k & 1] + NB;
             if (tx == kk) {
 #pragma unroll
-                for (int a = 0; a < 4; ++a) col[ty + 16 * a] = t[a][kb];
+                for (int a = kb; a < 4; ++a) col[ty + 16 * a] = t[a][kb];
             }
             if (ty == kk) {
 #pragma unroll
-                for (int b = 0; b < 4; ++b) row[tx + 16 * b] = x[kb][b];
+                for (int b = 0; b <= kb; ++b) row[tx + 16 * b] = x[kb][b];
             }
             __syncthreads();
             const double piv = col[k];
+            if (tid == 0) pivot[k] = piv;
             ok = ok && piv > 0.0;
-            const double inv = 1.0 / piv;
+            const double inv = fast_rcp(piv);
+            double cj[4], rj[4];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
+            for (int b = kb; b < 4; ++b) cj[b] = col[tx + 16 * b];
+#pragma unroll
+            for (int b = 0; b <= kb; ++b) rj[b] = row[tx + 16 * b];
+#pragma unroll
+            for (int a = kb; a < 4; ++a) {
                 const int i = ty + 16 * a;
-                if (i == k) rs[a] = piv;
                 const double m = i > k ? col[i] * inv : 0.0;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    if (tx + 16 * b > k) t[a][b] -= m * col[tx + 16 * b];
-                    x[a][b] -= m * row[tx + 16 * b];
-                }
+                for (int b = kb; b < 4; ++b) t[a][b] -= m * cj[b];
+#pragma unroll
+                for (int b = 0; b <= kb; ++b) x[a][b] -= m * rj[b];
             }
         }
     if (!ok) return false;
+    __syncthreads();
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
         const int i = ty + 16 * a;
-        const double s = 1.0 / sqrt(rs[a]);
+        const double s = 1.0 / sqrt(pivot[i]);
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
             const int j = tx + 16 * b;
@@ -250,13 +310,13 @@ __device__ bool factor_inverse(double (*T)[PR], double (*buf)[2 * NB], int nv, d
 // P_i = A_ik inv(L_kk)^T (the block of L, stored by the tiles of column
 // kb + 1), A_ij -= P_i P_j^T; the tile (kb + 1, kb + 1) goes on to its own
 // factor and inverse, so a block column is one launch.  kb = -1: the first
-// diagonal block only.  Measured: one launch of a 768-orbital molecule (up to
-// 66 tiles) is bound by the elimination's chain of 64 barriers.
+// diagonal block only.  768 orbitals: 33 us a launch, about half of it the
+// chain of 64 eliminations (60 us with loads one at a time and unmasked rows).
 __global__ void __launch_bounds__(256) k_eig_chol(const EigMol *mols, double *A, double *L,
                                                   int kb, int *info)
 {
     __shared__ __align__(16) double T0[NB][PR], T1[NB][PR], T2[NB][PR];
-    __shared__ double buf[2][2 * NB];
+    __shared__ double buf[2][2 * NB], pivot[NB];
     const EigMol M = mols[blockIdx.y];
     const int n = M.n, nblk = (n + NB - 1) / NB, left = nblk - 1 - kb;
     if (left <= 0) return;
@@ -310,7 +370,7 @@ __global__ void __launch_bounds__(256) k_eig_chol(const EigMol *mols, double *A,
         __syncthreads();
     }
     const int b0 = NB * (kb + 1);
-    const bool ok = factor_inverse(kb < 0 ? T0 : T2, buf, min(NB, n - b0),
+    const bool ok = factor_inverse(kb < 0 ? T0 : T2, buf, pivot, min(NB, n - b0),
                                    Lm + b0 + (long long)b0 * n, n);
     if (!ok && threadIdx.x == 0) info[M.mol] = 1;
 }
@@ -319,11 +379,6 @@ __global__ void __launch_bounds__(256) k_eig_chol(const EigMol *mols, double *A,
 // triangular solves of 16-column strips in LDS: X[r][c], rows padded to 64
 
 constexpr int XS = 17;  // row length of the strip (doubles)
-
-__device__ __forceinline__ double ldg(const double *M, int n, int r, int c)
-{
-    return (r < n && c < n) ? M[r + (long long)c * n] : 0.0;
-}
 
 // X <- L^-1 X (forward) or L^-T X (backward) for the strip, block row by block
 // row: the four wavefronts take 16 rows each; the products with the earlier
@@ -379,14 +434,22 @@ __global__ void __launch_bounds__(256) k_eig_trsm(const EigMol *mols, const doub
     if (c0 >= n || info[M.mol] != 0) return;
     const int rows = (n + NB - 1) / NB * NB;
     const double *src = in + M.w0;
-    if (TRANS) {
-        for (int e = threadIdx.x; e < 16 * rows; e += 256) {
-            const int c = e & 15, r = e >> 4;
-            X[r * XS + c] = ldg(src, n, c0 + c, r);
+    // batches of 64 rows: four loads per thread under way at a time, sixteen
+    // with the unrolling
+#pragma unroll 4
+    for (int r0 = 0; r0 < rows; r0 += NB) {
+        double v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int e = threadIdx.x + 256 * q;
+            v[q] = TRANS ? ldg(src, n, c0 + (e & 15), r0 + (e >> 4))
+                         : ldg(src, n, r0 + (e & 63), c0 + (e >> 6));
         }
-    } else {
-        for (int c = 0; c < 16; ++c)
-            for (int r = threadIdx.x; r < rows; r += 256) X[r * XS + c] = ldg(src, n, r, c0 + c);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int e = threadIdx.x + 256 * q;
+            X[(r0 + (TRANS ? e >> 4 : e & 63)) * XS + (TRANS ? e & 15 : e >> 6)] = v[q];
+        }
     }
     __syncthreads();
     strip_solve<true>(L + M.w0, n, X);
@@ -437,69 +500,79 @@ __device__ __forceinline__ double block_sum4(double v, double *red)
     return red[0] + red[1] + red[2] + red[3];
 }
 
-// One column k of every molecule with n > TBX_TRD_LDS + k: workgroup
-// blockIdx.x takes the trailing columns k + 1 + TRD_COLS blockIdx.x ...; every
-// workgroup forms w, x and v_k itself (O(n) work), which saves a launch.
+// One column k of every molecule with n > TBX_TRD_TAIL + k (and n - k at most
+// 256 Q): workgroup blockIdx.x takes the trailing columns k + 1 + TRD_COLS
+// blockIdx.x ...; every workgroup forms w, x and v_k itself (O(n) work), which
+// saves a launch.  The launch is bound by its chain of dependent steps, so
+// the trailing columns are loaded before it begins: 4.3 / 5.1 / 6.0 us a column
+// at up to 256 / 512 / 768 rows, 7.3 us with the loads after the reflector.
+template <int Q>
 __global__ void __launch_bounds__(TRD_THREADS) k_trd_step(const EigMol *mols, TrdPtr T, int k)
 {
-    __shared__ double v[TBX_EIG_MAXN], w[TBX_EIG_MAXN], vn[TBX_EIG_MAXN];
+    constexpr int LEN = TRD_THREADS * Q;
+    __shared__ double v[LEN], w[LEN], vn[LEN];  // rows k ..
     __shared__ double red[2][4];
-    constexpr int Q = TBX_EIG_MAXN / TRD_THREADS;
     const EigMol M = mols[blockIdx.y];
-    const int n = M.n;
-    const int i0 = k + 1 + TRD_COLS * blockIdx.x;
-    if (n <= TBX_TRD_LDS + k || i0 >= n) return;
+    const int n = M.n, len = n - k;
+    const int i0 = 1 + TRD_COLS * blockIdx.x;  // columns and rows count from k
+    if (n <= TBX_TRD_TAIL + k || i0 >= len) return;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    double *A = T.A + M.w0, *V = T.V + M.w0;
-    const double *pold = T.p + ((k + 1) & 1) * T.pstride + M.a0;
-    double *pnew = T.p + (k & 1) * T.pstride + M.a0;
+    double *A = T.A + M.w0 + (long long)k * n + k, *V = T.V + M.w0 + (long long)k * n + k;
+    const double *pold = T.p + ((k + 1) & 1) * T.pstride + M.a0 + k;
+    double *pnew = T.p + (k & 1) * T.pstride + M.a0 + k;
     // the pending update of column k - 1: rows k.. of v and w
     double vr[Q], pr[Q], xr[Q];
     double s = 0.0, tau0 = 0.0;
+    if (k > 0) tau0 = T.tau[M.a0 + k - 1];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         const int i = tid + TRD_THREADS * q;
-        const bool in = i >= k && i < n;
-        vr[q] = (in && k > 0) ? V[i + (long long)(k - 1) * n] : 0.0;
-        pr[q] = (in && k > 0) ? pold[i] : 0.0;
-        xr[q] = in ? A[i + (long long)k * n] : 0.0;
-        s += vr[q] * pr[q];
+        vr[q] = (i < len && k > 0) ? V[i - n] : 0.0;
+        pr[q] = (i < len && k > 0) ? pold[i] : 0.0;
+        xr[q] = i < len ? A[i] : 0.0;
     }
-    if (k > 0) tau0 = T.tau[M.a0 + k - 1];
+    double a[TRD_COLS / 4][4 * Q];
+#pragma unroll
+    for (int c = 0; c < TRD_COLS / 4; ++c) {
+        const int i = i0 + wv + 4 * c;
+#pragma unroll
+        for (int q = 0; q < 4 * Q; ++q) {
+            const int j = 1 + lane + 64 * q;
+            a[c][q] = (i < len && j < len) ? A[(long long)i * n + j] : 0.0;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) s += vr[q] * pr[q];
     s = block_sum4(s, red[0]);
     const double h = 0.5 * tau0 * s;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         const int i = tid + TRD_THREADS * q;
         pr[q] = tau0 * (pr[q] - h * vr[q]);  // w
-        if (i >= k && i < n) {
-            v[i] = vr[q];
-            w[i] = pr[q];
-        }
+        v[i] = vr[q];
+        w[i] = pr[q];
     }
     __syncthreads();
-    const double vk = v[k], wk = w[k];
+    const double vk = v[0], wk = w[0];
     double xx = 0.0;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         const int i = tid + TRD_THREADS * q;
         xr[q] -= vr[q] * wk + pr[q] * vk;
-        if (i < n) vn[i] = xr[q];
-        if (i >= k + 2 && i < n) xx += xr[q] * xr[q];
+        vn[i] = xr[q];
+        if (i >= 2) xx += xr[q] * xr[q];
     }
     xx = block_sum4(xx, red[1]);
-    const double dk = vn[k], alpha = vn[k + 1];
+    const double dk = vn[0], alpha = vn[1];
     double beta, tau, scale;
     reflector(alpha, xx, beta, tau, scale);
-    __syncthreads();  // vn[k + 1] is read before it is replaced
+    __syncthreads();  // vn[1] is read before it is replaced
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         const int i = tid + TRD_THREADS * q;
-        if (i > k && i < n) {
-            const double x = i == k + 1 ? 1.0 : xr[q] * scale;
-            vn[i] = x;
-            if (blockIdx.x == 0) V[i + (long long)k * n] = x;
-        }
+        const double x = i == 1 ? 1.0 : xr[q] * scale;
+        vn[i] = x;
+        if (blockIdx.x == 0 && i > 0 && i < len) V[i] = x;
     }
     if (blockIdx.x == 0 && tid == 0) {
         T.d[M.a0 + k] = dk;
@@ -507,90 +580,100 @@ __global__ void __launch_bounds__(TRD_THREADS) k_trd_step(const EigMol *mols, Tr
         T.tau[M.a0 + k] = tau;
     }
     __syncthreads();
-    // update and product of this workgroup's trailing columns, one per wavefront
+    // update and product of this workgroup's trailing columns, two per wavefront
+    double acc[TRD_COLS / 4];
 #pragma unroll
     for (int c = 0; c < TRD_COLS / 4; ++c) {
         const int i = i0 + wv + 4 * c;
-        if (i >= n) break;
-        double *a = A + (long long)i * n;
-        const double vi = v[i], wi = w[i];
-        double acc = 0.0;
-        for (int j = k + 1 + lane; j < n; j += 64) {
-            const double x = a[j] - (vi * w[j] + wi * v[j]);
-            a[j] = x;
-            acc += x * vn[j];
+        const bool in = i < len;
+        const double vi = in ? v[i] : 0.0, wi = in ? w[i] : 0.0;
+        acc[c] = 0.0;
+#pragma unroll
+        for (int q = 0; q < 4 * Q; ++q) {
+            const int j = 1 + lane + 64 * q;
+            if (in && j < len) {
+                const double x = a[c][q] - (vi * w[j] + wi * v[j]);
+                A[(long long)i * n + j] = x;
+                acc[c] += x * vn[j];
+            }
         }
-        acc = wsum(acc);
-        if (lane == 0) pnew[i] = acc;
+    }
+#pragma unroll
+    for (int c = 0; c < TRD_COLS / 4; ++c) {
+        const double t = wsum(acc[c]);
+        const int i = i0 + wv + 4 * c;
+        if (lane == 0 && i < len) pnew[i] = t;
     }
 }
 
-// The remaining (at most TBX_TRD_LDS) columns in LDS, one workgroup per
-// molecule.  Each wavefront keeps the rows lane and lane + 64 of v, w and the
-// new reflector in registers and forms them redundantly, so a column costs one
-// barrier: after it every wavefront reads the column and p, then the
-// wavefronts take the trailing rows in turn.
-constexpr int TL_THREADS = 512;
-constexpr int TL = TBX_TRD_LDS;
-constexpr int TLD = TL + 1;
+// The remaining (at most TBX_TRD_TAIL) columns, one workgroup of four
+// wavefronts per molecule, with the whole rest of A in registers: lane and
+// lane + 64 are a thread's rows, the columns j = wave + 4 t are in a[.][t].
+// Each wavefront forms v, w and the new reflector redundantly, so a column
+// costs one barrier: before it the wavefronts leave their share of p = A v and
+// the next column (by symmetry the row of the lane that holds it) in LDS.  The
+// factors of column j are read from their lane (v_readlane).  Columns that are
+// done are still updated, eight at a time: their reflector entries are zero.
+// 1.7 us a column at 128 rows, 215 us in all; with A in LDS, eight wavefronts
+// and a reduction per row 378 us; in registers with a branch per column 375 us.
+constexpr int TL_THREADS = 256;
+constexpr int TL = TBX_TRD_TAIL;
+constexpr int TLT = TL / 4;  // columns per thread
 
-__global__ void __launch_bounds__(TL_THREADS) k_trd_lds(const EigMol *mols, TrdPtr T,
-                                                        const int *info)
+__global__ void __launch_bounds__(TL_THREADS) k_trd_tail(const EigMol *mols, TrdPtr T,
+                                                         double *anorm, int *info)
 {
-    extern __shared__ double sh[];
-    double *A = sh;                   // [TL][TLD]
-    double *pb = A + TL * TLD;        // [2][TL]
-    double *vb = pb + 2 * TL;         // [2][TL] v of the pending update
-    double *wb = vb + 2 * TL;         // [2][TL]
+    __shared__ double part[2][4][TL];  // p by wavefront
+    __shared__ double xcol[2][TL];     // the next column, pending update not applied
     const EigMol M = mols[blockIdx.x];
     const int n = M.n;
     if (info[M.mol] != 0) return;
     const int k0 = n > TL ? n - TL : 0, nt = n - k0;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    constexpr int NW = TL_THREADS / 64;
-    const double *Ag = T.A + M.w0;
-    double *V = T.V + M.w0;
-    for (int c = wv; c < nt; c += NW)
-        for (int r = lane; r < nt; r += 64) A[c * TLD + r] = Ag[(k0 + r) + (long long)(k0 + c) * n];
-    double v[2] = {0.0, 0.0}, p[2] = {0.0, 0.0}, w[2];
-    double tau = 0.0;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const double *Ag = T.A + M.w0 + (long long)k0 * n + k0;
+    double *V = T.V + M.w0 + (long long)k0 * n + k0;
+    double a[2][TLT];
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+        for (int t = 0; t < TLT; ++t) {
+            const int j = wv + 4 * t, r = lane + 64 * q;
+            a[q][t] = (r < nt && j < nt) ? Ag[r + (long long)j * n] : 0.0;
+        }
+    double v[2] = {0.0, 0.0}, p[2] = {0.0, 0.0}, w[2], x[2];
+    double tau = 0.0, mx = 0.0;
+    bool bad = false;
     if (k0 > 0) {
-        const double *pold = T.p + ((k0 + 1) & 1) * T.pstride + M.a0;
+        const double *pold = T.p + ((k0 + 1) & 1) * T.pstride + M.a0 + k0;
         tau = T.tau[M.a0 + k0 - 1];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const int r = lane + 64 * q;
             if (r < nt) {
-                v[q] = V[(k0 + r) + (long long)(k0 - 1) * n];
-                p[q] = pold[k0 + r];
+                v[q] = V[r - n];
+                p[q] = pold[r];
             }
         }
     }
-    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) x[q] = lane + 64 * q < nt ? Ag[lane + 64 * q] : 0.0;
     for (int k = 0; k < nt; ++k) {
-        // w of the pending update
+        // w of the pending update, then the column itself
         const double s = wsum(v[0] * p[0] + v[1] * p[1]);
         const double h = 0.5 * tau * s;
 #pragma unroll
         for (int q = 0; q < 2; ++q) w[q] = tau * (p[q] - h * v[q]);
-        double *vs = vb + (k & 1) * TL, *ws = wb + (k & 1) * TL;
-        // every wavefront writes the same values (and reads them itself)
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            vs[lane + 64 * q] = v[q];
-            ws[lane + 64 * q] = w[q];
-        }
-        const double vk = vs[k], wk = ws[k];
-        double x[2], xx = 0.0;
+        const double vk = lane_of(k < 64 ? v[0] : v[1], k & 63);
+        const double wk = lane_of(k < 64 ? w[0] : w[1], k & 63);
+        double xx = 0.0;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const int r = lane + 64 * q;
-            x[q] = (r >= k && r < nt) ? A[k * TLD + r] - (v[q] * wk + w[q] * vk) : 0.0;
+            x[q] = r >= k && r < nt ? x[q] - (v[q] * wk + w[q] * vk) : 0.0;
             if (r >= k + 2) xx += x[q] * x[q];
         }
-        // d_k and alpha = x[k + 1], read from their lanes
-        const double dk = __shfl(k < 64 ? x[0] : x[1], k & 63, 64);
-        const double alpha = __shfl(k + 1 < 64 ? x[0] : x[1], (k + 1) & 63, 64);
+        const double dk = lane_of(k < 64 ? x[0] : x[1], k & 63);
+        const double alpha = lane_of(k + 1 < 64 ? x[0] : x[1], (k + 1) & 63);
         xx = wsum(xx);
         double beta = 0.0, scale = 0.0;
         tau = 0.0;
@@ -599,44 +682,78 @@ __global__ void __launch_bounds__(TL_THREADS) k_trd_lds(const EigMol *mols, TrdP
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const int r = lane + 64 * q;
-            vn[q] = r <= k ? 0.0 : (r == k + 1 ? 1.0 : x[q] * scale);
-            if (r >= nt) vn[q] = 0.0;
+            vn[q] = r <= k || r >= nt ? 0.0 : (r == k + 1 ? 1.0 : x[q] * scale);
         }
         if (wv == 0) {
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const int r = lane + 64 * q;
-                if (r > k && r < nt) V[(k0 + r) + (long long)(k0 + k) * n] = vn[q];
+                if (r > k && r < nt) V[r + (long long)k * n] = vn[q];
             }
+            bad = bad || !(fabs(dk) < 1e300) || !(fabs(beta) < 1e300);
+            mx = fmax(mx, fmax(fabs(dk), fabs(beta)));
             if (lane == 0) {
                 T.d[M.a0 + k0 + k] = dk;
                 T.e[M.a0 + k0 + k] = beta;
                 T.tau[M.a0 + k0 + k] = tau;
             }
         }
-        double *pn = pb + (k & 1) * TL;
-        for (int i = k + 1 + wv; i < nt; i += NW) {
-            double *a = A + i * TLD;
-            const double vi = vs[i], wi = ws[i];
-            double acc = 0.0;
+        double acc[2] = {0.0, 0.0};
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                const int r = lane + 64 * q;
-                if (r > k && r < nt) {
-                    const double y = a[r] - (vi * w[q] + wi * v[q]);
-                    a[r] = y;
-                    acc += y * vn[q];
+        for (int b = 0; b < TLT / 8; ++b)
+            if (32 * b + 31 > k && 32 * b < nt) {  // uniform
+#pragma unroll
+                for (int t = 8 * b; t < 8 * b + 8; ++t) {
+                    const int j = (wv + 4 * t) & 63;
+                    const double vj = lane_of(v[t / 16], j), wj = lane_of(w[t / 16], j);
+                    const double nj = lane_of(vn[t / 16], j);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        a[q][t] -= v[q] * wj;
+                        a[q][t] -= w[q] * vj;
+                        acc[q] += a[q][t] * nj;
+                    }
                 }
             }
-            acc = wsum(acc);
-            if (lane == 0) pn[i] = acc;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) part[k & 1][wv][lane + 64 * q] = acc[q];
+        if (k + 1 < nt && lane == ((k + 1) & 63)) {  // row k + 1 of this wavefront's columns
+            double *xc = xcol[k & 1] + wv;
+            if (k + 1 < 64) {
+#pragma unroll
+                for (int t = 0; t < TLT; ++t) xc[4 * t] = a[0][t];
+            } else {
+#pragma unroll
+                for (int t = 16; t < TLT; ++t) xc[4 * t] = a[1][t];
+            }
         }
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const int r = lane + 64 * q;
             v[q] = vn[q];
-            p[q] = (r > k && r < nt) ? pn[r] : 0.0;
+            p[q] = x[q] = 0.0;
+            if (r > k && r < nt) {
+                p[q] = (part[k & 1][0][r] + part[k & 1][1][r]) +
+                       (part[k & 1][2][r] + part[k & 1][3][r]);
+                x[q] = xcol[k & 1][r];
+            }
+        }
+    }
+    // scale of the tridiagonal matrix (largest |d|, |e|); a matrix with a
+    // non-finite entry is marked: its results are NaN
+    if (wv == 0) {
+        for (int i = lane; i < k0; i += 64) {
+            const double di = T.d[M.a0 + i], ei = T.e[M.a0 + i];
+            bad = bad || !(fabs(di) < 1e300) || !(fabs(ei) < 1e300);
+            mx = fmax(mx, fmax(fabs(di), fabs(ei)));
+        }
+#pragma unroll
+        for (int s = 32; s >= 1; s >>= 1) mx = fmax(mx, __shfl_xor(mx, s, 64));
+        const bool any = __any(bad);
+        if (lane == 0) {
+            anorm[M.mol] = mx;
+            if (any) info[M.mol] = TBX_EIG_NONFINITE;
         }
     }
 }
@@ -656,9 +773,11 @@ __device__ __forceinline__ int dc_levels(int n)
 }
 
 // Root j of 1/rho + sum_i z_i^2 / (d_i - x) = 0, the j-th of K ascending
-// poles, by LPR lanes together: x = d[org] + tau.  Two-pole rational
-// interpolation of both partial sums (R.-C. Li, LAPACK working note 89), kept
-// inside a bracket by bisection.  The loop ends in at most 100 steps.
+// poles, by LPR lanes together (a quad, or the wavefront): x = d[org] + tau.
+// Rational interpolation at the two poles next to the root with the weight of
+// the nearer one fixed (R.-C. Li, LAPACK working note 89), kept inside a bracket
+// by bisection: 4 evaluations on average, about 10 for the slowest root.  The
+// loop ends in at most 100 steps.
 template <int LPR>
 __device__ __forceinline__ void secular_root(int K, const double *d, const double *z, double rho,
                                              int j, int sub, double &tau, int &org)
@@ -668,58 +787,66 @@ __device__ __forceinline__ void secular_root(int K, const double *d, const doubl
         tau = rho * z[0] * z[0];
         return;
     }
-    const double rhoinv = 1.0 / rho;
+    const double rhoinv = fast_rcp(rho);
     const bool last = j == K - 1;
     const int jl = last ? K - 2 : j;  // interpolation poles jl, jl + 1
     double psi, phi, dpsi, dphi, lo, hi;
     auto eval = [&](double dorg, double t) {
-        double s0 = 0.0, s1 = 0.0, g0 = 0.0, g1 = 0.0;
+        double s[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
         for (int i = sub; i < K; i += LPR) {
             const double zi = z[i];
             const double q = zi * fast_rcp((d[i] - dorg) - t);
-            if (i <= jl) {
-                s0 += zi * q;
-                g0 += q * q;
-            } else {
-                s1 += zi * q;
-                g1 += q * q;
-            }
+            const double q0 = i <= jl ? q : 0.0, q1 = q - q0;
+            s[0] += zi * q0;
+            s[1] += zi * q1;
+            s[2] += q0 * q0;
+            s[3] += q1 * q1;
         }
-        psi = gsum<LPR>(s0);
-        phi = gsum<LPR>(s1);
-        dpsi = gsum<LPR>(g0);
-        dphi = gsum<LPR>(g1);
+        if (LPR == 64) {
+            wsum4(s);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) s[k] = qsum(s[k]);
+        }
+        psi = s[0];
+        phi = s[1];
+        dpsi = s[2];
+        dphi = s[3];
     };
+    const double gap = d[jl + 1] - d[jl], za = z[jl] * z[jl], zb = z[jl + 1] * z[jl + 1];
+    // first guess from the value in the middle of the interval: the two poles
+    // next to the root kept, the others as a constant
     if (last) {
         org = K - 1;
         double zz = 0.0;
         for (int i = sub; i < K; i += LPR) zz += z[i] * z[i];
         lo = 0.0;
-        hi = rho * gsum<LPR>(zz) * (1.0 + 4.0 * kEps);
-        tau = 0.5 * hi;
-    } else {
-        const double gap = d[j + 1] - d[j], half = 0.5 * gap;
-        const double za = z[j] * z[j], zb = z[j + 1] * z[j + 1];
-        eval(d[j], half);
+        hi = rho * (LPR == 64 ? wsum(zz) : qsum(zz)) * (1.0 + 4.0 * kEps);
+        const double mid = 0.5 * hi;
+        eval(d[org], mid);
         const double w = rhoinv + psi + phi;
-        const double c = w + za / half - zb / half;
-        if (w >= 0.0) {
-            org = j;
-            lo = 0.0;
-            hi = half;
-            const double a = c * gap + za + zb, b = za * gap;
-            const double q = sqrt(fabs(a * a - 4.0 * b * c));
-            tau = a > 0.0 ? 2.0 * b / (a + q) : (a - q) / (2.0 * c);
-        } else {
-            org = j + 1;
-            lo = -half;
-            hi = 0.0;
-            const double a = c * gap - za - zb, b = zb * gap;
-            const double q = sqrt(fabs(a * a + 4.0 * b * c));
-            tau = a < 0.0 ? 2.0 * b / (a - q) : -(a + q) / (2.0 * c);
-        }
-        if (!(tau > lo && tau < hi)) tau = 0.5 * (lo + hi);
+        if (w < 0.0) lo = mid; else hi = mid;
+        const double c = w + za * fast_rcp(gap + mid) + zb * fast_rcp(mid);
+        const double a = za + zb - c * gap, b = zb * gap, q = sqrt(fabs(a * a + 4.0 * b * c));
+        tau = (a < 0.0 ? 2.0 * b : a + q) * fast_rcp(a < 0.0 ? q - a : 2.0 * c);
+    } else {
+        const double half = 0.5 * gap;
+        eval(d[j], half);
+        const double w = rhoinv + psi + phi, c = w + (za - zb) * fast_rcp(half);
+        const bool left = w >= 0.0;
+        org = left ? j : j + 1;
+        lo = left ? 0.0 : -half;
+        hi = left ? half : 0.0;
+        // c tau^2 - a tau + b = 0 with the signs of the side
+        const double a = c * gap + (left ? za + zb : -za - zb), b = left ? za * gap : -zb * gap;
+        const double q = sqrt(fabs(a * a - 4.0 * b * c));
+        const bool small = left ? a > 0.0 : a < 0.0;  // the root without cancellation
+        const double num = small ? 2.0 * b : (left ? a - q : a + q);
+        const double den = small ? (left ? a + q : a - q) : 2.0 * c;
+        tau = num * fast_rcp(den);
     }
+    if (!(tau > lo && tau < hi)) tau = 0.5 * (lo + hi);
     const double dorg = d[org];
     const double p1 = d[jl] - dorg, p2 = d[jl + 1] - dorg;
     for (int it = 0; it < 100; ++it) {
@@ -729,18 +856,21 @@ __device__ __forceinline__ void secular_root(int K, const double *d, const doubl
         if (!(fabs(w) > kEps * err)) break;
         if (w < 0.0) lo = tau; else hi = tau;
         const double D1 = p1 - tau, D2 = p2 - tau;
-        double c = w - D1 * dpsi - D2 * dphi;
         const double a = (D1 + D2) * w - D1 * D2 * dw, b = D1 * D2 * w;
-        double eta;
+        double c;
         if (last) {
-            c = fabs(c);
-            const double q = sqrt(fabs(a * a - 4.0 * b * c));
-            eta = a >= 0.0 ? (a + q) / (2.0 * c) : 2.0 * b / (a - q);
+            c = fabs(w - D1 * dpsi - D2 * dphi);
         } else {
-            const double q = sqrt(fabs(a * a - 4.0 * b * c));
-            eta = a <= 0.0 ? (a - q) / (2.0 * c) : 2.0 * b / (a + q);
+            const bool left = org == j;
+            const double r = fast_rcp(left ? D1 : D2);
+            c = left ? w - D2 * dw + gap * za * r * r : w - D1 * dw - gap * zb * r * r;
         }
-        if (!(w * eta < 0.0)) eta = -w / dw;
+        const double q = sqrt(fabs(a * a - 4.0 * b * c));
+        const bool small = last ? a < 0.0 : a > 0.0;
+        const double num = small ? 2.0 * b : (last ? a + q : a - q);
+        const double den = small ? (last ? a - q : a + q) : 2.0 * c;
+        double eta = num * fast_rcp(den);
+        if (!(w * eta < 0.0)) eta = -w * fast_rcp(dw);
         double t = tau + eta;
         if (!(t > lo && t < hi)) t = 0.5 * (lo + hi);
         if (t == tau || !(t > lo && t < hi)) break;
@@ -815,15 +945,18 @@ __device__ __forceinline__ void sibling_zero(double *Q, int n, int lev, int s, i
 
 // Leaves: one workgroup solves a segment of at most 64 rows by merges from
 // single rows, everything in LDS.  Four lanes per entry; at each level all
-// merges of the segment run together.
+// merges of the segment run together.  Bound by the chain of its phases, the
+// roots first: 98 us for 50 rows (222 us with a serial deflation pass and the
+// vectors' products on the vector unit).
 constexpr int LN = TBX_DC_LEAF;
 constexpr int LQ = LN + 1;
 
 struct LeafShared {
     double Q[2][LN * LQ];  // eigenvectors of the children / merged, [column][row]
-    double U[LN * LQ];     // [root][entry] of the secular vectors
-    double d[LN], z[LN], ds[LN], zs[LN], dk[LN], zk[LN], zh[LN], tau[LN], lam[LN], e[LN];
-    int src[LN], nd[LN], df[LN], org[LN], idx[LN], K[LN], nrot[LN], pos[LN];
+    double U[LN * LQ];     // [root][entry] of the secular vectors, zero outside the segment
+    double d[LN], z[LN], ds[LN], zs[LN], dk[LN], zk[LN], zh[LN], tau[LN], lam[LN], e[LN], zmax[LN],
+        rho[LN];
+    int src[LN], nd[LN], df[LN], org[LN], idx[LN], K[LN], nrot[LN], pos[LN], lo[LN], hi[LN];
     Rot rot[LN];
 };
 
@@ -870,12 +1003,12 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const doubl
         // this entry's segment and its split
         int lo = 0, hi = 0, mid = 0;
         if (el < N) {
-            int s = (int)(((long long)el << lev) / N);
-            while (seg_at(N, lev, s + 1) <= el) ++s;
-            while (seg_at(N, lev, s) > el) --s;
-            lo = seg_at(N, lev, s);
-            hi = seg_at(N, lev, s + 1);
-            mid = seg_at(N, lev + 1, 2 * s + 1);
+            int s = ((el << lev) + N - 1) / N;
+            while ((N * (s + 1)) >> lev <= el) ++s;
+            while ((N * s) >> lev > el) --s;
+            lo = (N * s) >> lev;
+            hi = (N * (s + 1)) >> lev;
+            mid = (N * (2 * s + 1)) >> (lev + 1);
         }
         const int len = hi - lo;
         const bool act = el < N, merge = act && mid > lo && mid < hi;
@@ -888,16 +1021,24 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const doubl
                 z *= (el >= mid && ecut < 0.0) ? -0.70710678118654752440 : 0.70710678118654752440;
             }
             W.z[el] = z;
+            W.lo[el] = lo;
+            W.hi[el] = hi;
+            W.rho[el] = rho;
             W.src[el] = el;  // every slot holds a column, whatever the order below makes of them
         }
         __syncthreads();
         if (act) {  // rank sort within the segment
             int r = 0;
+            double zm = 0.0;
             const double de = W.d[el];
+#pragma unroll 4
             for (int f = lo + sub; f < hi; f += 4) {
                 const double df = W.d[f];
                 r += (df < de || (df == de && f < el)) ? 1 : 0;
+                zm = fmax(zm, fabs(W.z[f]));
             }
+            zm = qmax(zm);
+            if (el == lo && sub == 0) W.zmax[lo] = zm;
             r += __builtin_amdgcn_update_dpp(0, r, 0xB1, 0xf, 0xf, false);
             r += __builtin_amdgcn_update_dpp(0, r, 0x4E, 0xf, 0xf, false);
             if (sub == 0) {
@@ -907,18 +1048,46 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const doubl
             }
         }
         __syncthreads();
-        if (act && el == lo && sub == 0) {
-            double zmax = 0.0;
-            for (int f = lo; f < hi; ++f) zmax = fmax(zmax, fabs(W.zs[f]));
-            const double dmax = fmax(fabs(W.ds[lo]), fabs(W.ds[hi - 1]));
-            const double tol = 16.0 * kEps * fmax(dmax, scale * zmax);
-            int nr = 0;
-            W.K[lo] = deflate(len, W.ds + lo, W.zs + lo, W.src + lo, rho, tol, W.nd + lo,
-                              W.df + lo, W.rot + lo, nr);
-            W.nrot[lo] = nr;
+        if (tid < LN) {  // one lane per sorted entry
+            int slo = 0, shi = 0;
+            double srho = 0.0, tol = 0.0;
+            if (tid < N) {
+                slo = W.lo[tid];
+                shi = W.hi[tid];
+                srho = W.rho[tid];
+                tol = 16.0 * kEps * fmax(fmax(fabs(W.ds[slo]), fabs(W.ds[shi - 1])),
+                                         scale * W.zmax[slo]);
+            }
+            const double dt = W.ds[tid], zt = W.zs[tid];
+            const bool keep = tid < N && srho * fabs(zt) > tol;
+            const unsigned long long below = (1ull << tid) - 1ull, from = ~((1ull << slo) - 1ull);
+            const unsigned long long mask = __ballot(keep) & from, prev = mask & below;
+            bool close = false;
+            if (keep && prev) {
+                const int a = 63 - __clzll((long long)prev);
+                const double zp = W.zs[a];
+                close = fabs((dt - W.ds[a]) * zp * zt) <= tol * (zp * zp + zt * zt);
+            }
+            const unsigned long long in = shi < 64 ? (1ull << shi) - 1ull : ~0ull;
+            const bool serial = (__ballot(close) & from & in) != 0;
+            const int before = __popcll(prev);
+            if (tid < N) {
+                if (!serial) {  // no two neighbours are close: what the serial pass would keep
+                    if (keep) W.nd[slo + before] = tid - slo;
+                    else W.df[slo + (tid - slo - before)] = tid - slo;
+                }
+                if (tid == slo) {
+                    int nr = 0;
+                    W.K[slo] = serial ? deflate(shi - slo, W.ds + slo, W.zs + slo, W.src + slo, srho,
+                                                tol, W.nd + slo, W.df + slo, W.rot + slo, nr)
+                                      : __popcll(mask & in);
+                    W.nrot[slo] = nr;
+                }
+            }
         }
         __syncthreads();
         const int K = act ? W.K[lo] : 0;
+        for (int i = tid; i < LN * LQ; i += 256) W.U[i] = 0.0;
         // rotations (each row on its own), then the kept entries compacted
         if (act && sub == 0) {
             for (int t = 0; t < W.nrot[lo]; ++t) {
@@ -959,7 +1128,7 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const doubl
                 const double del = (di - W.dk[lo + W.org[lo + j]]) - W.tau[lo + j];
                 pr *= j == t ? -del : del * fast_rcp(di - W.dk[lo + j]);
             }
-            pr = gprod<4>(pr);
+            pr = qprod(pr);
             if (sub == 0) W.zh[el] = copysign(sqrt(fabs(pr)), W.zk[el]);
         }
         __syncthreads();
@@ -967,13 +1136,16 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const doubl
             if (t < K) {  // normalised secular vectors
                 const double dorg = W.dk[lo + W.org[el]], tau = W.tau[el];
                 double nn = 0.0;
+#pragma unroll 4
                 for (int i = sub; i < K; i += 4) {
                     const double u = W.zh[lo + i] * fast_rcp((W.dk[lo + i] - dorg) - tau);
-                    W.U[el * LQ + i] = u;
+                    W.U[el * LQ + lo + i] = u;
                     nn += u * u;
                 }
-                const double inv = 1.0 / sqrt(gsum<4>(nn));
-                for (int i = sub; i < K; i += 4) W.U[el * LQ + i] *= inv;
+                const double inv = 1.0 / sqrt(qsum(nn));
+                for (int i = sub; i < K; i += 4) W.U[el * LQ + lo + i] *= inv;
+            } else if (sub == 0) {
+                W.U[el * LQ + el] = 1.0;  // deflated: the vector itself
             }
             int r = 0;  // place among the segment's new eigenvalues
             const double le = W.lam[el];
@@ -989,23 +1161,44 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const doubl
             }
         }
         __syncthreads();
-        // new vectors: lane = row, four wavefronts over the columns
-        const int row = tid & 63;
-        for (int c = tid >> 6; c < N; c += 4) {
-            int s = (int)(((long long)c << lev) / N);
-            while (seg_at(N, lev, s + 1) <= c) ++s;
-            while (seg_at(N, lev, s) > c) --s;
-            const int l0 = seg_at(N, lev, s), l1 = seg_at(N, lev, s + 1);
-            const int Kc = W.K[l0];
-            double acc = 0.0;
-            if (row >= l0 && row < l1) {
-                if (c - l0 < Kc) {
-                    for (int i = 0; i < Kc; ++i) acc += Q[W.idx[l0 + i] * LQ + row] * W.U[c * LQ + i];
-                } else {
-                    acc = Q[W.idx[c] * LQ + row];
+        // new vectors: Q (columns idx) times the block-diagonal U on MFMA, a
+        // 32 x 32 quarter per wavefront
+        const int lane = tid & 63, li = lane & 15, lk = lane >> 4, wv = tid >> 6;
+        const int sr = 32 * (wv >> 1), sc = 32 * (wv & 1);
+        dbl4 acc[2][2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) acc[u][q] = dbl4{0.0, 0.0, 0.0, 0.0};
+        if (sr < N && sc < N) {
+            // the entries of the columns' segments, which are also their rows
+            const int klo = W.lo[sc], khi = W.hi[min(sc + 31, N - 1)];
+            const int kend = sr < khi && sr + 32 > klo ? khi : klo;
+            for (int ks = klo & ~3; ks < kend; ks += 4) {
+                const int kk = ks + lk;
+                const double *qc = Q + (kk < N ? W.idx[kk] : 0) * LQ;
+                double x[2], y[2];
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    x[u] = qc[sr + 16 * u + li];
+                    y[u] = W.U[(sc + 16 * u + li) * LQ + kk];  // zero for kk >= N
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) acc[u][q] = mfma(x[u], y[q], acc[u][q]);
+            }
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int c = sc + 16 * q + li;
+                if (c < N) {
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            Qn[W.pos[c] * LQ + sr + 16 * u + lk + 4 * r] = acc[u][q][r];
                 }
             }
-            if (row < N) Qn[W.pos[c] * LQ + row] = acc;
         }
         __syncthreads();
         cur ^= 1;
@@ -1060,7 +1253,7 @@ __global__ void __launch_bounds__(PREP_THREADS) k_dc_prep(const EigMol *mols, Dc
     double *d = sh, *z = d + N, *ds = z + N, *zs = ds + N;
     Rot *rot = reinterpret_cast<Rot *>(zs + N);
     int *src = reinterpret_cast<int *>(rot + N), *nd = src + N, *df = nd + N;
-    __shared__ int sK, snrot;
+    __shared__ int sK, snrot, wcnt[PREP_THREADS / 64];
     __shared__ double zred[PREP_THREADS / 64];
     const double *dc = D.d + g.par * M.astride + M.a0 + g.lo;
     double *Q = D.q[g.par] + M.w0;
@@ -1094,27 +1287,72 @@ __global__ void __launch_bounds__(PREP_THREADS) k_dc_prep(const EigMol *mols, Dc
         src[r] = i;
     }
     __syncthreads();
+    double zmax = 0.0;
+    for (int q = 0; q < PREP_THREADS / 64; ++q) zmax = fmax(zmax, zred[q]);
+    const double dmax = fmax(fabs(ds[0]), fabs(ds[N - 1]));
+    const double tol = 16.0 * kEps * fmax(dmax, D.anorm[M.mol] * zmax);
+    // the entries with a z that counts, in order; where no two neighbours among
+    // them are close the serial pass would keep just these
+    const int per = (N + PREP_THREADS - 1) / PREP_THREADS, i0 = tid * per, i1 = min(i0 + per, N);
+    int cnt = 0;
+    for (int i = i0; i < i1; ++i) cnt += rho * fabs(zs[i]) > tol ? 1 : 0;
+    int inc = cnt;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+        const int y = __shfl_up(inc, s, 64);
+        if ((tid & 63) >= s) inc += y;
+    }
+    if ((tid & 63) == 63) wcnt[tid >> 6] = inc;
+    __syncthreads();
+    int kept = inc - cnt, total = 0;
+    for (int q = 0; q < PREP_THREADS / 64; ++q) {
+        if (q < (tid >> 6)) kept += wcnt[q];
+        total += wcnt[q];
+    }
+    for (int i = i0; i < i1; ++i) {
+        if (rho * fabs(zs[i]) > tol) nd[kept++] = i;
+        else df[i - kept] = i;
+    }
+    __syncthreads();
+    bool close = false;
+    for (int i = tid + 1; i < total; i += PREP_THREADS) {
+        const int a = nd[i - 1], b = nd[i];
+        const double za = zs[a], zb = zs[b];
+        close = close || fabs((ds[b] - ds[a]) * za * zb) <= tol * (za * za + zb * zb);
+    }
+    const bool serial = __syncthreads_or(close) != 0;
     if (tid == 0) {
-        double zmax = 0.0;
-        for (int q = 0; q < PREP_THREADS / 64; ++q) zmax = fmax(zmax, zred[q]);
-        const double dmax = fmax(fabs(ds[0]), fabs(ds[N - 1]));
-        const double tol = 16.0 * kEps * fmax(dmax, D.anorm[M.mol] * zmax);
         int nr = 0;
-        sK = deflate(N, ds, zs, src, rho, tol, nd, df, rot, nr);
+        sK = serial ? deflate(N, ds, zs, src, rho, tol, nd, df, rot, nr) : total;
         snrot = nr;
         D.K[M.a0 + g.lo] = sK;
         D.rho[M.a0 + g.lo] = rho;
     }
     __syncthreads();
     const int K = sK, nrot = snrot;
-    for (int r = tid; r < N; r += PREP_THREADS)
-        for (int t = 0; t < nrot; ++t) {
-            double *qa = Q + g.lo + r + (long long)(g.lo + rot[t].a) * n;
-            double *qb = Q + g.lo + r + (long long)(g.lo + rot[t].b) * n;
-            const double x = *qa, y = *qb, c = rot[t].c, s = rot[t].s;
-            *qa = c * x + s * y;
-            *qb = c * y - s * x;
+    // rotations, a row per thread, eight loaded at a time (a column that the
+    // rotation before has just changed is taken from its register)
+    constexpr int RB = 8;
+    for (int r = tid; r < N; r += PREP_THREADS) {
+        double *q = Q + g.lo + r + (long long)g.lo * n;
+        for (int t0 = 0; t0 < nrot; t0 += RB) {
+            double x[RB], y[RB], last = 0.0;
+#pragma unroll
+            for (int u = 0; u < RB; ++u) {
+                x[u] = t0 + u < nrot ? q[(long long)rot[t0 + u].a * n] : 0.0;
+                y[u] = t0 + u < nrot ? q[(long long)rot[t0 + u].b * n] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < RB; ++u)
+                if (t0 + u < nrot) {
+                    const Rot R = rot[t0 + u];
+                    const double xa = u > 0 && R.a == rot[t0 + u - 1].b ? last : x[u];
+                    q[(long long)R.a * n] = R.c * xa + R.s * y[u];
+                    last = R.c * y[u] - R.s * xa;
+                    q[(long long)R.b * n] = last;
+                }
         }
+    }
     const int o = M.a0 + g.lo;
     for (int i = tid; i < N; i += PREP_THREADS) {
         if (i < K) {
@@ -1130,7 +1368,7 @@ __global__ void __launch_bounds__(PREP_THREADS) k_dc_prep(const EigMol *mols, Dc
     }
 }
 
-// roots: eight lanes each, 32 per workgroup, the poles in LDS
+// roots: one wavefront each, the poles in LDS
 __global__ void __launch_bounds__(256) k_dc_secular(const EigMol *mols, DcPtr D, int lev,
                                                     const int *info)
 {
@@ -1139,18 +1377,18 @@ __global__ void __launch_bounds__(256) k_dc_secular(const EigMol *mols, DcPtr D,
     Seg g;
     if (!dc_seg(M.n, lev, blockIdx.z, g) || info[M.mol] != 0) return;
     const int o = M.a0 + g.lo, K = D.K[o];
-    if (32 * (int)blockIdx.x >= K) return;
+    if (4 * (int)blockIdx.x >= K) return;
     for (int i = threadIdx.x; i < K; i += 256) {
         d[i] = D.dk[o + i];
         z[i] = D.zk[o + i];
     }
     __syncthreads();
-    const int j = 32 * blockIdx.x + (threadIdx.x >> 3), sub = threadIdx.x & 7;
+    const int j = 4 * blockIdx.x + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (j >= K) return;
     double tau;
     int org;
-    secular_root<8>(K, d, z, D.rho[o], j, sub, tau, org);
-    if (sub == 0) {
+    secular_root<64>(K, d, z, D.rho[o], j, lane, tau, org);
+    if (lane == 0) {
         D.tau[o + j] = tau;
         D.org[o + j] = org;
         D.lam[o + j] = d[org] + tau;
@@ -1315,33 +1553,14 @@ __global__ void __launch_bounds__(256) k_dc_gemm(const EigMol *mols, DcPtr D, in
     }
 }
 
-// Scale of the tridiagonal matrix (largest |d|, |e|) of each molecule; a
-// matrix with a non-finite entry is marked (TBX_EIG_NONFINITE): its results are NaN.
-__global__ void __launch_bounds__(64) k_dc_scale(const EigMol *mols, const double *d,
-                                                 const double *e, double *anorm, int *info)
-{
-    const EigMol M = mols[blockIdx.x];
-    if (info[M.mol] != 0) return;
-    double mx = 0.0;
-    bool bad = false;
-    for (int i = threadIdx.x; i < M.n; i += 64) {
-        const double x = d[M.a0 + i], y = i + 1 < M.n ? e[M.a0 + i] : 0.0;
-        bad = bad || !(fabs(x) < 1e300) || !(fabs(y) < 1e300);
-        mx = fmax(mx, fmax(fabs(x), fabs(y)));
-    }
-#pragma unroll
-    for (int s = 32; s >= 1; s >>= 1) mx = fmax(mx, __shfl_xor(mx, s, 64));
-    const bool any = __any(bad);
-    if (threadIdx.x == 0) {
-        anorm[M.mol] = mx;
-        if (any) info[M.mol] = TBX_EIG_NONFINITE;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // back-transformation of 16 eigenvectors per workgroup: each wavefront holds
 // four of them in registers (rows lane + 64 r) and applies the reflectors from
-// the last to the first; then the strip is solved with L^T in LDS.
+// the last to the first, panels of eight staged in LDS (the next panel loaded
+// meanwhile, in the space the strip takes later); then the strip is solved with
+// L^T in LDS.  768 orbitals: 556 us, of which the solve takes 107 (1081 us with
+// each reflector read from L2 by every wavefront and four separate sums).
+constexpr int BP = 8;
 template <int R>
 __global__ void __launch_bounds__(256) k_eig_back(const EigMol *mols, const double *Z,
                                                   const double *V, const double *tau,
@@ -1361,42 +1580,72 @@ __global__ void __launch_bounds__(256) k_eig_back(const EigMol *mols, const doub
         return;
     }
     if (tid < 16 && c0 + tid < n) ev[M.a0 + c0 + tid] = eval[M.a0 + c0 + tid];
-    const double *Zm = Z + M.w0, *Vm = V + M.w0;
-    double z[4][R], v[R], vx[R];
+    const double *Zm = Z + M.w0, *Vm = V + M.w0, *tm = tau + M.a0;
+    const int rows = (n + NB - 1) / NB * NB;  // <= 64 R
+    double z[4][R];
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
         for (int r = 0; r < R; ++r) z[c][r] = ldg(Zm, n, lane + 64 * r, c0 + 4 * wv + c);
-    auto fetch = [&](int k) {  // reflector k: rows k + 1 ..
+    // panel q: reflectors n - 3 - BP q - b, b = 0 .. BP - 1 (two per wavefront)
+    constexpr int RS = R < 4 ? R : 4;
+    double px[BP / 4][R], ptau = 0.0;
+    __shared__ double pt[2][BP];
+    auto fetch = [&](int q) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int row = lane + 64 * r;
-            vx[r] = (64 * r + 63 > k && row > k && row < n) ? Vm[row + (long long)k * n] : 0.0;
+        for (int b = 0; b < BP / 4; ++b) {
+            const int k = n - 3 - BP * q - (wv + 4 * b);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int row = lane + 64 * r;
+                px[b][r] = (k >= 0 && row > k && row < n) ? Vm[row + (long long)k * n] : 0.0;
+            }
         }
+        const int k = n - 3 - BP * q - tid;
+        if (tid < BP && k >= 0) ptau = tm[k];
     };
-    if (n > 2) fetch(n - 3);
-    for (int k = n - 3; k >= 0; --k) {
-        const double tk = tau[M.a0 + k];
+    const int npan = n > 2 ? (n - 2 + BP - 1) / BP : 0;
+    if (npan > 0) fetch(0);
+    for (int q = 0; q < npan; ++q) {
+        double *P = X + (q & 1) * BP * 64 * R;
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = vx[r];
-        if (k > 0) fetch(k - 1);
-        double s[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int b = 0; b < BP / 4; ++b)
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (64 * r + 63 > k) {  // uniform: the rows above k are zero in v
+            for (int r = 0; r < R; ++r) P[(wv + 4 * b) * 64 * R + lane + 64 * r] = px[b][r];
+        if (tid < BP) pt[q & 1][tid] = ptau;
+        __syncthreads();  // also: the panel before this one is done with
+        if (q + 1 < npan) fetch(q + 1);
+        for (int b = 0; b < BP; ++b) {
+            const int k = n - 3 - BP * q - b;
+            if (k < 0) break;
+            const double tk = pt[q & 1][b];
+            const double *pv = P + b * 64 * R + lane;
+            // v is zero above row k: blocks of RS registers of rows there are left out
+            double v[R], s[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                for (int c = 0; c < 4; ++c) s[c] += v[r] * z[c][r];
-            }
+            for (int g = 0; g < R; g += RS)
+                if (64 * (g + RS) > k) {  // uniform
 #pragma unroll
-        for (int c = 0; c < 4; ++c) s[c] = tk * wsum(s[c]);
+                    for (int r = g; r < g + RS; ++r) v[r] = pv[64 * r];
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (64 * r + 63 > k) {
+                    for (int r = g; r < g + RS; ++r)
 #pragma unroll
-                for (int c = 0; c < 4; ++c) z[c][r] -= s[c] * v[r];
-            }
+                        for (int c = 0; c < 4; ++c) s[c] += v[r] * z[c][r];
+                }
+            wsum4(s);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) s[c] *= tk;
+#pragma unroll
+            for (int g = 0; g < R; g += RS)
+                if (64 * (g + RS) > k) {
+#pragma unroll
+                    for (int r = g; r < g + RS; ++r)
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) z[c][r] -= s[c] * v[r];
+                }
+        }
     }
-    const int rows = (n + NB - 1) / NB * NB;
+    __syncthreads();
 #pragma unroll
     for (int c = 0; c < 4; ++c)
 #pragma unroll
@@ -1427,14 +1676,13 @@ extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, in
     const int nmax = n_host[0];
     if (nmax > TBX_EIG_MAXN) return hipErrorInvalidValue;
     const size_t strip = sizeof(double) * XS * (size_t)((nmax + NB - 1) / NB * NB);
-    const size_t lds_trd = sizeof(double) * (TL * TLD + 6 * TL);
     const size_t lds_leaf = sizeof(LeafShared);
     const size_t lds_prep = (4 * sizeof(double) + sizeof(Rot) + 3 * sizeof(int)) * (size_t)nmax;
     const size_t lds_max = sizeof(double) * XS * TBX_EIG_MAXN;
     const size_t prep_max = (4 * sizeof(double) + sizeof(Rot) + 3 * sizeof(int)) * TBX_EIG_MAXN;
     hipError_t e = hipSuccess;
     if ((e = allow_lds(k_eig_trsm<false>, lds_max)) || (e = allow_lds(k_eig_trsm<true>, lds_max)) ||
-        (e = allow_lds(k_trd_lds, lds_trd)) || (e = allow_lds(k_dc_leaf, lds_leaf)) ||
+        (e = allow_lds(k_dc_leaf, lds_leaf)) ||
         (e = allow_lds(k_dc_prep, prep_max)) || (e = allow_lds(k_eig_back<2>, lds_max)) ||
         (e = allow_lds(k_eig_back<4>, lds_max)) || (e = allow_lds(k_eig_back<8>, lds_max)) ||
         (e = allow_lds(k_eig_back<12>, lds_max)) || (e = allow_lds(k_eig_back<16>, lds_max)))
@@ -1460,13 +1708,17 @@ extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, in
     hipLaunchKernelGGL(k_eig_trsm<true>, dim3(ns, nm), dim3(256), strip, s, mols, B1, B0, B2, info);
     // A in B2, the reflectors go to B0
     const TrdPtr T{B2, B0, wk->d, wk->e, wk->tau, wk->p, wk->stride};
-    for (int k = 0; nmax > TBX_TRD_LDS + k; ++k) {
-        const int cnt = above(TBX_TRD_LDS + k);
-        hipLaunchKernelGGL(k_trd_step, dim3((nmax - k - 1 + TRD_COLS - 1) / TRD_COLS, cnt),
-                           dim3(TRD_THREADS), 0, s, mols, T, k);
+    for (int k = 0; nmax > TBX_TRD_TAIL + k; ++k) {
+        const int cnt = above(TBX_TRD_TAIL + k);
+        const dim3 grid((nmax - k - 1 + TRD_COLS - 1) / TRD_COLS, cnt), blk(TRD_THREADS);
+        switch ((nmax - k + 255) / 256) {
+        case 1: hipLaunchKernelGGL(k_trd_step<1>, grid, blk, 0, s, mols, T, k); break;
+        case 2: hipLaunchKernelGGL(k_trd_step<2>, grid, blk, 0, s, mols, T, k); break;
+        case 3: hipLaunchKernelGGL(k_trd_step<3>, grid, blk, 0, s, mols, T, k); break;
+        default: hipLaunchKernelGGL(k_trd_step<4>, grid, blk, 0, s, mols, T, k); break;
+        }
     }
-    hipLaunchKernelGGL(k_trd_lds, dim3(nm), dim3(TL_THREADS), lds_trd, s, mols, T, info);
-    hipLaunchKernelGGL(k_dc_scale, dim3(nm), dim3(64), 0, s, mols, wk->d, wk->e, wk->anorm, info);
+    hipLaunchKernelGGL(k_trd_tail, dim3(nm), dim3(TL_THREADS), 0, s, mols, T, wk->anorm, info);
     // eigenvectors by parity in B2, B3
     int levels = 0;
     while (((nmax + (1 << levels) - 1) >> levels) > TBX_DC_LEAF) ++levels;
@@ -1495,7 +1747,7 @@ extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, in
         const unsigned ms = 1u << lev;
         hipLaunchKernelGGL(k_dc_prep, dim3(1, cnt, ms), dim3(PREP_THREADS), lds_prep, s, mols, D,
                            lev, info);
-        hipLaunchKernelGGL(k_dc_secular, dim3((seg + 31) / 32, cnt, ms), dim3(256), 0, s, mols, D,
+        hipLaunchKernelGGL(k_dc_secular, dim3((seg + 3) / 4, cnt, ms), dim3(256), 0, s, mols, D,
                            lev, info);
         hipLaunchKernelGGL(k_dc_zhat, dim3((seg + 3) / 4, cnt, ms), dim3(256), 0, s, mols, D, lev,
                            info);
@@ -1512,7 +1764,9 @@ extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, in
         if (m1 <= m0) continue;
         const int nx = n_host[m0];
         const dim3 grid((nx + 15) / 16, m1 - m0);
-        const size_t lds = sizeof(double) * XS * (size_t)((nx + NB - 1) / NB * NB);
+        // the strip, or two panels of reflectors before it
+        const size_t lds = sizeof(double) * std::max(XS * ((nx + NB - 1) / NB * NB),
+                                                     2 * BP * 64 * cap[q]);
         const EigMol *mm = mols + m0;
         switch (cap[q]) {
         case 16: hipLaunchKernelGGL(k_eig_back<16>, grid, dim3(256), lds, s, mm, B2, B0, wk->tau, B1, wk->ev, H, ev, info); break;
