@@ -859,6 +859,12 @@ static hipError_t upload_mols(DevTables &d, const HostMols &hm, hipStream_t s)
         if (tr.y != 1 || trans[3 * tr.x] != 0.0 || trans[3 * tr.x + 1] != 0.0 ||
             trans[3 * tr.x + 2] != 0.0)
             mt.zero_image = 0;
+    double pairs = 0.0;
+    for (int m = 0; m < hm.nmol; ++m) {
+        const double n = hm.mol_atom[m + 1] - hm.mol_atom[m];
+        pairs += n * n * hm.mol_tr[m].y;
+    }
+    mt.atom_pairs = (int)std::min(pairs / std::max(1, hm.nat), (double)INT_MAX);
     mt.trans = reinterpret_cast<const double *>(at(o_trans));
     mt.mol_tr = reinterpret_cast<const int2 *>(at(o_mol_tr));
     mt.mol_atom = reinterpret_cast<const int *>(at(o_mol_atom));

@@ -11,10 +11,10 @@
 // without forming either array:
 //   dE/dR_i  += sum_{j,T} (dEdcn_i + dEdcn_j) f'(r) v / r,   v = R_i - R_j - T
 //   sigma_m  += sum_{i in m} dEdcn_i sum_{j,T} f'(r) v v^T / r.
-// One wavefront per atom i; its lanes walk the atoms j of i's molecule and
-// the molecule's translations.  Every sum over j is a wavefront reduction,
-// so cn and dE/dR need no atomics; sigma is summed per molecule with FP64
-// atomics (six per wavefront).
+// One or four wavefronts per atom i; their lanes walk the atoms j of i's
+// molecule and the molecule's translations.  Every sum over j is a reduction
+// within the workgroup, so cn and dE/dR need no atomics; sigma is summed per
+// molecule with FP64 atomics (nine per atom).
 #include <hip/hip_runtime.h>
 
 #include "tbx_tables.h"
@@ -35,109 +35,195 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
-// counting function and its r-derivative
-__device__ __forceinline__ void dexp_count(const CnPar &c, double r, double r0, double &f,
-                                           double &df)
+// Counting function of the pair vector v, r2 = |v|^2, and with GRAD its
+// r-derivative over r.  One division gives 1/r; the two others are the factors'.
+template <bool GRAD>
+__device__ __forceinline__ void dexp_count(const CnPar &c, double r2, double r0, double &f,
+                                           double &dfr)
 {
+    const double ir = 1.0 / sqrt(r2);
     const double a0 = r0, a1 = r0 + c.rshift;
-    const double e1 = exp(-c.ka * (a0 / r - 1.0)), e2 = exp(-c.kb * (a1 / r - 1.0));
+    const double e1 = exp(-c.ka * (a0 * ir - 1.0)), e2 = exp(-c.kb * (a1 * ir - 1.0));
     const double s1 = 1.0 / (1.0 + e1), s2 = 1.0 / (1.0 + e2);
-    const double ir2 = 1.0 / (r * r);
-    // d/dr 1/(1+exp(-k (a/r - 1))) = -k a e / (r^2 (1+e)^2) = -k a e s^2 / r^2
-    const double d1 = -c.ka * a0 * e1 * s1 * s1 * ir2;
-    const double d2 = -c.kb * a1 * e2 * s2 * s2 * ir2;
     f = s1 * s2;
-    df = d1 * s2 + s1 * d2;
+    if (GRAD) {
+        // d/dr 1/(1+exp(-k (a/r - 1))) = -k a e s^2 / r^2
+        const double d1 = -c.ka * a0 * (e1 * s1) * s1, d2 = -c.kb * a1 * (e2 * s2) * s2;
+        dfr = (d1 * s2 + s1 * d2) * (ir * ir * ir);
+    }
 }
 
-__global__ void __launch_bounds__(256) k_ncoord(TbxMols mt, CnPar c, const double *xyz,
-                                                double *cn)
+// Sums of one atom i over the atoms j of its molecule and the translations,
+// by W wavefronts: the pairs (T, j) are dealt to the lanes in one flat range.
+// Molecules (one translation) take them as they come, nearly all lie within
+// the cutoff.  With lattice images most do not: each wavefront queues those
+// that do in LDS and takes them 64 at a time, so the exponentials run on full
+// wavefronts.  One wavefront per atom and a loop over the translations left
+// the lanes beyond the cell's atoms idle and ran the exponentials for each
+// translation: 6 crystals of 6..96 atoms 127 us (cn) and 145 us (gradient), now
+// 13 and 15; 1536 atoms 21 and 43 us, now 15 and 29.  W = 4 where an atom has enough pairs to share (tbx_launch_ncoord).
+constexpr int QN = 128;  // queue entries per wavefront
+struct Queue {
+    double v[3][QN];
+    int j[QN];
+};
+
+// sums: GRAD false: cn; true: dE/dR (3) and the strain sums (6)
+template <bool GRAD, int W>
+__device__ __forceinline__ void atom_sums(const TbxMols &mt, const CnPar &c, const double *xyz,
+                                          const double *dEdcn, int i, int wv, Queue &q,
+                                          double (&sum)[GRAD ? 9 : 1])
 {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
-    if (i >= mt.nat) return;  // whole wavefronts leave together
     const int m = mt.at_mol[i];
-    const int a0 = mt.mol_atom[m], a1 = mt.mol_atom[m + 1];
+    const int a0 = mt.mol_atom[m], nj = mt.mol_atom[m + 1] - a0;
     const int2 tr = mt.mol_tr[m];
     const double xi = xyz[3 * i], yi = xyz[3 * i + 1], zi = xyz[3 * i + 2];
-    const double ri = c.rcov[mt.at_sp[i]];
-    double acc = 0.0;
-    for (int t = tr.x; t < tr.x + tr.y; ++t) {
-        const double tx = mt.trans[3 * t], ty = mt.trans[3 * t + 1], tz = mt.trans[3 * t + 2];
-        for (int j = a0 + lane; j < a1; j += 64) {
+    const double ri = c.rcov[mt.at_sp[i]], ei = GRAD ? dEdcn[i] : 0.0;
+    auto add = [&](double vx, double vy, double vz, int j) {
+        double f, dfr;
+        dexp_count<GRAD>(c, vx * vx + vy * vy + vz * vz, ri + c.rcov[mt.at_sp[j]], f, dfr);
+        if (!GRAD) {
+            sum[0] += f;
+        } else {
+            const double w = (ei + dEdcn[j]) * dfr, ws = ei * dfr;
+            sum[0] += w * vx;
+            sum[1] += w * vy;
+            sum[2] += w * vz;
+            const double sx = ws * vx, sy = ws * vy;
+            sum[3] += sx * vx;  // xx xy yy xz yz zz
+            sum[4] += sx * vy;
+            sum[5] += sy * vy;
+            sum[6] += sx * vz;
+            sum[7] += sy * vz;
+            sum[8] += ws * vz * vz;
+        }
+    };
+    if (tr.y == 1) {
+        const double tx = mt.trans[3 * tr.x], ty = mt.trans[3 * tr.x + 1],
+                     tz = mt.trans[3 * tr.x + 2];
+        for (int j = a0 + lane + 64 * wv; j < a0 + nj; j += 64 * W) {
             const double vx = xi - xyz[3 * j] - tx, vy = yi - xyz[3 * j + 1] - ty,
                          vz = zi - xyz[3 * j + 2] - tz;
             const double r2 = vx * vx + vy * vy + vz * vz;
             if (r2 < kEpsR2 || r2 > c.cutoff2) continue;
-            double f, df;
-            dexp_count(c, sqrt(r2), ri + c.rcov[mt.at_sp[j]], f, df);
-            acc += f;
+            add(vx, vy, vz, j);
+        }
+        return;
+    }
+    // (t, jj) of this lane, advanced by 64 W pairs a step
+    const int st = 64 * W / nj, sj = 64 * W - st * nj, p0 = lane + 64 * wv;
+    int t = p0 / nj, jj = p0 - t * nj, nq = 0;
+    const long long steps = ((long long)nj * tr.y + 64 * W - 1) / (64 * W);
+    for (long long s = 0; s < steps; ++s) {
+        bool in = t < tr.y;
+        double vx = 0.0, vy = 0.0, vz = 0.0;
+        const int j = a0 + jj;
+        if (in) {
+            const double *T = mt.trans + 3 * (tr.x + t);
+            vx = xi - xyz[3 * j] - T[0];
+            vy = yi - xyz[3 * j + 1] - T[1];
+            vz = zi - xyz[3 * j + 2] - T[2];
+            const double r2 = vx * vx + vy * vy + vz * vz;
+            in = !(r2 < kEpsR2 || r2 > c.cutoff2);
+        }
+        const unsigned long long mask = __ballot(in);
+        if (in) {
+            const int o = nq + __popcll(mask & ((1ull << lane) - 1ull));
+            q.v[0][o] = vx;
+            q.v[1][o] = vy;
+            q.v[2][o] = vz;
+            q.j[o] = j;
+        }
+        nq += __popcll(mask);
+        __builtin_amdgcn_wave_barrier();
+        if (nq >= 64) {  // the last 64 of the queue
+            nq -= 64;
+            add(q.v[0][nq + lane], q.v[1][nq + lane], q.v[2][nq + lane], q.j[nq + lane]);
+        }
+        __builtin_amdgcn_wave_barrier();
+        t += st;
+        jj += sj;
+        if (jj >= nj) {
+            jj -= nj;
+            ++t;
         }
     }
-    acc = wave_sum(acc);
-    if (lane == 0) cn[i] = acc;
+    if (lane < nq) add(q.v[0][lane], q.v[1][lane], q.v[2][lane], q.j[lane]);
+}
+
+// Sums over the wavefront, then over the W wavefronts of the atom; on lane 0
+// of its first one.
+template <int W, int N>
+__device__ __forceinline__ void reduce(double (&sum)[N], int wv, double (*part)[9])
+{
+#pragma unroll
+    for (int k = 0; k < N; ++k) sum[k] = wave_sum(sum[k]);
+    if (W == 1) return;
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int k = 0; k < N; ++k) part[wv][k] = sum[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        sum[k] = 0.0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) sum[k] += part[w][k];
+    }
+}
+
+template <int W>
+__global__ void __launch_bounds__(256) k_ncoord(TbxMols mt, CnPar c, const double *xyz,
+                                                double *cn)
+{
+    __shared__ Queue q[4];
+    __shared__ double part[4][9];
+    const int i = W == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+    const int wv = W == 1 ? 0 : threadIdx.x >> 6;
+    if (i >= mt.nat) return;  // whole atoms leave together
+    double sum[1] = {0.0};
+    atom_sums<false, W>(mt, c, xyz, nullptr, i, wv, q[threadIdx.x >> 6], sum);
+    reduce<W>(sum, wv, part);
+    if ((threadIdx.x & 63) == 0 && wv == 0) cn[i] = sum[0];
 }
 
 // dE/dR (accumulated into grad) and sigma (accumulated, per molecule) from
 // dE/dcn
+template <int W>
 __global__ void __launch_bounds__(256) k_ncoord_grad(TbxMols mt, CnPar c, const double *xyz,
                                                      const double *dEdcn, double *grad,
                                                      double *sigma)
 {
-    const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63;
+    __shared__ Queue q[4];
+    __shared__ double part[4][9];
+    const int i = W == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
+    const int wv = W == 1 ? 0 : threadIdx.x >> 6, lane = threadIdx.x & 63;
     if (i >= mt.nat) return;
-    const int m = mt.at_mol[i];
-    const int a0 = mt.mol_atom[m], a1 = mt.mol_atom[m + 1];
-    const int2 tr = mt.mol_tr[m];
-    const double xi = xyz[3 * i], yi = xyz[3 * i + 1], zi = xyz[3 * i + 2];
-    const double ri = c.rcov[mt.at_sp[i]];
-    const double ei = dEdcn[i];
-    double g[3] = {0.0, 0.0, 0.0};
-    double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};  // xx xy yy xz yz zz
-    for (int t = tr.x; t < tr.x + tr.y; ++t) {
-        const double tx = mt.trans[3 * t], ty = mt.trans[3 * t + 1], tz = mt.trans[3 * t + 2];
-        for (int j = a0 + lane; j < a1; j += 64) {
-            const double vx = xi - xyz[3 * j] - tx, vy = yi - xyz[3 * j + 1] - ty,
-                         vz = zi - xyz[3 * j + 2] - tz;
-            const double r2 = vx * vx + vy * vy + vz * vz;
-            if (r2 < kEpsR2 || r2 > c.cutoff2) continue;
-            const double r = sqrt(r2);
-            double f, df;
-            dexp_count(c, r, ri + c.rcov[mt.at_sp[j]], f, df);
-            const double dr = df / r;
-            const double w = (ei + dEdcn[j]) * dr;
-            g[0] += w * vx;
-            g[1] += w * vy;
-            g[2] += w * vz;
-            const double ws = ei * dr;
-            s[0] += ws * vx * vx;
-            s[1] += ws * vx * vy;
-            s[2] += ws * vy * vy;
-            s[3] += ws * vx * vz;
-            s[4] += ws * vy * vz;
-            s[5] += ws * vz * vz;
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) g[k] = wave_sum(g[k]);
-#pragma unroll
-    for (int k = 0; k < 6; ++k) s[k] = wave_sum(s[k]);
+    double sum[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    atom_sums<true, W>(mt, c, xyz, dEdcn, i, wv, q[threadIdx.x >> 6], sum);
+    reduce<W>(sum, wv, part);
+    if (wv != 0) return;
     if (lane == 0) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) grad[3 * i + k] += g[k];
+        for (int k = 0; k < 3; ++k) grad[3 * i + k] += sum[k];
     }
     // sigma (3, 3) column-major from the packed symmetric sums
     if (lane < 9) {
         static constexpr int kPack[9] = {0, 1, 3, 1, 2, 4, 3, 4, 5};
         double v = 0.0;
 #pragma unroll
-        for (int k = 0; k < 9; ++k) v = (lane == k) ? s[kPack[k]] : v;
-        if (v != 0.0) unsafeAtomicAdd(&sigma[9 * m + lane], v);
+        for (int k = 0; k < 9; ++k) v = (lane == k) ? sum[3 + kPack[k]] : v;
+        if (v != 0.0) unsafeAtomicAdd(&sigma[9 * mt.at_mol[i] + lane], v);
     }
 }
 
 } // namespace
+
+// Four wavefronts per atom from 384 pairs (atoms times translations) an atom
+// on average, so that each has more than one step to share; one for the small
+// molecules of a batch, where a step already covers the molecule.
+static bool share_atoms(const TbxMols *mol) { return mol->atom_pairs >= 384; }
 
 extern "C" hipError_t tbx_launch_ncoord(const TbxMols *mol, const double *rcov, double ka,
                                         double kb, double rshift, double cutoff,
@@ -146,8 +232,11 @@ extern "C" hipError_t tbx_launch_ncoord(const TbxMols *mol, const double *rcov, 
     if (mol->nat <= 0) return hipSuccess;
     const CnPar c{rcov, ka, kb, rshift, cutoff * cutoff};
     (void)hipGetLastError();
-    hipLaunchKernelGGL(k_ncoord, dim3((mol->nat + 3) / 4), dim3(256), 0, stream, *mol, c, xyz,
-                       cn);
+    if (share_atoms(mol))
+        hipLaunchKernelGGL(k_ncoord<4>, dim3(mol->nat), dim3(256), 0, stream, *mol, c, xyz, cn);
+    else
+        hipLaunchKernelGGL(k_ncoord<1>, dim3((mol->nat + 3) / 4), dim3(256), 0, stream, *mol, c,
+                           xyz, cn);
     return hipGetLastError();
 }
 
@@ -159,7 +248,11 @@ extern "C" hipError_t tbx_launch_ncoord_grad(const TbxMols *mol, const double *r
     if (mol->nat <= 0) return hipSuccess;
     const CnPar c{rcov, ka, kb, rshift, cutoff * cutoff};
     (void)hipGetLastError();
-    hipLaunchKernelGGL(k_ncoord_grad, dim3((mol->nat + 3) / 4), dim3(256), 0, stream, *mol, c,
-                       xyz, dEdcn, grad, sigma);
+    if (share_atoms(mol))
+        hipLaunchKernelGGL(k_ncoord_grad<4>, dim3(mol->nat), dim3(256), 0, stream, *mol, c, xyz,
+                           dEdcn, grad, sigma);
+    else
+        hipLaunchKernelGGL(k_ncoord_grad<1>, dim3((mol->nat + 3) / 4), dim3(256), 0, stream, *mol,
+                           c, xyz, dEdcn, grad, sigma);
     return hipGetLastError();
 }

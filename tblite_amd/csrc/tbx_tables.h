@@ -237,6 +237,7 @@ struct TbxMols {
     int nmol, nat;
     int ntrans;
     int zero_image;                // every structure has the one translation T = 0
+    int atom_pairs;                // pairs (j, T) of an atom on average
     const double *trans;           // [3*ntrans] translation vectors of all molecules
     const int2 *mol_tr;            // [nmol] (first, count): translations of molecule m
     const int *mol_atom;           // [nmol+1] first atom
