@@ -46,12 +46,11 @@ extern "C" hipError_t tbx_launch_gradient(int mode, const TbxSpecies *sp, const 
                                           const double *Sb, const double *Db, const double *Qb,
                                           const double *Hb, const double *Sf, const double *Df,
                                           double *grad, double *dse, double *sigma,
-                                          const int *nnl, int *flag, int chunk,
+                                          int zero_sigma, const int *nnl, int *flag, int chunk,
                                           hipStream_t stream);
 extern "C" hipError_t tbx_launch_dedcn(const TbxSpecies *sp, const TbxMols *mol,
                                        const double *dse, const double *dsedcn, const double *P,
                                        double *dEdcn, hipStream_t stream);
-extern "C" hipError_t tbx_launch_fill(double *p, long long n, double v, hipStream_t stream);
 extern "C" hipError_t tbx_launch_scf(int what, const TbxMols *mol, int nspin, long long dstride,
                                      int mpdim, int vdim, const double *S, const double *mp,
                                      const double *P, const double *vao, const double *vmp,
@@ -617,8 +616,28 @@ static bool build_plans(const HostSpecies &hs, const HostMols &hm, const std::ve
     return true;
 }
 
-static int build_units(const HostSpecies &hs, HostMols &hm, const tbx_tiles &t)
+// Smaller units where the default ones would leave the chip idle: with fewer
+// than TBX_FULL_UNITS units (two workgroups per CU) the task caps shrink until
+// there are that many, down to the largest atom pair.
+#define TBX_FULL_UNITS 512
+static tbx_tiles fill_chip(const HostSpecies &hs, const HostMols &hm, tbx_tiles t)
 {
+    double tasks = 0.0;
+    for (int m = 0; m < hm.nmol; ++m) {
+        const double c = hm.mol_cart[m + 1] - hm.mol_cart[m];
+        tasks += 0.5 * c * c * hm.mol_tr[m].y;
+    }
+    const int cap = (int)std::min(tasks / TBX_FULL_UNITS, 256.0), need = hs.maxnc * hs.maxnc;
+    t.fwd_unit_tasks = std::max(need, std::min(t.fwd_unit_tasks, cap));
+    t.grad_unit_tasks = std::max(need, std::min(t.grad_unit_tasks, cap));
+    return t;
+}
+
+// fill: shrink the units of small batches (the tile shapes are the defaults,
+// not a caller's choice)
+static int build_units(const HostSpecies &hs, HostMols &hm, tbx_tiles t, bool fill)
+{
+    if (fill) t = fill_chip(hs, hm, t);
     std::vector<char> far, ffar;
     build_units_list(hs, hm, false, t.grad_unit_tasks, t.grad_unit_pairs, t.grad_band, hm.useg,
                      hm.unit_seg, &far);
@@ -977,6 +996,7 @@ struct tbx_batch {
     HostSpecies hs;
     HostMols hm;
     tbx_tiles tiles = kDefaultTiles;
+    bool tiles_set = false;  // chosen by the caller (tbx_batch_set_tiles)
     double cutoff = 0.0;  // neighbour cutoff (bohr)
     DevTables tab;
     DevBuf flag, dse_tmp;
@@ -1195,7 +1215,7 @@ static int prepare_single(tbx_context *ctx, const tbx_geom *geom, const tbx_list
     if (!reuse_mols) {
         hm_new.trans.assign(geom->trans, geom->trans + 3 * geom->ntrans);
         hm_new.mol_tr.assign(1, make_int2(0, geom->ntrans));
-        if ((st = build_units(ctx->hs, hm_new, kDefaultTiles))) return st;
+        if ((st = build_units(ctx->hs, hm_new, kDefaultTiles, true))) return st;
         HIP_TRY(hipStreamSynchronize(s));
         HIP_TRY(upload_mols(ctx->tab, hm_new, s));
         ctx->hm = std::move(hm_new);
@@ -1349,15 +1369,12 @@ extern "C" int tbx_get_hamiltonian_gradient(tbx_context *ctx, const tbx_geom *ge
     HIP_TRY(ctx->dse.reserve(sizeof(double) * hm.nsh));
     HIP_TRY(ctx->sigma.reserve(sizeof(double) * 9));
     HIP_TRY(ctx->dEdcn.reserve(sizeof(double) * nat));
-    HIP_TRY(tbx_launch_fill(ctx->grad.as<double>(), 3LL * nat, 0.0, s));
-    HIP_TRY(tbx_launch_fill(ctx->dse.as<double>(), hm.nsh, 0.0, s));
-    HIP_TRY(tbx_launch_fill(ctx->sigma.as<double>(), 9, 0.0, s));
     HIP_TRY(tbx_launch_gradient(0, &ctx->tab.sp, &ctx->tab.mt, ctx->xyz.as<double>(),
                                 ctx->se.as<double>(), ctx->P.as<double>(), ctx->W.as<double>(), ctx->vao.as<double>(),
                                 ctx->vdp.as<double>(), ctx->vqp.as<double>(), nspin, (long long)n2,
                                 nao, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
                                 ctx->grad.as<double>(),
-                                ctx->dse.as<double>(), ctx->sigma.as<double>(),
+                                ctx->dse.as<double>(), ctx->sigma.as<double>(), 1,
                                 list ? ctx->nnl.as<int>() : nullptr, ctx->flag.as<int>(), 0, s));
     HIP_TRY(tbx_launch_dedcn(&ctx->tab.sp, &ctx->tab.mt, ctx->dse.as<double>(),
                              ctx->dsedcn.as<double>(), ctx->P.as<double>(),
@@ -1407,15 +1424,12 @@ extern "C" int tbx_get_hamiltonian_adjoint(tbx_context *ctx, const tbx_geom *geo
     HIP_TRY(ctx->grad.reserve(sizeof(double) * 3 * nat));
     HIP_TRY(ctx->dse.reserve(sizeof(double) * hm.nsh));
     HIP_TRY(ctx->sigma.reserve(sizeof(double) * 9));
-    HIP_TRY(tbx_launch_fill(ctx->grad.as<double>(), 3LL * nat, 0.0, s));
-    HIP_TRY(tbx_launch_fill(ctx->dse.as<double>(), hm.nsh, 0.0, s));
-    HIP_TRY(tbx_launch_fill(ctx->sigma.as<double>(), 9, 0.0, s));
     HIP_TRY(tbx_launch_gradient(1, &ctx->tab.sp, &ctx->tab.mt, ctx->xyz.as<double>(),
                                 ctx->se.as<double>(), nullptr, nullptr, nullptr, nullptr, nullptr,
                                 1, 0, 0, ctx->S.as<double>(), ctx->D.as<double>(),
                                 ctx->Q.as<double>(), ctx->H.as<double>(), nullptr, nullptr,
                                 ctx->grad.as<double>(),
-                                ctx->dse.as<double>(), ctx->sigma.as<double>(),
+                                ctx->dse.as<double>(), ctx->sigma.as<double>(), 1,
                                 list ? ctx->nnl.as<int>() : nullptr, ctx->flag.as<int>(), 0, s));
     std::vector<double> g(3 * nat), e(hm.nsh), sg(9);
     HIP_TRY(hipMemcpyAsync(g.data(), ctx->grad.p, sizeof(double) * 3 * nat, hipMemcpyDeviceToHost, s));
@@ -1475,7 +1489,7 @@ static int batch_create(tbx_context *ctx, const tbx_batch_desc *desc, const int 
     }
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess) e = upload_species(b->tab, b->hs, desc->cutoff, ctx->stream);
-    if ((st = build_units(b->hs, b->hm, b->tiles))) {
+    if ((st = build_units(b->hs, b->hm, b->tiles, !b->tiles_set))) {
         tbx_batch_delete(b);
         return st;
     }
@@ -1515,11 +1529,12 @@ extern "C" int tbx_batch_set_tiles(tbx_batch *b, const tbx_tiles *tiles)
 {
     if (!b || !tiles) return fail(TBX_ERR_ARG, "null argument");
     if (int st = check_tiles(b->hs, tiles)) return st;
-    if (int st = build_units(b->hs, b->hm, *tiles)) {
-        (void)build_units(b->hs, b->hm, b->tiles);  // keep the host copy of the current units
+    if (int st = build_units(b->hs, b->hm, *tiles, false)) {
+        (void)build_units(b->hs, b->hm, b->tiles, !b->tiles_set);  // keep the host copy of the current units
         return st;
     }
     b->tiles = *tiles;
+    b->tiles_set = true;
     HIP_TRY(hipSetDevice(b->ctx->device));
     // The batch's kernels run on the callers' streams: wait for every stream
     // of the device, so that no launch still reads the units replaced here.
@@ -1531,7 +1546,9 @@ extern "C" int tbx_batch_set_tiles(tbx_batch *b, const tbx_tiles *tiles)
 }
 
 // Geometry hint of the pair order (see build_units_list); the cutoff is the
-// batch's neighbour cutoff.
+// batch's neighbour cutoff.  Up to TBX_HINT_UNITS units a hint is not worth its
+// launches (three workgroups per CU run at once).
+#define TBX_HINT_UNITS 768
 static int set_hint(HostMols &hm, const double *xyz, double skin, double cutoff)
 {
     if (xyz) {  // validate before anything changes
@@ -1555,10 +1572,17 @@ extern "C" int tbx_batch_order_pairs(tbx_batch *b, const double *xyz, double ski
     const std::vector<double> old_xyz = b->hm.hint_xyz;
     const double old_near2 = b->hm.near2;
     if (int st = set_hint(b->hm, xyz, skin, b->cutoff)) return st;
-    if (int st = build_units(b->hs, b->hm, b->tiles)) {
+    // Where every unit fits the chip at once the distant ones cost nothing
+    // (they end after their pair vectors), and the check of the hint and the
+    // launch of the far units would be most of the overhead: the present
+    // geometry-independent units stay.
+    if (xyz && old_xyz.empty() && b->hm.fhead.size() <= TBX_HINT_UNITS &&
+        b->hm.uhead.size() <= TBX_HINT_UNITS)
+        return set_hint(b->hm, nullptr, 0.0, b->cutoff);
+    if (int st = build_units(b->hs, b->hm, b->tiles, !b->tiles_set)) {
         b->hm.hint_xyz = old_xyz;  // keep the host copy of the current units
         b->hm.near2 = old_near2;
-        (void)build_units(b->hs, b->hm, b->tiles);
+        (void)build_units(b->hs, b->hm, b->tiles, !b->tiles_set);
         return st;
     }
     HIP_TRY(hipSetDevice(b->ctx->device));
@@ -1618,7 +1642,7 @@ extern "C" int tbx_batch_plan_stats(const tbx_batch_desc *desc, const tbx_tiles 
     if (st) return st;
     const tbx_tiles t = tiles ? *tiles : kDefaultTiles;
     if ((st = check_tiles(hs, &t))) return st;
-    if ((st = build_units(hs, hm, t))) return st;
+    if ((st = build_units(hs, hm, t, false))) return st;
     tbx_plan_stats s = {};
     s.ndense = hm.ndense;
     s.nunit_fwd = (long long)hm.fhead.size();
@@ -1845,12 +1869,9 @@ static int batch_gradient(tbx_batch *b, const double *d_xyz, const double *d_se,
     if (b->hs.diat) return fail(TBX_ERR_ARG, kNoDiatGradient);
     hipStream_t s = pick_stream(b, stream);
     HIP_TRY(mark(b, 4, s));
-    HIP_TRY(tbx_launch_fill(d_grad, 3LL * b->hm.nat, 0.0, s));
-    HIP_TRY(tbx_launch_fill(b->dse_tmp.as<double>(), b->hm.nsh, 0.0, s));
-    HIP_TRY(tbx_launch_fill(d_sigma, 9LL * b->hm.nmol, 0.0, s));
     HIP_TRY(tbx_launch_gradient(0, &b->tab.sp, &b->tab.mt, d_xyz, d_se, d_P, d_W, d_vao, d_vdp,
                                 d_vqp, 1, b->hm.ndense, b->hm.nao, nullptr, nullptr, nullptr,
-                                nullptr, d_S, d_D, d_grad, b->dse_tmp.as<double>(), d_sigma,
+                                nullptr, d_S, d_D, d_grad, b->dse_tmp.as<double>(), d_sigma, 1,
                                 nullptr, b->flag.as<int>(), b->tiles.grad_chunk, s));
     HIP_TRY(tbx_launch_dedcn(&b->tab.sp, &b->tab.mt, b->dse_tmp.as<double>(), d_dsedcn, d_P,
                              d_dEdcn, s));
@@ -1902,13 +1923,9 @@ extern "C" int tbx_batch_gradient_noalloc(tbx_batch *b, const double *d_xyz, con
     double *dse = scratch_ptr(b->ctx->device);
     if (!dse) return fail(TBX_ERR_DEVICE, "no static scratch on device %d", b->ctx->device);
     hipStream_t s = pick_stream(b, stream);
-    // the scratch keeps the previous call's sums: clear it (a fill kernel)
-    HIP_TRY(tbx_launch_fill(dse, b->hm.nsh, 0.0, s));
-    HIP_TRY(tbx_launch_fill(d_grad, 3LL * b->hm.nat, 0.0, s));
-    HIP_TRY(tbx_launch_fill(d_sigma, 9LL * b->hm.nmol, 0.0, s));
     HIP_TRY(tbx_launch_gradient(0, &b->tab.sp, &b->tab.mt, d_xyz, d_se, d_P, d_W, d_vao, d_vdp,
                                 d_vqp, 1, b->hm.ndense, b->hm.nao, nullptr, nullptr, nullptr,
-                                nullptr, nullptr, nullptr, d_grad, dse, d_sigma, nullptr,
+                                nullptr, nullptr, nullptr, d_grad, dse, d_sigma, 1, nullptr,
                                 b->flag.as<int>(),
                                 b->tiles.grad_chunk, s));
     HIP_TRY(tbx_launch_dedcn(&b->tab.sp, &b->tab.mt, dse, d_dsedcn, d_P, d_dEdcn, s));
@@ -1925,11 +1942,9 @@ static int batch_adjoint(tbx_batch *b, const double *d_xyz, const double *d_se,
     if (b->hs.diat) return fail(TBX_ERR_ARG, kNoDiatGradient);
     hipStream_t s = pick_stream(b, stream);
     HIP_TRY(mark(b, 6, s));
-    HIP_TRY(tbx_launch_fill(d_dxyz, 3LL * b->hm.nat, 0.0, s));
-    HIP_TRY(tbx_launch_fill(d_dse, b->hm.nsh, 0.0, s));
     HIP_TRY(tbx_launch_gradient(1, &b->tab.sp, &b->tab.mt, d_xyz, d_se, nullptr, nullptr,
                                 nullptr, nullptr, nullptr, 1, 0, 0, d_Sbar, d_Dbar, d_Qbar,
-                                d_Hbar, d_S, d_D, d_dxyz, d_dse, b->dse_tmp.as<double>(),
+                                d_Hbar, d_S, d_D, d_dxyz, d_dse, b->dse_tmp.as<double>(), 0,
                                 nullptr, b->flag.as<int>(), b->tiles.grad_chunk, s));
     HIP_TRY(mark(b, 7, s));
     return TBX_OK;

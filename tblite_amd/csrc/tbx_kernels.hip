@@ -41,7 +41,7 @@
 // the wavefront with DPP segmented scans, then per pair in LDS, and leave as
 // FP64 atomics into dE/dR, dE/dse and sigma.  Far units are not dispatched
 // while the hint holds; k_gradient_far runs them (persistent) when it does
-// not.  k_onsite adds the on-site dE/dse of the adjoint.
+// not.  k_begin zeroes the outputs first, with the on-site dE/dse of the adjoint.
 //
 // All arithmetic is FP64.
 #include <hip/hip_runtime.h>
@@ -1886,62 +1886,137 @@ __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient_far(GradArgs 
     }
 }
 
+// What a launch needs before its main kernel, in one launch (a small molecule's
+// call is bound by its launches, about 2 us each on the host and 1.5..3 us on
+// the device; these were up to five): workgroup by workgroup
+//   fill blocks   zeros in up to four arrays
+//   onsite blocks dE/dse of the on-site blocks (adjoint), stored, so dse needs
+//                 no zeros
+//   hint block    does the pair-order hint still hold?  One workgroup looks at
+//                 every atom and stores the answer; above TBX_HINT_ONE atoms
+//                 (32 rounds of 1024) this block only clears the flag and
+//                 k_hint_check follows.
+#define TBX_HINT_ONE 32768
+struct BeginArgs {
+    double *p[4];
+    long long n[4];
+    int nfill, nonsite, hint;  // blocks of each kind
+    int *stale;
+};
+
+__device__ __forceinline__ bool atom_moved(const TbxMols &mt, const double *xyz, int i)
+{
+    const double dx = xyz[3 * i] - mt.hint[3 * i], dy = xyz[3 * i + 1] - mt.hint[3 * i + 1],
+                 dz = xyz[3 * i + 2] - mt.hint[3 * i + 2];
+    return !(dx * dx + dy * dy + dz * dz <= mt.hint_r2);  // NaN counts as moved
+}
+
 // stale = 1 if any atom moved more than sqrt(hint_r2) from its hint position
 __global__ void k_hint_check(TbxMols mt, const double *xyz, int *stale)
 {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    bool moved = false;
-    if (i < mt.nat) {
-        const double dx = xyz[3 * i] - mt.hint[3 * i], dy = xyz[3 * i + 1] - mt.hint[3 * i + 1],
-                     dz = xyz[3 * i + 2] - mt.hint[3 * i + 2];
-        moved = !(dx * dx + dy * dy + dz * dz <= mt.hint_r2);  // NaN counts as moved
-    }
+    const bool moved = i < mt.nat && atom_moved(mt, xyz, i);
     if (__any(moved) && (threadIdx.x & 63) == 0) atomicOr(stale, 1);
 }
 
-__global__ void k_fill_int(int *p, int v)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
-}
+#define BEGIN_THREADS 1024
+#define BEGIN_FILL (4 * BEGIN_THREADS)  // elements of a fill block
 
 // On-site blocks of the adjoint: H = S (se_i + se_j)/2 contributes to dE/dse
-// only.  16 lanes per atom, looping over its Cartesian pairs.
-__global__ void __launch_bounds__(NTHREADS) k_onsite(GradArgs A)
+// only.  16 lanes per atom share its Cartesian pairs; the sums of its shells
+// are stored by the first of them.
+__device__ __forceinline__ void onsite_atom(const GradArgs &A, int i, int sub)
 {
     const TbxSpecies &sp = A.sp;
     const TbxMols &mt = A.mol;
-    const int i = blockIdx.x * (NTHREADS / 16) + (threadIdx.x >> 4);
-    if (i >= mt.nat) return;
-    const int spi = mt.at_sp[i];
-    const int nci = sp.ncart[spi];
-    const int m = mt.at_mol[i];
-    const int nao = mt.mol_nao[m];
-    const long long dense0 = mt.mol_dense[m];
-    for (int tk = threadIdx.x & 15; tk < nci * nci; tk += 16) {
-        const int ci = tk / nci, cj = tk - ci * nci;
-        const int ei_ = sp.cart_exp[spi * TBX_MAXCART + ci];
-        const int ej_ = sp.cart_exp[spi * TBX_MAXCART + cj];
-        const int ish = sp.cart_sh[spi * TBX_MAXCART + ci];
-        const int jsh = sp.cart_sh[spi * TBX_MAXCART + cj];
-        const int ki = ei_ >> 12, kj = ej_ >> 12;
-        const int sloti = ish + sp.msh * spi, slotj = jsh + sp.msh * spi;
-        const int li = sp.ang[sloti], lj = sp.ang[slotj];
-        const int muj0 = mt.at_ao[i] + sp.sh_ao[slotj];
-        const int nui0 = mt.at_ao[i] + sp.sh_ao[sloti];
-        double wHon = 0.0;
-        for (int a = 0; a < cart_n(lj, kj); ++a)
-            for (int b = 0; b < cart_n(li, ki); ++b)
-                wHon += cart_w(lj, kj, a) * cart_w(li, ki, b) *
-                        A.Hb[dense0 + (long long)(nui0 + cart_m(li, ki, b)) * nao + muj0 +
-                             cart_m(lj, kj, a)];
-        if (wHon == 0.0) continue;
-        // the same-centre overlap of the pair (a species constant)
-        const double s = sp.onsite[((spi * TBX_MAXCART + ci) * TBX_MAXCART + cj) * 10];
-        if (s != 0.0) {
-            unsafeAtomicAdd(&A.dse[mt.at_sh[i] + ish], 0.5 * wHon * s);
-            unsafeAtomicAdd(&A.dse[mt.at_sh[i] + jsh], 0.5 * wHon * s);
+    double acc[MAXSH];
+#pragma unroll
+    for (int q = 0; q < MAXSH; ++q) acc[q] = 0.0;
+    int nsh = 0, sh0 = 0;
+    if (i < mt.nat) {
+        const int spi = mt.at_sp[i];
+        const int nci = sp.ncart[spi];
+        const int m = mt.at_mol[i];
+        const int nao = mt.mol_nao[m];
+        const long long dense0 = mt.mol_dense[m];
+        nsh = sp.nsh[spi];
+        sh0 = mt.at_sh[i];
+        for (int tk = sub; tk < nci * nci; tk += 16) {
+            const int ci = tk / nci, cj = tk - ci * nci;
+            const int ki = sp.cart_exp[spi * TBX_MAXCART + ci] >> 12;
+            const int kj = sp.cart_exp[spi * TBX_MAXCART + cj] >> 12;
+            const int ish = sp.cart_sh[spi * TBX_MAXCART + ci];
+            const int jsh = sp.cart_sh[spi * TBX_MAXCART + cj];
+            const int sloti = ish + sp.msh * spi, slotj = jsh + sp.msh * spi;
+            const int li = sp.ang[sloti], lj = sp.ang[slotj];
+            // the same-centre overlap of the pair (a species constant)
+            const double s = sp.onsite[((spi * TBX_MAXCART + ci) * TBX_MAXCART + cj) * 10];
+            const int muj0 = mt.at_ao[i] + sp.sh_ao[slotj];
+            const int nui0 = mt.at_ao[i] + sp.sh_ao[sloti];
+            double wHon = 0.0;
+            for (int a = 0; a < cart_n(lj, kj); ++a)
+                for (int b = 0; b < cart_n(li, ki); ++b)
+                    wHon += cart_w(lj, kj, a) * cart_w(li, ki, b) *
+                            A.Hb[dense0 + (long long)(nui0 + cart_m(li, ki, b)) * nao + muj0 +
+                                 cart_m(lj, kj, a)];
+            if (s != 0.0) {
+                const double t = 0.5 * wHon * s;
+#pragma unroll
+                for (int q = 0; q < MAXSH; ++q) acc[q] += (q == ish ? t : 0.0) + (q == jsh ? t : 0.0);
+            }
         }
     }
+#pragma unroll
+    for (int q = 0; q < MAXSH; ++q) {
+#pragma unroll
+        for (int d = 8; d >= 1; d >>= 1) acc[q] += __shfl_xor(acc[q], d, 16);
+        if (sub == 0 && q < nsh) A.dse[sh0 + q] = acc[q];
+    }
+}
+
+__global__ void __launch_bounds__(BEGIN_THREADS) k_begin(GradArgs A, BeginArgs B)
+{
+    int b = blockIdx.x;
+    if (b < B.nfill) {
+        long long k = (long long)b * BEGIN_FILL + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < 4; ++q, k += BEGIN_THREADS) {
+            long long e = k;
+#pragma unroll
+            for (int f = 0; f < 4; ++f) {
+                if (e >= 0 && e < B.n[f]) B.p[f][e] = 0.0;
+                e -= B.n[f];
+            }
+        }
+        return;
+    }
+    b -= B.nfill;
+    if (b < B.nonsite) {
+        onsite_atom(A, b * (BEGIN_THREADS / 16) + (threadIdx.x >> 4), threadIdx.x & 15);
+        return;
+    }
+    bool moved = false;
+    if (A.mol.nat <= TBX_HINT_ONE)
+        for (int i = threadIdx.x; i < A.mol.nat; i += BEGIN_THREADS)
+            moved = atom_moved(A.mol, A.xyz, i) || moved;
+    const int any = __syncthreads_or(moved);
+    if (threadIdx.x == 0) *B.stale = any ? 1 : 0;
+}
+
+// k_begin for the given arrays (n zero: none), and k_hint_check where it is
+// left to it
+static void launch_begin(const GradArgs &a, BeginArgs b, bool onsite, hipStream_t stream)
+{
+    long long n = 0;
+    for (int f = 0; f < 4; ++f) n += b.n[f];
+    b.nfill = (int)((n + BEGIN_FILL - 1) / BEGIN_FILL);
+    b.nonsite = onsite ? (a.mol.nat + BEGIN_THREADS / 16 - 1) / (BEGIN_THREADS / 16) : 0;
+    const int blocks = b.nfill + b.nonsite + b.hint;
+    if (blocks > 0)
+        hipLaunchKernelGGL(k_begin, dim3(blocks), dim3(BEGIN_THREADS), 0, stream, a, b);
+    if (b.hint && a.mol.nat > TBX_HINT_ONE)
+        hipLaunchKernelGGL(k_hint_check, dim3((a.mol.nat + 255) / 256), dim3(256), 0, stream, a.mol,
+                           a.xyz, b.stale);
 }
 
 // Neighbour-list check of the single-structure entry points: pairs (j <= i,
@@ -1999,8 +2074,6 @@ __global__ void k_dedcn(CnArgs A)
 // ---------------------------------------------------------------------------
 // launchers (host side of this translation unit)
 
-extern "C" hipError_t tbx_launch_fill(double *p, long long n, double v, hipStream_t stream);
-
 extern "C" hipError_t tbx_launch_forward(const TbxSpecies *sp, const TbxMols *mol,
                                          const double *xyz, const double *se, double *S, double *D,
                                          double *Q, double *H, long long ndense, const int *nnl,
@@ -2010,20 +2083,24 @@ extern "C" hipError_t tbx_launch_forward(const TbxSpecies *sp, const TbxMols *mo
     FwdArgs a{*sp, *mol, xyz, se, S, D, Q, H, accumulate, chunk > 0 ? chunk : FWD_CHUNK_DEFAULT,
               flag};
     (void)hipGetLastError();  // launch errors are read below; drop stale ones
-    if (mol->nfunit_far > 0) {  // does the pair-order hint still hold for the far units?
-        if (nnl) return hipErrorInvalidValue;  // the flag serves one purpose per launch
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, flag, 0);
-        hipLaunchKernelGGL(k_hint_check, dim3((mol->nat + 255) / 256), dim3(256), 0, stream,
-                           *mol, xyz, flag);
-    }
-    if (accumulate) {  // lattice images add into the same elements
+    if (mol->nfunit_far > 0 && nnl) return hipErrorInvalidValue;  // one purpose of flag per launch
+    // does the pair-order hint still hold for the far units?  Lattice images
+    // add into zeroed outputs.
+    GradArgs g{};
+    g.mol = *mol;
+    g.xyz = xyz;
+    BeginArgs begin{};
+    begin.stale = flag;
+    begin.hint = mol->nfunit_far > 0;
+    if (accumulate) {
         double *outs[4] = {S, H, D, Q};
         const long long n[4] = {ndense, ndense, 3 * ndense, 6 * ndense};
         for (int k = 0; k < 4; ++k) {
-            const hipError_t e = tbx_launch_fill(outs[k], n[k], 0.0, stream);
-            if (e != hipSuccess) return e;
+            begin.p[k] = outs[k];
+            begin.n[k] = n[k];
         }
     }
+    launch_begin(g, begin, false, stream);
     if (mol->nfunit > 0) {
         if (sp->kdiat)
             hipLaunchKernelGGL(k_forward<true>, dim3(mol->nfunit), dim3(NTHREADS), 0, stream, a);
@@ -2044,7 +2121,7 @@ extern "C" hipError_t tbx_launch_gradient(int mode, const TbxSpecies *sp, const 
                                           const double *Sb, const double *Db, const double *Qb,
                                           const double *Hb, const double *Sf, const double *Df,
                                           double *grad, double *dse, double *sigma,
-                                          const int *nnl, int *flag, int chunk,
+                                          int zero_sigma, const int *nnl, int *flag, int chunk,
                                           hipStream_t stream)
 {
     // the per-element explicit terms need the forward's outputs and one
@@ -2056,11 +2133,18 @@ extern "C" hipError_t tbx_launch_gradient(int mode, const TbxSpecies *sp, const 
     (void)hipGetLastError();
     const int nfar = mol->nunit - mol->nunit_near;
     if (nfar > 0 && nnl) return hipErrorInvalidValue;  // the flag serves one purpose per launch
-    if (nfar > 0) {  // is the pair-order hint still good for the far units?
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, stream, flag, 0);
-        hipLaunchKernelGGL(k_hint_check, dim3((mol->nat + 255) / 256), dim3(256), 0, stream,
-                           *mol, xyz, flag);
-    }
+    // zeros (the adjoint's dse starts from its on-site part), and whether the
+    // pair-order hint is still good for the far units
+    BeginArgs begin{};
+    begin.stale = flag;
+    begin.hint = nfar > 0;
+    begin.p[0] = grad;
+    begin.n[0] = 3LL * mol->nat;
+    begin.p[1] = dse;
+    begin.n[1] = mode == GRAD_ADJOINT ? 0 : mol->nsh_tot;
+    begin.p[2] = sigma;
+    begin.n[2] = zero_sigma ? 9LL * mol->nmol : 0;
+    launch_begin(a, begin, mode == GRAD_ADJOINT, stream);
     const dim3 near(mol->nunit_near), far(nfar < 2048 ? nfar : 2048), blk(GTHREADS);
     const int *stale = flag;
     if (mol->nunit_near > 0) {
@@ -2084,10 +2168,6 @@ extern "C" hipError_t tbx_launch_gradient(int mode, const TbxSpecies *sp, const 
             hipLaunchKernelGGL((k_gradient_far<GRAD_ADJOINT, false>), far, blk, 0, stream, a,
                                stale);
     }
-    const int per = NTHREADS / 16;
-    if (mode == GRAD_ADJOINT)
-        hipLaunchKernelGGL(k_onsite, dim3((mol->nat + per - 1) / per), dim3(NTHREADS), 0, stream,
-                           a);
     if (nnl)
         hipLaunchKernelGGL(k_listcheck, dim3((mol->nat + 255) / 256), dim3(256), 0, stream, *sp,
                            *mol, xyz, nnl, flag);
@@ -2140,22 +2220,5 @@ extern "C" hipError_t tbx_launch_copy(const double *src, double *dst, long long 
     if (n <= 0) return hipSuccess;
     (void)hipGetLastError();
     hipLaunchKernelGGL(k_copy, dim3(4096), dim3(256), 0, stream, src, dst, n);
-    return hipGetLastError();
-}
-
-// Fill kernel (used instead of hipMemsetAsync so that callers may capture the
-// launches in a HIP graph).
-__global__ void k_fill(double *p, long long n, double v)
-{
-    const long long k = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) p[k] = v;
-}
-
-extern "C" hipError_t tbx_launch_fill(double *p, long long n, double v, hipStream_t stream)
-{
-    if (n <= 0) return hipSuccess;
-    const long long nb = (n + 255) / 256;
-    (void)hipGetLastError();
-    hipLaunchKernelGGL(k_fill, dim3((unsigned)nb), dim3(256), 0, stream, p, n, v);
     return hipGetLastError();
 }
