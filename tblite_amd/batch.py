@@ -157,6 +157,8 @@ class Batch:
                                           p(self.ao_off), p(self.dense_off)))
         # per-molecule views of the setup, for host-side references
         self._shell_tables()
+        self._se_tables = {}  # by device (_selfenergy_tables)
+        self._selfenergy_tables(self.torch_device)
         # the GFN2 coordination number (xtb/gfn2.f90:640): D3 covalent radii
         self.rcov = np.array([params.covalent_rad(int(z)) for z in self.nums])
         self.set_ncoord(self.rcov)
@@ -188,12 +190,31 @@ class Batch:
     def tensor_xyz(self):
         return torch.tensor(self.xyz0.reshape(-1), dtype=torch.float64, device=self.torch_device)
 
+    def _selfenergy_tables(self, device):
+        """The shells' atoms, levels and CN slopes on ``device``, uploaded once
+        and again when the host arrays have changed.  Used on another stream
+        than the one they were uploaded on, they are recorded there, so that
+        their memory outlives that use."""
+        src = (self.sh_atom, self.selfenergy_sp, self.kcn_sh)
+        ent = self._se_tables.get(device)
+        if ent is None or not all(np.array_equal(a, b) for a, b in zip(ent[0], src)):
+            stream = torch.cuda.current_stream(device) if device.type == "cuda" else None
+            # torch.tensor copies: a CPU tensor must not share the caller's arrays
+            ent = (tuple(np.array(a) for a in src),
+                   tuple(torch.tensor(a, device=device) for a in src), stream)
+            self._se_tables[device] = ent
+        elif ent[2] is not None:
+            cur = torch.cuda.current_stream(device)
+            if cur != ent[2]:
+                for t in ent[1]:
+                    t.record_stream(cur)
+        return ent[1]
+
     def selfenergy(self, cn):
         """``get_selfenergy`` over the batch (torch, differentiable in ``cn``)."""
-        cn_sh = cn[torch.as_tensor(self.sh_atom, device=cn.device)]
-        se0 = torch.as_tensor(self.selfenergy_sp, device=cn.device)
-        kcn = torch.as_tensor(self.kcn_sh, device=cn.device)
-        return se0 - kcn * cn_sh, -kcn
+        # index_select: its backward is one index_add, that of cn[atom] sorts
+        atom, se0, kcn = self._selfenergy_tables(cn.device)
+        return se0 - kcn * cn.index_select(0, atom), -kcn
 
     def molecule_translations(self, m):
         """Translation vectors (ntr, 3) of structure ``m`` (one zero vector for
