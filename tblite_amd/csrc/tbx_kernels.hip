@@ -754,7 +754,7 @@ __device__ __forceinline__ DiatFrame diat_frame(const double v[3])
 // Rotation of shell l to the diatomic frame (harmtr, :264-335): entry (r, c),
 // r a function of the molecular frame, c one of the bond frame (both 0..2l,
 // p in y, z, x order, d in m = -2..2 order); the bond axis is c = l.
-__device__ double diat_rot(const DiatFrame &F, int l, int r, int c)
+__device__ __forceinline__ double diat_rot(const DiatFrame &F, int l, int r, int c)
 {
     if (l == 0) return 1.0;
     const double ct = F.ct, st = F.st, cp = F.cp, sp = F.sp;
@@ -802,40 +802,69 @@ __device__ double diat_rot(const DiatFrame &F, int l, int r, int c)
     }
 }
 
-// Element (mj, mi) of the scaled overlap of a shell pair (lj on atom j, li on
-// atom i) at bond vector v: in the bond frame T = R_j^T S R_i, the elements
-// of equal m (m = -L..L, L = min(lj, li), at T[lj + m][li + m]) are scaled by
-// ksig, kpi or kdel for |m| = 0, 1, 2 (scale_diatomic_frame, :642-689), and
-// the block is taken back, R_j T' R_i^T (diat_trafo, :99-156).  The others
-// are unchanged and R is orthogonal, so the element is sv plus the rotated
-// changes.  S(c, d) of the shell pair comes from its Cartesian tasks
-// (task0 first, row-major by the Cartesian function of atom i).
-__device__ double diat_element(const double (*acc)[10], int task0, int ncj, int lj, int li,
-                               int mj, int mi, const double v[3], const double *k3, double sv)
+// Scaled overlap block of a shell pair (LJ on atom j, LI on atom i) at bond
+// vector v: in the bond frame T = R_j^T S R_i, the elements of equal m (m =
+// -L..L, L = min(LJ, LI), at T[LJ + m][LI + m]) are scaled by ksig, kpi or
+// kdel for |m| = 0, 1, 2 (scale_diatomic_frame, :642-689), and the block is
+// taken back, R_j T' R_i^T (diat_trafo, :99-156).  The others are unchanged and
+// R is orthogonal, so the block is S plus the rotated changes.  S comes from
+// the shell pair's Cartesian tasks (acc, row-major by the Cartesian function of
+// atom i); out[mi * (2 LJ + 1) + mj].  One lane does the whole block with the
+// rotations' entries in registers: 256 molecules of 8..128 atoms take 368 us
+// of forward against 823 us with every element forming T for itself from
+// run-time indices.
+template <int LJ, int LI>
+__device__ __forceinline__ void diat_block(const double (*acc)[10], const double v[3],
+                                           const double *k3, bool off, double *out)
 {
-    if (!(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] > 0.0)) return sv;
-    const DiatFrame F = diat_frame(v);
-    const int L = min(lj, li);
-    double T[5] = {0.0, 0.0, 0.0, 0.0, 0.0};  // T[m + 2]
-    for (int c = 0; c < 2 * lj + 1; ++c)
-        for (int d = 0; d < 2 * li + 1; ++d) {
+    constexpr int NJ = 2 * LJ + 1, NI = 2 * LI + 1, NCJ = ncart_of(LJ);
+    constexpr int L = LJ < LI ? LJ : LI;
+    double S[NI][NJ];
+#pragma unroll
+    for (int d = 0; d < NI; ++d)
+#pragma unroll
+        for (int c = 0; c < NJ; ++c) {
             double sc = 0.0;
-            for (int a = 0; a < sph_n(lj, c); ++a)
-                for (int b = 0; b < sph_n(li, d); ++b)
-                    sc += sph_w(lj, c, a) * sph_w(li, d, b) *
-                          acc[task0 + sph_c(li, d, b) * ncj + sph_c(lj, c, a)][0];
 #pragma unroll
-            for (int m = -2; m <= 2; ++m)
-                if (m >= -L && m <= L)
-                    T[m + 2] += diat_rot(F, lj, c, lj + m) * sc * diat_rot(F, li, d, li + m);
+            for (int a = 0; a < 3; ++a)
+#pragma unroll
+                for (int b = 0; b < 3; ++b)
+                    if (a < sph_n(LJ, c) && b < sph_n(LI, d))
+                        sc += sph_w(LJ, c, a) * sph_w(LI, d, b) *
+                              acc[sph_c(LI, d, b) * NCJ + sph_c(LJ, c, a)][0];
+            S[d][c] = sc;
         }
-    double out = sv;
+    if (off && v[0] * v[0] + v[1] * v[1] + v[2] * v[2] > 0.0) {
+        const DiatFrame F = diat_frame(v);
+        double T[2 * L + 1], D[NI][NJ];
 #pragma unroll
-    for (int m = -2; m <= 2; ++m)
-        if (m >= -L && m <= L)
-            out += (k3[m < 0 ? -m : m] - 1.0) * T[m + 2] * diat_rot(F, lj, mj, lj + m) *
-                   diat_rot(F, li, mi, li + m);
-    return out;
+        for (int m = -L; m <= L; ++m) {
+            double t = 0.0;
+#pragma unroll
+            for (int d = 0; d < NI; ++d)
+#pragma unroll
+                for (int c = 0; c < NJ; ++c)
+                    t += diat_rot(F, LJ, c, LJ + m) * S[d][c] * diat_rot(F, LI, d, LI + m);
+            T[m + L] = (k3[m < 0 ? -m : m] - 1.0) * t;
+        }
+#pragma unroll
+        for (int d = 0; d < NI; ++d)
+#pragma unroll
+            for (int c = 0; c < NJ; ++c) {
+                D[d][c] = S[d][c];
+#pragma unroll
+                for (int m = -L; m <= L; ++m)
+                    D[d][c] += T[m + L] * diat_rot(F, LJ, c, LJ + m) * diat_rot(F, LI, d, LI + m);
+            }
+#pragma unroll
+        for (int d = 0; d < NI; ++d)
+#pragma unroll
+            for (int c = 0; c < NJ; ++c) S[d][c] = D[d][c];
+    }
+#pragma unroll
+    for (int d = 0; d < NI; ++d)
+#pragma unroll
+        for (int c = 0; c < NJ; ++c) out[d * NJ + c] = S[d][c];
 }
 
 // One workgroup per forward unit.  (1) stage pairs and shell pairs; (2) one
@@ -853,7 +882,11 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
     __shared__ FwdStage U;
     __shared__ __align__(16) double acc[TBX_UNIT_TASKS][10];  // S, D (3), Q (6) per task
     __shared__ double hfac[TBX_UNIT_TASKS];  // H0 / S per shell pair
-    __shared__ int spk[TBX_UNIT_TASKS], spp[TBX_UNIT_TASKS];  // kept pairs, first entry
+    // kept pairs, first entry; after the work items (DIAT) the scaled overlap
+    // blocks of the shell pairs, at their first tasks
+    __shared__ __align__(16) int spkp[2 * TBX_UNIT_TASKS];
+    int *spk = spkp, *spp = spkp + TBX_UNIT_TASKS;
+    double *hover = reinterpret_cast<double *>(spkp);
     __shared__ int tinfo[TBX_UNIT_TASKS];    // type | ki << 4 | kj << 8 | shell pair << 12 | pair << 20
     __shared__ __align__(16) int coff[TBX_UNIT_TASKS + 1];  // chunk offsets, then element offsets
     __shared__ unsigned char spmap[TBX_UNIT_PAIRS * 16];     // first task of (pair, ish, jsh)
@@ -974,6 +1007,30 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
     }
     __syncthreads();
     if (tid < npair) tbx_row_map_pair(U.sinfo, roff, U.pinf, U.pext, npair, tid, rowpair);
+    if (DIAT) {  // the overlap entering H0, one lane per shell pair (nspair <= NTHREADS)
+        const bool off = tid < nspair && spk[tid] >= 0;
+        __syncthreads();  // spk is read before the blocks overwrite it
+        if (tid < nspair) {
+            const int4 e = unpack_spl(U.spl[tid]);  // pair, jsh, ish, type
+            const PairInfo pr = U.pinf[e.x];
+            const int task0 = spmap[16 * e.x + 4 * e.z + e.y];
+            const double v[3] = {U.pv[e.x][0], U.pv[e.x][1], U.pv[e.x][2]};
+            const double *k3 = sp.kdiat + 3 * (pr.spi + sp.nsp * pr.spj);
+            const double (*ac)[10] = acc + task0;
+            double *out = hover + task0;
+            switch (e.w) {  // 3 l_i + l_j
+            case 0: diat_block<0, 0>(ac, v, k3, off, out); break;
+            case 1: diat_block<1, 0>(ac, v, k3, off, out); break;
+            case 2: diat_block<2, 0>(ac, v, k3, off, out); break;
+            case 3: diat_block<0, 1>(ac, v, k3, off, out); break;
+            case 4: diat_block<1, 1>(ac, v, k3, off, out); break;
+            case 5: diat_block<2, 1>(ac, v, k3, off, out); break;
+            case 6: diat_block<0, 2>(ac, v, k3, off, out); break;
+            case 7: diat_block<1, 2>(ac, v, k3, off, out); break;
+            default: diat_block<2, 2>(ac, v, k3, off, out); break;
+            }
+        }
+    }
     __syncthreads();
     for (int base = 0; base < nel; base += NTHREADS) {
         const int e = base + tid;
@@ -1037,12 +1094,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
                 qv[5] += 1.5 * sq[5] - ts;
                 for (int c = 0; c < 3; ++c) d[c] += vv[c] * sv;
             }
-            double hv = sv;  // overlap entering H0
-            if (DIAT && spk[spx] >= 0) {
-                const double vv[3] = {U.pv[p][0], U.pv[p][1], U.pv[p][2]};
-                hv = diat_element(acc, task0, ncj, lj, li, mj, mi, vv,
-                                  sp.kdiat + 3 * (pr.spi + sp.nsp * pr.spj), sv);
-            }
+            // overlap entering H0
+            const double hv = DIAT ? hover[task0 + mi * (2 * lj + 1) + mj] : sv;
             if (accum) {
                 put(A.S + idx, sv, true);
                 put(A.H + idx, hfac[spx] * hv, true);
