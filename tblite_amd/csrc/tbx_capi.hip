@@ -1494,7 +1494,7 @@ static int batch_create(tbx_context *ctx, const tbx_batch_desc *desc, const int 
         return st;
     }
     if (e == hipSuccess) e = upload_mols(b->tab, b->hm, ctx->stream);
-    if (e == hipSuccess) e = b->flag.reserve(sizeof(int));
+    if (e == hipSuccess) e = b->flag.reserve(sizeof(int) * 256);  // an answer per hint block (k_begin)
     // scratch of the gradient / adjoint launches: dE/dse (plain) or sigma (adjoint)
     if (e == hipSuccess)
         e = b->dse_tmp.reserve(sizeof(double) * std::max({1, b->hm.nsh, 9 * b->hm.nmol}));

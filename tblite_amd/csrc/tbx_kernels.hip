@@ -8,7 +8,7 @@
 // major) and the per-type task offsets.  One workgroup runs one unit; it
 // copies the plan to LDS with one 16-byte load per lane.  With a geometry
 // hint the pairs of a molecule closer than cutoff + skin come first and the
-// others fill units of their own (TBX_UNIT_FAR); k_hint_check tells every
+// others fill units of their own (TBX_UNIT_FAR); k_begin tells every
 // launch whether any atom moved more than skin/2 from the hint, and while
 // none did those units are known to hold no pair inside the cutoff.
 //
@@ -46,6 +46,7 @@
 // All arithmetic is FP64.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstddef>
 
@@ -608,7 +609,8 @@ struct FwdArgs {
     double *S, *D, *Q, *H;
     int accumulate;      // 1: add into zeroed outputs (lattice images), 0: plain stores
     int chunk;           // primitive pairs per work item
-    const int *stale;    // nonzero: the pair-order hint no longer holds (far units run whole)
+    const int *stale;    // any nonzero: the pair-order hint no longer holds (far units run whole)
+    int nstale;          // entries of stale (hint blocks of k_begin)
 };
 
 // 1D factors V[m] = int (y+pa)^(a+m) (y+pb)^b, m = 0..2 (moments about A)
@@ -896,10 +898,12 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
     const int tid = threadIdx.x;
     const TbxUnitHead H = mt.funit[xcd_unit(blockIdx.x, gridDim.x)];
     const bool accum = A.accumulate != 0;
-    if ((H.nel & TBX_UNIT_FAR) && *A.stale == 0) {
-        // outputs with lattice images are zero-filled before the launch
-        if (!accum) far_zero_unit(A, H, U, coff, false);
-        return;
+    if (H.nel & TBX_UNIT_FAR) {
+        if (!__syncthreads_or(tid < A.nstale ? A.stale[tid] : 0)) {
+            // outputs with lattice images are zero-filled before the launch
+            if (!accum) far_zero_unit(A, H, U, coff, false);
+            return;
+        }
     }
     const int npair = H.counts & 255, nseg = (H.counts >> 8) & 255, nspair = H.counts >> 16;
     const int nao = H.nao;
@@ -1926,13 +1930,13 @@ __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient(GradArgs A)
 
 // The far gradient units (no pair within cutoff + skin at the pair-order
 // hint): nothing to do while every atom is within skin/2 of its hint
-// position (flag 0, set by k_hint_check), since then every such pair is
+// position (every answer of k_begin 0), since then every such pair is
 // still beyond the cutoff.  Otherwise the workgroups walk them.
 template <int MODE, bool EX>
 __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient_far(GradArgs A,
-                                                                     const int *stale)
+                                                                     const int *stale, int nstale)
 {
-    if (*stale == 0) return;
+    if (!__syncthreads_or((int)threadIdx.x < nstale ? stale[threadIdx.x] : 0)) return;
     for (int u = A.mol.nunit_near + blockIdx.x; u < A.mol.nunit; u += gridDim.x) {
         __syncthreads();  // the previous unit's LDS is read until its last phase
         gradient_unit<MODE, EX>(A, u);
@@ -1945,11 +1949,14 @@ __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient_far(GradArgs 
 //   fill blocks   zeros in up to four arrays
 //   onsite blocks dE/dse of the on-site blocks (adjoint), stored, so dse needs
 //                 no zeros
-//   hint block    does the pair-order hint still hold?  One workgroup looks at
-//                 every atom and stores the answer; above TBX_HINT_ONE atoms
-//                 (32 rounds of 1024) this block only clears the flag and
-//                 k_hint_check follows.
-#define TBX_HINT_ONE 32768
+//   hint blocks   does the pair-order hint still hold?  Each of up to
+//                 TBX_HINT_BLOCKS workgroups looks at its share of the atoms and
+//                 stores its own answer (nothing to clear first, and the same
+//                 whichever launch of the batch writes it); the far units read
+//                 all of them, one per lane.  A clearing launch and one that
+//                 sets a single flag took 6 us at 11 000 atoms; one workgroup for
+//                 all atoms 13 us.
+#define TBX_HINT_BLOCKS 256  // <= GTHREADS, NTHREADS
 struct BeginArgs {
     double *p[4];
     long long n[4];
@@ -1957,19 +1964,17 @@ struct BeginArgs {
     int *stale;
 };
 
+// hint blocks of a launch that has far units
+static int hint_blocks(const TbxMols &mol, bool far)
+{
+    return far ? std::min(TBX_HINT_BLOCKS, (mol.nat + 1023) / 1024) : 0;
+}
+
 __device__ __forceinline__ bool atom_moved(const TbxMols &mt, const double *xyz, int i)
 {
     const double dx = xyz[3 * i] - mt.hint[3 * i], dy = xyz[3 * i + 1] - mt.hint[3 * i + 1],
                  dz = xyz[3 * i + 2] - mt.hint[3 * i + 2];
     return !(dx * dx + dy * dy + dz * dz <= mt.hint_r2);  // NaN counts as moved
-}
-
-// stale = 1 if any atom moved more than sqrt(hint_r2) from its hint position
-__global__ void k_hint_check(TbxMols mt, const double *xyz, int *stale)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const bool moved = i < mt.nat && atom_moved(mt, xyz, i);
-    if (__any(moved) && (threadIdx.x & 63) == 0) atomicOr(stale, 1);
 }
 
 #define BEGIN_THREADS 1024
@@ -2048,16 +2053,16 @@ __global__ void __launch_bounds__(BEGIN_THREADS) k_begin(GradArgs A, BeginArgs B
         onsite_atom(A, b * (BEGIN_THREADS / 16) + (threadIdx.x >> 4), threadIdx.x & 15);
         return;
     }
+    b -= B.nonsite;
+    const int per = (A.mol.nat + B.hint - 1) / B.hint, i1 = min((b + 1) * per, A.mol.nat);
     bool moved = false;
-    if (A.mol.nat <= TBX_HINT_ONE)
-        for (int i = threadIdx.x; i < A.mol.nat; i += BEGIN_THREADS)
-            moved = atom_moved(A.mol, A.xyz, i) || moved;
+    for (int i = b * per + threadIdx.x; i < i1; i += BEGIN_THREADS)
+        moved = atom_moved(A.mol, A.xyz, i) || moved;
     const int any = __syncthreads_or(moved);
-    if (threadIdx.x == 0) *B.stale = any ? 1 : 0;
+    if (threadIdx.x == 0) B.stale[b] = any ? 1 : 0;
 }
 
-// k_begin for the given arrays (n zero: none), and k_hint_check where it is
-// left to it
+// k_begin for the given arrays (n zero: none)
 static void launch_begin(const GradArgs &a, BeginArgs b, bool onsite, hipStream_t stream)
 {
     long long n = 0;
@@ -2067,9 +2072,6 @@ static void launch_begin(const GradArgs &a, BeginArgs b, bool onsite, hipStream_
     const int blocks = b.nfill + b.nonsite + b.hint;
     if (blocks > 0)
         hipLaunchKernelGGL(k_begin, dim3(blocks), dim3(BEGIN_THREADS), 0, stream, a, b);
-    if (b.hint && a.mol.nat > TBX_HINT_ONE)
-        hipLaunchKernelGGL(k_hint_check, dim3((a.mol.nat + 255) / 256), dim3(256), 0, stream, a.mol,
-                           a.xyz, b.stale);
 }
 
 // Neighbour-list check of the single-structure entry points: pairs (j <= i,
@@ -2134,7 +2136,7 @@ extern "C" hipError_t tbx_launch_forward(const TbxSpecies *sp, const TbxMols *mo
 {
     const int accumulate = mol->ntrans > 1;
     FwdArgs a{*sp, *mol, xyz, se, S, D, Q, H, accumulate, chunk > 0 ? chunk : FWD_CHUNK_DEFAULT,
-              flag};
+              flag, hint_blocks(*mol, mol->nfunit_far > 0)};
     (void)hipGetLastError();  // launch errors are read below; drop stale ones
     if (mol->nfunit_far > 0 && nnl) return hipErrorInvalidValue;  // one purpose of flag per launch
     // does the pair-order hint still hold for the far units?  Lattice images
@@ -2144,7 +2146,7 @@ extern "C" hipError_t tbx_launch_forward(const TbxSpecies *sp, const TbxMols *mo
     g.xyz = xyz;
     BeginArgs begin{};
     begin.stale = flag;
-    begin.hint = mol->nfunit_far > 0;
+    begin.hint = a.nstale;
     if (accumulate) {
         double *outs[4] = {S, H, D, Q};
         const long long n[4] = {ndense, ndense, 3 * ndense, 6 * ndense};
@@ -2190,7 +2192,7 @@ extern "C" hipError_t tbx_launch_gradient(int mode, const TbxSpecies *sp, const 
     // pair-order hint is still good for the far units
     BeginArgs begin{};
     begin.stale = flag;
-    begin.hint = nfar > 0;
+    begin.hint = hint_blocks(*mol, nfar > 0);
     begin.p[0] = grad;
     begin.n[0] = 3LL * mol->nat;
     begin.p[1] = dse;
@@ -2212,14 +2214,17 @@ extern "C" hipError_t tbx_launch_gradient(int mode, const TbxSpecies *sp, const 
     }
     if (nfar > 0) {
         if (mode == GRAD_PLAIN && ex)
-            hipLaunchKernelGGL((k_gradient_far<GRAD_PLAIN, true>), far, blk, 0, stream, a, stale);
+            hipLaunchKernelGGL((k_gradient_far<GRAD_PLAIN, true>), far, blk, 0, stream, a, stale,
+                               begin.hint);
         else if (mode == GRAD_PLAIN)
-            hipLaunchKernelGGL((k_gradient_far<GRAD_PLAIN, false>), far, blk, 0, stream, a, stale);
+            hipLaunchKernelGGL((k_gradient_far<GRAD_PLAIN, false>), far, blk, 0, stream, a, stale,
+                               begin.hint);
         else if (ex)
-            hipLaunchKernelGGL((k_gradient_far<GRAD_ADJOINT, true>), far, blk, 0, stream, a, stale);
+            hipLaunchKernelGGL((k_gradient_far<GRAD_ADJOINT, true>), far, blk, 0, stream, a, stale,
+                               begin.hint);
         else
-            hipLaunchKernelGGL((k_gradient_far<GRAD_ADJOINT, false>), far, blk, 0, stream, a,
-                               stale);
+            hipLaunchKernelGGL((k_gradient_far<GRAD_ADJOINT, false>), far, blk, 0, stream, a, stale,
+                               begin.hint);
     }
     if (nnl)
         hipLaunchKernelGGL(k_listcheck, dim3((mol->nat + 255) / 256), dim3(256), 0, stream, *sp,
