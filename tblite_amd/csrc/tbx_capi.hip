@@ -410,7 +410,9 @@ struct HostMols {
         cart_atom, ao_atom, sh_off, unit_seg, funit_seg, uplan, fplan, sh_aog, tiles, dtiles;
     std::vector<long long> mol_dense;
     std::vector<TbxSeg> useg, fseg;
-    std::vector<TbxUnitHead> uhead, fhead;
+    std::vector<TbxUnitHead> uhead, fhead;  // fhead: the near units, then the far ones
+    std::vector<TbxUnitHead> fmain;         // forward launch: near units and zero units
+    std::vector<int> zplan;                 // runs of the zero units
     // optional geometry hint (bohr, [3*nat]) for the order of the pairs in the
     // units: pairs within sqrt(near2) there come first in each molecule
     std::vector<double> hint_xyz;
@@ -418,6 +420,17 @@ struct HostMols {
     int nunit_near = 0;  // gradient units holding a pair within cutoff + skin at the hint
     int nfunit_far = 0;  // forward units holding none
 };
+
+// Is the pair (i, j, image itr) within cutoff + skin at the hint geometry?
+static bool pair_near(const HostMols &hm, int i, int j, int itr)
+{
+    double r2 = 0.0;
+    for (int c = 0; c < 3; ++c) {
+        const double d = hm.hint_xyz[3 * i + c] - hm.hint_xyz[3 * j + c] - hm.trans[3 * itr + c];
+        r2 += d * d;
+    }
+    return i == j && r2 < 1e-12 ? true : r2 <= hm.near2;
+}
 
 // Work units (see TbxSeg): the half list of every molecule, cut into units of
 // bounded task count.  Gradient: j < i (j <= i with lattice images); forward:
@@ -432,15 +445,7 @@ static void build_units_list(const HostSpecies &hs, const HostMols &hm, bool dia
 {
     band = std::max(band, 1);
     const bool hinted = hm.hint_xyz.size() == 3 * (size_t)hm.nat;
-    auto near = [&](int i, int j, int itr) {
-        if (!hinted) return true;
-        double r2 = 0.0;
-        for (int c = 0; c < 3; ++c) {
-            const double d = hm.hint_xyz[3 * i + c] - hm.hint_xyz[3 * j + c] - hm.trans[3 * itr + c];
-            r2 += d * d;
-        }
-        return i == j && r2 < 1e-12 ? true : r2 <= hm.near2;
-    };
+    auto near = [&](int i, int j, int itr) { return !hinted || pair_near(hm, i, j, itr); };
     useg.clear();
     unit_seg.assign(1, 0);
     if (unit_far) unit_far->clear();
@@ -616,6 +621,81 @@ static bool build_plans(const HostSpecies &hs, const HostMols &hm, const std::ve
     return true;
 }
 
+// The units of a forward launch: the near units and, where a hint leaves far
+// pairs, the zero units of their elements, molecule by molecule and in equal
+// shares along each, so that stores and arithmetic run side by side on every CU
+// and both touch a molecule's columns at about the same time.  Outputs with
+// lattice images are zeroed before the launch and need no zero units.
+static void build_forward_launch(const HostSpecies &hs, HostMols &hm,
+                                 const std::vector<TbxUnitHead> &near)
+{
+    hm.fmain.clear();
+    hm.zplan.clear();
+    if (hm.nfunit_far == 0 || hm.trans.size() > 3) {
+        hm.fmain = near;
+        return;
+    }
+    std::vector<TbxUnitHead> zero;
+    std::vector<double> x[3];  // the molecule's hint geometry, for a vectorised row of pair_near
+    std::vector<char> far;
+    size_t u = 0;
+    for (int m = 0; m < hm.nmol; ++m) {
+        const int a0 = hm.mol_atom[m], a1 = hm.mol_atom[m + 1], n = a1 - a0;
+        for (int c = 0; c < 3; ++c) {
+            x[c].resize(n);
+            for (int j = 0; j < n; ++j) x[c][j] = hm.hint_xyz[3 * (a0 + j) + c];
+        }
+        far.assign(n + 1, 0);  // ends with a pair that is not far
+        zero.clear();
+        int elems = TBX_ZERO_ELEMS;
+        auto put = [&](int i, int row0, int rows) {
+            const int cols = hs.nao[hm.at_sp[i]];
+            for (int r = 0; r < rows; r += TBX_ZERO_ROWS) {
+                const int len = std::min(rows - r, TBX_ZERO_ROWS);
+                if (elems >= TBX_ZERO_ELEMS) {
+                    TbxUnitHead h{};
+                    h.dense0 = hm.mol_dense[m];
+                    h.plan = (int)(hm.zplan.size() / 4);
+                    h.nao = hm.mol_nao[m];
+                    h.ao_m = hm.mol_ao[m];
+                    h.mol = m;
+                    h.nel = TBX_UNIT_ZERO;
+                    zero.push_back(h);
+                    elems = 0;
+                }
+                hm.zplan.insert(hm.zplan.end(), {hm.at_ao[i], cols, row0 + r, len});
+                ++zero.back().counts;
+                elems += cols * len;
+            }
+        };
+        for (int i = 0; i < n; ++i) {
+            const double p[3] = {x[0][i], x[1][i], x[2][i]};
+            for (int j = 0; j < n; ++j) {
+                double r2 = 0.0;
+                for (int c = 0; c < 3; ++c) r2 += (p[c] - x[c][j]) * (p[c] - x[c][j]);
+                far[j] = !(r2 <= hm.near2);
+            }
+            far[i] = !pair_near(hm, a0 + i, a0 + i, hm.mol_tr[m].x);
+            for (int j = 0, j0 = -1; j <= n; ++j) {
+                if (far[j] && j0 < 0) j0 = j;
+                if (!far[j] && j0 >= 0) {
+                    const int row0 = hm.at_ao[a0 + j0];
+                    put(a0 + i, row0, (j < n ? hm.at_ao[a0 + j] : hm.mol_nao[m]) - row0);
+                    j0 = -1;
+                }
+            }
+        }
+        size_t e = u;
+        while (e < near.size() && near[e].mol == m) ++e;
+        const size_t nn = e - u, nz = zero.size();
+        for (size_t k = 0, z = 0; k < nn || z < nz;) {  // nn near units and nz zero units, mixed
+            if (z >= nz || (k < nn && k * nz <= z * nn)) hm.fmain.push_back(near[u + k++]);
+            else hm.fmain.push_back(zero[z++]);
+        }
+        u = e;
+    }
+}
+
 // Smaller units where the default ones would leave the chip idle: with fewer
 // than TBX_FULL_UNITS units (two workgroups per CU) the task caps shrink until
 // there are that many, down to the largest atom pair.
@@ -655,14 +735,14 @@ static int build_units(const HostSpecies &hs, HostMols &hm, tbx_tiles t, bool fi
     hm.nunit_near = (int)near.size();
     near.insert(near.end(), farh.begin(), farh.end());
     hm.uhead.swap(near);
-    // forward units of such pairs stay in place (the XCD-contiguous unit
-    // order), flagged: while the hint holds they only write zero blocks
-    hm.nfunit_far = 0;
-    for (size_t u = 0; u < hm.fhead.size(); ++u)
-        if (ffar[u]) {
-            hm.fhead[u].nel |= TBX_UNIT_FAR;
-            ++hm.nfunit_far;
-        }
+    // forward units of such pairs too; while the hint holds their elements are
+    // zeros, written by the zero units
+    std::vector<TbxUnitHead> fnear, ffarh;
+    for (size_t u = 0; u < hm.fhead.size(); ++u) (ffar[u] ? ffarh : fnear).push_back(hm.fhead[u]);
+    hm.nfunit_far = (int)ffarh.size();
+    build_forward_launch(hs, hm, fnear);
+    hm.fhead.swap(fnear);
+    hm.fhead.insert(hm.fhead.end(), ffarh.begin(), ffarh.end());
     return TBX_OK;
 }
 
@@ -854,6 +934,10 @@ static hipError_t upload_mols(DevTables &d, const HostMols &hm, hipStream_t s)
 {
     Arena &a = d.mol_host;
     a.host.clear();
+    // the plans are nearly all of it (60 MB for 1536 atoms): not to be copied as the arena grows
+    a.host.reserve(4 * (hm.uplan.size() + hm.fplan.size() + hm.zplan.size()) +
+                   sizeof(TbxUnitHead) * (hm.uhead.size() + hm.fmain.size() + hm.fhead.size()) +
+                   128 * hm.at_sp.size() + 65536);
     const std::vector<double> &trans = hm.trans;
     const size_t o_mol_tr = a.add(hm.mol_tr);
     const size_t o_trans = a.add(trans), o_mol_atom = a.add(hm.mol_atom),
@@ -862,9 +946,11 @@ static hipError_t upload_mols(DevTables &d, const HostMols &hm, hipStream_t s)
                  o_at_mol = a.add(hm.at_mol), o_at_sh = a.add(hm.at_sh), o_at_ao = a.add(hm.at_ao),
                  o_at_cart = a.add(hm.at_cart), o_cart_atom = a.add(hm.cart_atom),
                  o_ao_atom = a.add(hm.ao_atom), o_mol_ao = a.add(hm.mol_ao),
-                 o_uhead = a.add(hm.uhead), o_uplan = a.add(hm.uplan), o_fhead = a.add(hm.fhead),
+                 o_uhead = a.add(hm.uhead), o_uplan = a.add(hm.uplan), o_fmain = a.add(hm.fmain),
                  o_fplan = a.add(hm.fplan), o_sh_aog = a.add(hm.sh_aog), o_tiles = a.add(hm.tiles), o_dtiles = a.add(hm.dtiles),
-                 o_hint = a.add(hm.hint_xyz);
+                 o_hint = a.add(hm.hint_xyz), o_zplan = a.add(hm.zplan),
+                 o_ffar = a.add(std::vector<TbxUnitHead>(hm.fhead.end() - hm.nfunit_far,
+                                                         hm.fhead.end()));
     const hipError_t e = upload_arena(d.mols, a, s);
     if (e != hipSuccess) return e;
     const char *base = static_cast<const char *>(d.mols.p);
@@ -901,8 +987,10 @@ static hipError_t upload_mols(DevTables &d, const HostMols &hm, hipStream_t s)
     mt.nunit = (int)hm.uhead.size();
     mt.unit = reinterpret_cast<const TbxUnitHead *>(at(o_uhead));
     mt.plan = reinterpret_cast<const int *>(at(o_uplan));
-    mt.nfunit = (int)hm.fhead.size();
-    mt.funit = reinterpret_cast<const TbxUnitHead *>(at(o_fhead));
+    mt.nfunit = (int)hm.fmain.size();
+    mt.funit = reinterpret_cast<const TbxUnitHead *>(at(o_fmain));
+    mt.ffunit = reinterpret_cast<const TbxUnitHead *>(at(o_ffar));
+    mt.zplan = reinterpret_cast<const int *>(at(o_zplan));
     mt.fplan = reinterpret_cast<const int *>(at(o_fplan));
     mt.nsh_tot = hm.nsh;
     mt.nao_tot = hm.nao;
@@ -915,7 +1003,7 @@ static hipError_t upload_mols(DevTables &d, const HostMols &hm, hipStream_t s)
     // (a little less than) half the skin away from the hint
     const bool hinted = hm.hint_xyz.size() == 3 * (size_t)hm.nat && hm.nat > 0;
     mt.nunit_near = hinted ? hm.nunit_near : mt.nunit;
-    mt.nfunit_far = hinted ? hm.nfunit_far : 0;
+    mt.nfunit_far = hm.nfunit_far;  // none without a hint
     mt.hint = hinted ? reinterpret_cast<const double *>(at(o_hint)) : nullptr;
     mt.hint_r2 = 0.25 * 0.999 * hm.skin * hm.skin;
     return hipSuccess;
@@ -1774,6 +1862,50 @@ extern "C" int tbx_batch_plan_stats(const tbx_batch_desc *desc, const tbx_tiles 
         }
         for (unsigned char c : hit)
             if (c != 1) ++s.bad_elems;
+        // the zero units write exactly the elements of the far units, and the
+        // launch holds every near unit
+        if (!fwd || hm.nfunit_far == 0) continue;
+        long long nzero = 0, nnear = 0;
+        std::vector<unsigned char> zhit((size_t)hm.ndense, 0);
+        for (const TbxUnitHead &h : hm.fmain) {
+            if (!(h.nel & TBX_UNIT_ZERO)) {
+                ++nnear;
+                continue;
+            }
+            const long long nao = hm.mol_nao[h.mol];
+            for (int k = 0; k < h.counts; ++k) {
+                const int *r = &hm.zplan[4 * ((size_t)h.plan + k)];
+                if (r[0] < 0 || r[1] < 1 || r[0] + r[1] > nao || r[2] < 0 || r[3] < 1 ||
+                    r[3] > TBX_ZERO_ROWS || r[2] + r[3] > nao || h.nao != nao ||
+                    h.dense0 != hm.mol_dense[h.mol]) {
+                    ++s.bad_elems;
+                    continue;
+                }
+                for (int c = r[0]; c < r[0] + r[1]; ++c)
+                    for (int e = r[2]; e < r[2] + r[3]; ++e) {
+                        unsigned char &z = zhit[h.dense0 + c * nao + e];
+                        if (z < 2) ++z;
+                    }
+                nzero += (long long)r[1] * r[3];
+            }
+        }
+        if (nnear != (long long)head.size() - hm.nfunit_far) ++s.bad_units;
+        long long nfar = 0;
+        for (size_t q = head.size() - hm.nfunit_far; q < head.size(); ++q) {
+            const PlanView v = plan_view(plan, head[q]);
+            const int4 *seg = reinterpret_cast<const int4 *>(v.sinfo);
+            for (int k = 0; k < v.nseg; ++k) {  // block A and mirror of every segment
+                const long long nao = head[q].nao, d0 = head[q].dense0;
+                const int4 g = seg[k];
+                for (int c = 0; c < g.w; ++c)
+                    for (int r = 0; r < (g.z & 0xffff); ++r, ++nfar)
+                        if (zhit[d0 + (g.x + c) * nao + g.y + r] != 1) ++s.bad_elems;
+                for (int c = 0; c < (g.z >> 16); ++c)
+                    for (int r = 0; r < g.w; ++r, ++nfar)
+                        if (zhit[d0 + (g.y + c) * nao + g.x + r] != 1) ++s.bad_elems;
+            }
+        }
+        if (nfar != nzero) ++s.bad_elems;
     }
     *out = s;
     return TBX_OK;

@@ -8,9 +8,11 @@
 // major) and the per-type task offsets.  One workgroup runs one unit; it
 // copies the plan to LDS with one 16-byte load per lane.  With a geometry
 // hint the pairs of a molecule closer than cutoff + skin come first and the
-// others fill units of their own (TBX_UNIT_FAR); k_begin tells every
-// launch whether any atom moved more than skin/2 from the hint, and while
-// none did those units are known to hold no pair inside the cutoff.
+// others fill units of their own; k_begin tells every launch whether any
+// atom moved more than skin/2 from the hint, and while none did those units
+// are known to hold no pair inside the cutoff: they do not run
+// (k_forward_far, k_gradient_far), and the forward's zero units
+// (TBX_UNIT_ZERO) write their elements.
 //
 // Forward, k_forward (get_hamiltonian, xtb/h0.f90:220-429): a unit's lanes
 // form the pair vectors, then one lane per shell pair counts its kept
@@ -676,23 +678,53 @@ __device__ __forceinline__ void put(double *p, double v, bool acc)
     if (acc) unsafeAtomicAdd(p, v); else *p = v;
 }
 
+// A zero unit (TBX_UNIT_ZERO): runs of zero blocks, a run per wavefront at a
+// time; its columns and rows are dealt to the lanes in one range, and the
+// quadrupole goes out in 16-byte stores.  Bound by the memory's writes, of
+// which the lines that a run shares with a near pair's block cost most: the
+// forward of (H2O)512, 755 MB of zeros, takes 79 us without them, these runs
+// alone 222 us and a fill of everything 141 us.  So the runs are as long as the
+// far atoms follow each other, in both triangles (the far work units' own
+// blocks, a mirror's rows one atom at a time, made the forward 469 us), and go
+// past the L2, which the near units' blocks need to complete their lines: 240 us
+// (279 through it; 8 clusters of 200 to 500 atoms 199 -> 138, 157 through it).
+__device__ __forceinline__ void zero_unit(const FwdArgs &A, const TbxUnitHead &H)
+{
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int4 *run = reinterpret_cast<const int4 *>(A.mol.zplan) + H.plan;
+    typedef double d2 __attribute__((ext_vector_type(2)));
+    const d2 z = {0.0, 0.0};
+    for (int q = wv; q < H.counts; q += NTHREADS / 64) {
+        const int4 g = run[q];  // first column, columns, first row, rows
+        const int rows = g.w, total = g.y * rows;
+        const float inv = 1.0f / (float)rows, inv3 = 1.0f / (float)(3 * rows);
+        const long long e0 = H.dense0 + (long long)g.x * H.nao + g.z;
+        // k / rows: exact, k + 0.5 is at least 0.5 / rows (> 1e-3) from a
+        // multiple and k / rows below 64, so the rounding (1e-5) cannot cross one
+        for (int k = lane; k < total; k += 64) {
+            const int c = (int)(((float)k + 0.5f) * inv);
+            const long long e = e0 + (long long)c * H.nao + (k - c * rows);
+            __builtin_nontemporal_store(0.0, A.S + e);
+            __builtin_nontemporal_store(0.0, A.H + e);
+        }
+        for (int k = lane; k < 3 * total; k += 64) {
+            const int c = (int)(((float)k + 0.5f) * inv3), r = k - 3 * c * rows;
+            const long long e = e0 + (long long)c * H.nao;
+            __builtin_nontemporal_store(0.0, A.D + 3 * e + r);
+            __builtin_nontemporal_store(z, reinterpret_cast<d2 *>(A.Q + 6 * e + 2 * r));
+        }
+    }
+}
+
 // A forward unit none of whose pairs is within the cutoff: its blocks are
 // zero.  They are the segments' rectangles, block A (rows of the atoms j,
 // columns of atom i) and the mirror (rows of atom i, columns of the atoms
-// j < i), so only the segment words of the plan are needed (read here unless
-// `staged`: a far unit, TBX_UNIT_FAR, known from the pair-order hint while
-// every atom stays within skin/2 of it, stages nothing else).  off: LDS of
-// 2 * TBX_UNIT_SEGS + 1 ints.
+// j < i).  off: LDS of 2 * TBX_UNIT_SEGS + 1 ints.
 __device__ __forceinline__ void far_zero_unit(const FwdArgs &A, const TbxUnitHead &H, FwdStage &U,
-                                              int *off, bool staged)
+                                              int *off)
 {
     const int tid = threadIdx.x;
-    const int npair = H.counts & 255, nseg = (H.counts >> 8) & 255;
-    if (!staged) {
-        const int4 *src = reinterpret_cast<const int4 *>(A.mol.fplan) + H.plan +
-                          ((10 * npair + 3) >> 2) + ((npair + 3) >> 2);
-        if (tid < nseg) U.sinfo[tid] = src[tid];
-    }
+    const int nseg = (H.counts >> 8) & 255;
     __syncthreads();
     if (tid == 0) tbx_elem_offsets(U.sinfo, nseg, off);  // block A and mirror of each segment
     __syncthreads();
@@ -879,7 +911,7 @@ __device__ __forceinline__ void diat_block(const double (*acc)[10], const double
 // every element of the molecule's matrices is written exactly once.  DIAT:
 // off-site H0 blocks from the diatomic-frame scaled overlap (sp.kdiat).
 template <bool DIAT>
-__global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
+__device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead &H)
 {
     __shared__ FwdStage U;
     __shared__ __align__(16) double acc[TBX_UNIT_TASKS][10];  // S, D (3), Q (6) per task
@@ -896,15 +928,7 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
     const TbxSpecies &sp = A.sp;
     const TbxMols &mt = A.mol;
     const int tid = threadIdx.x;
-    const TbxUnitHead H = mt.funit[xcd_unit(blockIdx.x, gridDim.x)];
     const bool accum = A.accumulate != 0;
-    if (H.nel & TBX_UNIT_FAR) {
-        if (!__syncthreads_or(tid < A.nstale ? A.stale[tid] : 0)) {
-            // outputs with lattice images are zero-filled before the launch
-            if (!accum) far_zero_unit(A, H, U, coff, false);
-            return;
-        }
-    }
     const int npair = H.counts & 255, nseg = (H.counts >> 8) & 255, nspair = H.counts >> 16;
     const int nao = H.nao;
     const long long dense0 = H.dense0;
@@ -928,7 +952,8 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
         live = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] <= sp.cutoff2;
     }
     if (!__syncthreads_or(live)) {
-        if (!accum) far_zero_unit(A, H, U, coff, true);
+        // outputs with lattice images are zero-filled before the launch
+        if (!accum) far_zero_unit(A, H, U, coff);
         return;
     }
     // shell pairs: screening counts and H0 factors (one lane per shell pair)
@@ -1126,6 +1151,30 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
     }
 }
 
+
+template <bool DIAT>
+__global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
+{
+    const TbxUnitHead H = A.mol.funit[xcd_unit(blockIdx.x, gridDim.x)];
+    if (H.nel & TBX_UNIT_ZERO) {  // unless the far units run (k_forward_far)
+        if (!__syncthreads_or((int)threadIdx.x < A.nstale ? A.stale[threadIdx.x] : 0))
+            zero_unit(A, H);
+        return;
+    }
+    forward_unit<DIAT>(A, H);
+}
+
+// The forward units of the pairs beyond cutoff + skin at the hint, when an
+// atom has left it (as k_gradient_far).
+template <bool DIAT>
+__global__ void __launch_bounds__(NTHREADS, 2) k_forward_far(FwdArgs A)
+{
+    if (!__syncthreads_or((int)threadIdx.x < A.nstale ? A.stale[threadIdx.x] : 0)) return;
+    for (int u = blockIdx.x; u < A.mol.nfunit_far; u += gridDim.x) {
+        __syncthreads();  // the previous unit's LDS is read until its last phase
+        forward_unit<DIAT>(A, A.mol.ffunit[u]);
+    }
+}
 
 // The explicit pair-vector terms of one spherical element (mu on atom j, nu
 // on atom i; e1 = (mu, nu), e2 = (nu, mu)) from the forward's S and
@@ -2161,6 +2210,13 @@ extern "C" hipError_t tbx_launch_forward(const TbxSpecies *sp, const TbxMols *mo
             hipLaunchKernelGGL(k_forward<true>, dim3(mol->nfunit), dim3(NTHREADS), 0, stream, a);
         else
             hipLaunchKernelGGL(k_forward<false>, dim3(mol->nfunit), dim3(NTHREADS), 0, stream, a);
+    }
+    if (mol->nfunit_far > 0) {
+        const dim3 far(std::min(mol->nfunit_far, 2048));
+        if (sp->kdiat)
+            hipLaunchKernelGGL(k_forward_far<true>, far, dim3(NTHREADS), 0, stream, a);
+        else
+            hipLaunchKernelGGL(k_forward_far<false>, far, dim3(NTHREADS), 0, stream, a);
     }
     if (nnl)
         hipLaunchKernelGGL(k_listcheck, dim3((mol->nat + 255) / 256), dim3(256), 0, stream, *sp,

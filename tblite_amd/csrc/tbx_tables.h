@@ -103,12 +103,21 @@ struct TbxUnitHead {
     int counts;        // npair | nseg << 8 | nspair << 16
     int nao, ao_m;     // AOs of the molecule, its first AO (global)
     int mol;
-    int nel;           // dense elements written (forward units) | TBX_UNIT_FAR
+    int nel;           // dense elements written (forward units), or TBX_UNIT_ZERO
 };
-// TbxUnitHead::nel flag of a forward unit none of whose pairs lies within
-// cutoff + skin at the pair-order hint; TBX_NEL_MASK gives the count
-#define TBX_UNIT_FAR (1 << 30)
+// TbxUnitHead::nel flag of a zero unit: `counts` runs of zero blocks, one
+// 16-byte word each at zplan[16 * plan ...]: (first column, columns, first row,
+// rows), all molecule-local.  The columns are those of one atom, the rows those
+// of consecutive atoms beyond cutoff + skin of it at the pair-order hint (in
+// both triangles, so the runs are long), at most TBX_ZERO_ROWS of them.
+// TBX_NEL_MASK gives the element count of the other units.
+#define TBX_UNIT_ZERO (1 << 30)
 #define TBX_NEL_MASK 0xffff
+#define TBX_ZERO_ROWS 128
+// A zero unit is filled up to TBX_ZERO_ELEMS elements: forward of 256 molecules
+// of 8 to 128 atoms 361 us at 1024, 370 at 512, 419 at 4096 (a unit of the last
+// holds up the stores of the near units on its CU), of (H2O)512 279, 276, 284.
+#define TBX_ZERO_ELEMS 1024
 
 // The dense elements of a forward unit, segment k after segment k - 1:
 // block A (rows: the AOs of the segment's atoms j, first AO seg.y, `rows` of
@@ -261,9 +270,13 @@ struct TbxMols {
     double hint_r2;                // squared displacement below which the far units stay dead
     const int *plan;               // their plans (16-byte words)
     int nfunit;
-    const TbxUnitHead *funit;      // [nfunit] forward units (j <= i, on-site pairs included)
-    int nfunit_far;                // forward units flagged TBX_UNIT_FAR
-    const int *fplan;
+    const TbxUnitHead *funit;      // [nfunit] forward units (j <= i, on-site pairs included) that
+                                   // hold a pair within cutoff + skin of the pair-order hint, and
+                                   // between them the zero units of the other pairs
+    int nfunit_far;
+    const TbxUnitHead *ffunit;     // [nfunit_far] forward units of those pairs, for a hint that
+                                   // no longer holds
+    const int *fplan, *zplan;
     int nsh_tot, nao_tot;
     const int *sh_aog;             // [nsh_tot+1] first AO (global) of every shell
     int ntile;
