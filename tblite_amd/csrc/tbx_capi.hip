@@ -1788,16 +1788,22 @@ extern "C" int tbx_batch_plan_stats(const tbx_batch_desc *desc, const tbx_tiles 
             // segment words, first task of each shell pair from the shell-pair list
             const int4 *seg = reinterpret_cast<const int4 *>(v.sinfo);
             const TbxPair *pinf = reinterpret_cast<const TbxPair *>(v.pairs);
-            std::vector<int> off(2 * v.nseg + 1), roff(v.nseg + 1);
+            std::vector<int> off(2 * v.nseg + 1);
             tbx_elem_offsets(seg, v.nseg, off.data());
-            // the row map the kernel reads the pair from (every row carries an
-            // element, so it has at most 2 * TBX_UNIT_TASKS entries)
-            tbx_row_offsets(seg, v.nseg, roff.data());
-            std::vector<unsigned char> rmap(2 * TBX_UNIT_TASKS, 255);
-            if (roff[v.nseg] > 2 * TBX_UNIT_TASKS) ++s.bad_units;
-            else
-                for (int q = 0; q < v.npair; ++q)
-                    tbx_row_map_pair(seg, roff.data(), pinf, v.pext, v.npair, q, rmap.data());
+            // the tables the kernel reads an element's place from
+            alignas(16) int eoff[2 * TBX_UNIT_SEGS];
+            int roff[TBX_UNIT_SEGS + 1] = {0};
+            std::vector<unsigned short> rmap(2 * TBX_UNIT_TASKS, 0xffff);
+            for (int k = 0; k < 2 * TBX_UNIT_SEGS; ++k) eoff[k] = k < 2 * v.nseg ? off[k] : INT_MAX;
+            for (int k = 0; k < v.nseg; ++k) roff[k + 1] = roff[k] + (seg[k].z & 0xffff);
+            const bool rows_ok = roff[v.nseg] <= 2 * TBX_UNIT_TASKS;
+            if (!rows_ok) ++s.bad_units;
+            for (int q = 0; rows_ok && q < v.npair; ++q) {
+                const int first = roff[v.pext[q] & 31] + pinf[q].aoj - seg[v.pext[q] & 31].y;
+                if (first < 0 || first + hs.nao[pinf[q].spj] > roff[(v.pext[q] & 31) + 1])
+                    ++s.bad_units;
+                else tbx_row_map_pair(seg, roff, pinf, v.pext, q, rmap.data());
+            }
             std::vector<int> spmap((size_t)16 * v.npair, -1);
             for (int q = 0; q < v.nspair; ++q) {
                 const int e = v.spl[q], ty = e >> 16, li = ty / 3, lj = ty % 3;
@@ -1812,11 +1818,16 @@ extern "C" int tbx_batch_plan_stats(const tbx_batch_desc *desc, const tbx_tiles 
                 const TbxElem el = tbx_elem_locate(off.data(), v.nseg, seg, pinf, v.pext, v.npair, e);
                 const int p = el.p, nul = el.nul, muj = el.muj;
                 const bool mirror = el.mirror != 0;
-                bool map_ok = roff[v.nseg] <= 2 * TBX_UNIT_TASKS;
+                bool map_ok = rows_ok;
                 if (map_ok) {
-                    const TbxElem em = tbx_elem_locate_map(off.data(), v.nseg, seg, pinf,
-                                                           roff.data(), rmap.data(), e);
-                    map_ok = em.p == p && em.nul == nul && em.muj == muj && em.mirror == el.mirror;
+                    const TbxElemRow er = tbx_elem_row(eoff, seg, roff, rmap.data(), e);
+                    const int jsp = pinf[p].spj, jsh = TBX_ROW_SHELL(er.row);
+                    map_ok = TBX_ROW_PAIR(er.row) == p && er.nul == nul &&
+                             er.mirror == el.mirror && er.k == (v.pext[p] & 31) &&
+                             seg[er.k].y + er.jr == pinf[p].aoj + muj &&
+                             hs.ao_sh[muj + TBX_MAXAO * jsp] == jsh &&
+                             hs.ao_m[muj + TBX_MAXAO * jsp] == TBX_ROW_M(er.row) &&
+                             hs.ang[jsh + hs.msh * jsp] == TBX_ROW_L(er.row);
                 }
                 if (!block_ok || !map_ok || p < 0 || p >= v.npair) {
                     ++s.bad_elems;

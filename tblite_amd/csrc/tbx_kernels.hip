@@ -719,16 +719,12 @@ __device__ __forceinline__ void zero_unit(const FwdArgs &A, const TbxUnitHead &H
 // A forward unit none of whose pairs is within the cutoff: its blocks are
 // zero.  They are the segments' rectangles, block A (rows of the atoms j,
 // columns of atom i) and the mirror (rows of atom i, columns of the atoms
-// j < i).  off: LDS of 2 * TBX_UNIT_SEGS + 1 ints.
-__device__ __forceinline__ void far_zero_unit(const FwdArgs &A, const TbxUnitHead &H, FwdStage &U,
-                                              int *off)
+// j < i).  off: the element offsets in LDS.
+__device__ __forceinline__ void far_zero_unit(const FwdArgs &A, const TbxUnitHead &H,
+                                              const FwdStage &U, const int *off)
 {
     const int tid = threadIdx.x;
-    const int nseg = (H.counts >> 8) & 255;
-    __syncthreads();
-    if (tid == 0) tbx_elem_offsets(U.sinfo, nseg, off);  // block A and mirror of each segment
-    __syncthreads();
-    const int total = off[2 * nseg];
+    const int nseg = (H.counts >> 8) & 255, total = H.nel;
     const long long dense0 = H.dense0;
     const int nao = H.nao;
     const double2 z = make_double2(0.0, 0.0);
@@ -915,16 +911,19 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
 {
     __shared__ FwdStage U;
     __shared__ __align__(16) double acc[TBX_UNIT_TASKS][10];  // S, D (3), Q (6) per task
-    __shared__ double hfac[TBX_UNIT_TASKS];  // H0 / S per shell pair
+    __shared__ double hfac[TBX_UNIT_TASKS];  // H0 / S of a shell pair, at its first task
     // kept pairs, first entry; after the work items (DIAT) the scaled overlap
     // blocks of the shell pairs, at their first tasks
     __shared__ __align__(16) int spkp[2 * TBX_UNIT_TASKS];
     int *spk = spkp, *spp = spkp + TBX_UNIT_TASKS;
     double *hover = reinterpret_cast<double *>(spkp);
     __shared__ int tinfo[TBX_UNIT_TASKS];    // type | ki << 4 | kj << 8 | shell pair << 12 | pair << 20
-    __shared__ __align__(16) int coff[TBX_UNIT_TASKS + 1];  // chunk offsets, then element offsets
+    __shared__ __align__(16) int coff[TBX_UNIT_TASKS + 1];  // chunk offsets
     __shared__ unsigned char spmap[TBX_UNIT_PAIRS * 16];     // first task of (pair, ish, jsh)
-    __shared__ unsigned char rowpair[2 * TBX_UNIT_TASKS];    // pair of each block-A row
+    // element and row offsets of the segments, words of the block-A rows (tbx_elem_row)
+    __shared__ __align__(16) int eoff[2 * TBX_UNIT_SEGS];
+    __shared__ int roff[TBX_UNIT_SEGS];
+    __shared__ unsigned short rowmap[2 * TBX_UNIT_TASKS];
     const TbxSpecies &sp = A.sp;
     const TbxMols &mt = A.mol;
     const int tid = threadIdx.x;
@@ -951,9 +950,21 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
         for (int c = 0; c < 3; ++c) U.pv[tid][c] = v[c];
         live = v[0] * v[0] + v[1] * v[1] + v[2] * v[2] <= sp.cutoff2;
     }
+    if (tid >= NTHREADS - 64) {  // the last wavefront: offsets of the segments, one per lane
+        const int k = tid - (NTHREADS - 64);
+        int4 g = make_int4(0, 0, 0, 0);
+        if (k < nseg) g = U.sinfo[k];
+        const int rows = g.z & 0xffff, el = g.w * rows, em = g.w * (g.z >> 16);
+        const int v = el + em + (rows << 16), ex = wave_scan(v) - v;  // at most 512 of each
+        if (k < TBX_UNIT_SEGS) {
+            eoff[2 * k] = k < nseg ? ex & 0xffff : INT_MAX;
+            eoff[2 * k + 1] = k < nseg ? (ex & 0xffff) + el : INT_MAX;
+            roff[k] = ex >> 16;
+        }
+    }
     if (!__syncthreads_or(live)) {
         // outputs with lattice images are zero-filled before the launch
-        if (!accum) far_zero_unit(A, H, U, coff);
+        if (!accum) far_zero_unit(A, H, U, eoff);
         return;
     }
     // shell pairs: screening counts and H0 factors (one lane per shell pair)
@@ -963,7 +974,17 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
         const bool on = shellpair_setup(sp, mt, A.xyz, U, A.se, k, true, kept, pi0, hs, sesum, dsr);
         spk[k] = on ? -1 : kept;  // on-site blocks: moments from the species table
         spp[k] = pi0;
-        hfac[k] = sesum * hs;
+        const int4 e = unpack_spl(U.spl[k]);  // pair, jsh, ish, type
+        const int ncp = ncart_of(e.w / 3) * ncart_of(e.w % 3);
+        const int task0 = U.toff[e.w] + (k - U.tsp[e.w]) * ncp;
+        spmap[16 * e.x + 4 * e.z + e.y] = (unsigned char)task0;
+        hfac[task0] = sesum * hs;
+    }
+    if (tid < npair) {
+        tbx_row_map_pair(U.sinfo, roff, U.pinf, U.pext, tid, rowmap);
+        // shell layout of the row atom, for the element phase
+        const int k = U.pext[tid] & 31;
+        if (tid == 0 || (U.pext[tid - 1] & 31) != k) U.sinfo[k].w |= U.pinf[tid].di << 8;
     }
     __syncthreads();
     // tasks: one Cartesian pair per lane
@@ -973,10 +994,6 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
         int spx;
         const int4 d = decode_task(U, tid, spx);
         tinfo[tid] = d.x | (d.y << 4) | (d.z << 8) | (spx << 12) | ((U.spl[spx] & 255) << 20);
-        if (d.w == 0) {  // the shell pair's first task, for the element phase
-            const int4 e = unpack_spl(U.spl[spx]);  // pair, jsh, ish, type
-            spmap[16 * e.x + 4 * e.z + e.y] = (unsigned char)tid;
-        }
         const int kept = spk[spx];
         if (kept >= 0) {
             nch = (kept + chunk - 1) / chunk;
@@ -999,7 +1016,7 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
 
     // (4) work items
     for (int c = tid; c < nchunk; c += NTHREADS) {
-        const int tk = find_last_le(coff, NTHREADS, c);
+        const int tk = find_task<TBX_UNIT_TASKS>(coff, c);
         const int info = tinfo[tk];
         const int t = info & 15, ki = (info >> 4) & 15, kj = (info >> 8) & 15;
         const int spx = (info >> 12) & 255;
@@ -1024,18 +1041,15 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
         for (int k = 0; k < 10; ++k) atomicAdd(&acc[tk][k], o[k]);
     }
 
-    // (5) one lane per dense element, located from the segment words
-    // (tbx_elem_locate): block A (rows of atoms j, the columns of atom i) and
-    // the mirror (rows of atom i, columns of the j < i); every element of the
-    // molecule's matrices is written by exactly one lane of one unit
-    __syncthreads();  // the items are done with coff
-    int *roff = coff + 2 * nseg + 1;  // row offsets after the element offsets
-    if (tid == 0) {
-        tbx_elem_offsets(U.sinfo, nseg, coff);
-        tbx_row_offsets(U.sinfo, nseg, roff);
-    }
+    // (5) one lane per dense element, located from the unit's tables
+    // (tbx_elem_row): block A (rows of atoms j, the columns of atom i) and the
+    // mirror (rows of atom i, columns of the j < i); every element of the
+    // molecule's matrices is written by exactly one lane of one unit.  The
+    // tables come from the phases before the work items, so no lane is left to
+    // run through the segments alone here, and a lane's chain is six LDS reads
+    // instead of fourteen: crystals 61 -> 51 us, 256 molecules of 8 to 128 atoms
+    // 361 -> 346, 640 of 8 to 256 1838 -> 1800.
     __syncthreads();
-    if (tid < npair) tbx_row_map_pair(U.sinfo, roff, U.pinf, U.pext, npair, tid, rowpair);
     if (DIAT) {  // the overlap entering H0, one lane per shell pair (nspair <= NTHREADS)
         const bool off = tid < nspair && spk[tid] >= 0;
         __syncthreads();  // spk is read before the blocks overwrite it
@@ -1059,22 +1073,21 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
             default: diat_block<2, 2>(ac, v, k3, off, out); break;
             }
         }
+        __syncthreads();
     }
-    __syncthreads();
     for (int base = 0; base < nel; base += NTHREADS) {
         const int e = base + tid;
         if (e < nel) {
-            const TbxElem el = tbx_elem_locate_map(coff, nseg, U.sinfo, U.pinf, roff, rowpair, e);
-            const int p = el.p, nul = el.nul, muj = el.muj;
+            const TbxElemRow el = tbx_elem_row(eoff, U.sinfo, roff, rowmap, e);
+            const int p = TBX_ROW_PAIR(el.row), jsh = TBX_ROW_SHELL(el.row);
+            const int mj = TBX_ROW_M(el.row), lj = TBX_ROW_L(el.row);
             const bool mirror = el.mirror != 0;
-            const PairInfo pr = U.pinf[p];
-            int ish, mi, li, jsh, mj, lj;
-            ao_decode(pr.di, nul, ish, mi, li);
-            ao_decode(pr.dj, muj, jsh, mj, lj);
+            const int4 g = U.sinfo[el.k];
+            int ish, mi, li;
+            ao_decode(g.w >> 8, el.nul, ish, mi, li);
             const int task0 = spmap[16 * p + 4 * ish + jsh];
-            const int spx = (tinfo[task0] >> 12) & 255;
             const int ncj = ncart_of(lj);
-            const int mu = pr.aoj + muj;
+            const int mu = g.y + el.jr, nu = g.x + el.nul;
             double v[10];
 #pragma unroll
             for (int q = 0; q < 10; ++q) v[q] = 0.0;
@@ -1099,7 +1112,6 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
             double d[3] = {v[1], v[2], v[3]};
             double qv[6] = {1.5 * v[4] - tr, 1.5 * v[5], 1.5 * v[6] - tr,
                             1.5 * v[7], 1.5 * v[8], 1.5 * v[9] - tr};
-            const int nu = pr.aoi + nul;
             long long idx;
             if (!mirror) {
                 idx = dense0 + (long long)nu * nao + mu;
@@ -1127,14 +1139,14 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
             const double hv = DIAT ? hover[task0 + mi * (2 * lj + 1) + mj] : sv;
             if (accum) {
                 put(A.S + idx, sv, true);
-                put(A.H + idx, hfac[spx] * hv, true);
+                put(A.H + idx, hfac[task0] * hv, true);
 #pragma unroll
                 for (int c = 0; c < 3; ++c) put(A.D + 3 * idx + c, d[c], true);
 #pragma unroll
                 for (int c = 0; c < 6; ++c) put(A.Q + 6 * idx + c, qv[c], true);
             } else {
                 A.S[idx] = sv;
-                A.H[idx] = hfac[spx] * hv;
+                A.H[idx] = hfac[task0] * hv;
                 // the 3 dipole components: one 16-byte store (aligned for either
                 // parity of idx) and one 8-byte store
                 const bool odd = (idx & 1) != 0;

@@ -181,62 +181,68 @@ __host__ __device__ inline TbxElem tbx_elem_locate(const int *off, int nseg, con
     return r;
 }
 
-// The pair search of tbx_elem_locate as a table, one byte per block-A row
-// of the unit (at most 2 * TBX_UNIT_TASKS, since every row carries at least
-// one element): roff[k] = the first entry of segment k (nseg + 1 of them),
-// map[roff[k] + r] = the last pair of segment k whose first AO of atom j is
-// at most the row's AO.  tbx_row_map_pair writes pair p's rows, from its
-// first AO of atom j up to the next pair's of the segment (one pair per lane).
-__host__ __device__ inline void tbx_row_offsets(const int4 *seg, int nseg, int *roff)
-{
-    int n = 0;
-    for (int k = 0; k < nseg; ++k) {
-        roff[k] = n;
-        n += seg[k].z & 0xffff;
-    }
-    roff[nseg] = n;
-}
-
+// The search of tbx_elem_locate from tables of the unit that the kernel forms in
+// LDS.  Segments: tbx_elem_offsets filled up to 2 * TBX_UNIT_SEGS entries with
+// INT_MAX, and roff[k], the first entry of segment k in the row table.  Rows: one
+// word per block-A row (at most 2 * TBX_UNIT_TASKS, since every row carries at
+// least one element) with the row's pair and, of its AO, the shell within atom
+// j, m and l; tbx_row_map_pair writes pair p's rows (one pair per lane).
+#define TBX_ROW_PAIR(w) ((w) & 127)
+#define TBX_ROW_SHELL(w) (((w) >> 7) & 3)
+#define TBX_ROW_M(w) (((w) >> 9) & 7)
+#define TBX_ROW_L(w) (((w) >> 12) & 3)
 __host__ __device__ inline void tbx_row_map_pair(const int4 *seg, const int *roff,
-                                                 const TbxPair *pinf, const int *pext, int npair,
-                                                 int p, unsigned char *map)
+                                                 const TbxPair *pinf, const int *pext, int p,
+                                                 unsigned short *map)
 {
-    const int k = pext[p] & 31;
-    const int4 g = seg[k];
-    const int rows = g.z & 0xffff;
-    const int r1 = (p + 1 < npair && (pext[p + 1] & 31) == k) ? pinf[p + 1].aoj - g.y : rows;
-    for (int r = pinf[p].aoj - g.y; r < r1; ++r)
-        if (r >= 0 && r < rows) map[roff[k] + r] = (unsigned char)p;
+    const int k = pext[p] & 31, desc = pinf[p].dj, nsh = desc & 7;
+    unsigned short *row = map + roff[k] + (pinf[p].aoj - seg[k].y);
+    for (int s = 0; s < nsh; ++s) {
+        const int l = (desc >> (3 + 2 * s)) & 3;
+        for (int m = 0; m < 2 * l + 1; ++m)
+            *row++ = (unsigned short)(p | (s << 7) | (m << 9) | (l << 12));
+    }
 }
 
-// tbx_elem_locate with the pair read from the row map
-__host__ __device__ inline TbxElem tbx_elem_locate_map(const int *off, int nseg, const int4 *seg,
-                                                      const TbxPair *pinf, const int *roff,
-                                                      const unsigned char *map, int e)
+// a / b for 0 <= a < 1024, 0 < b <= 512: a + 0.5 is at least 1e-3 of b away from
+// every multiple of b, the quotient below 1024 and its relative error 2e-7
+__host__ __device__ inline int tbx_div_small(int a, int b)
 {
-    int lo = 0, hi = 2 * nseg;  // last half-segment whose first element is <= e
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (off[mid] <= e) lo = mid; else hi = mid;
+#ifdef __HIP_DEVICE_COMPILE__
+    return (int)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
+#else
+    return (int)(((float)a + 0.5f) * (1.0f / (float)b));
+#endif
+}
+
+// Element e: its segment, AO within atom i, row of the segment and its word, and
+// whether it lies in the mirror.  Two rounds of independent reads find the
+// half-segment (16-byte aligned off).
+struct TbxElemRow {
+    int k, nul, jr, row, mirror;
+};
+__host__ __device__ inline TbxElemRow tbx_elem_row(const int *off, const int4 *seg,
+                                                   const int *roff, const unsigned short *map,
+                                                   int e)
+{
+    static_assert(TBX_UNIT_SEGS == 32, "search over four blocks of 16 offsets");
+    const int b = (off[16] <= e) + (off[32] <= e) + (off[48] <= e);
+    const int4 *blk = reinterpret_cast<const int4 *>(off + 16 * b);
+    int t = 0;
+    for (int k = 0; k < 4; ++k) {
+        const int4 v = blk[k];
+        t += (v.x <= e) + (v.y <= e) + (v.z <= e) + (v.w <= e);
     }
-    const int k = lo >> 1;
-    const int4 g = seg[k];
-    const int local = e - off[lo];
-    TbxElem r;
-    r.mirror = lo & 1;
-    int jao;  // molecule-local AO on the atom-j side
-    if (!r.mirror) {
-        const int rows = g.z & 0xffff;
-        const int c = local / rows;
-        r.nul = c;
-        jao = g.y + (local - c * rows);
-    } else {
-        const int c = local / g.w;
-        r.nul = local - c * g.w;
-        jao = g.y + c;
-    }
-    r.p = map[roff[k] + (jao - g.y)];
-    r.muj = jao - pinf[r.p].aoj;
+    const int h = 16 * b + t - 1;
+    TbxElemRow r;
+    r.k = h >> 1;
+    r.mirror = h & 1;
+    const int4 g = seg[r.k];
+    const int local = e - off[h], n = r.mirror ? g.w & 255 : g.z & 0xffff;
+    const int quot = tbx_div_small(local, n), rem = local - quot * n;
+    r.nul = r.mirror ? rem : quot;
+    r.jr = r.mirror ? quot : rem;
+    r.row = map[roff[r.k] + r.jr];
     return r;
 }
 
