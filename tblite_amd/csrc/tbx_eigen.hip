@@ -12,13 +12,14 @@
 //   k_trd_step    one Householder column of A per launch (n > TBX_TRD_TAIL)
 //   k_trd_tail    the last TBX_TRD_TAIL columns, the whole rest of A in registers
 //   k_dc_leaf     eigenpairs of tridiagonal blocks of at most 64 rows by divide
-//                 and conquer from single rows, in LDS
+//                 and conquer from single rows, in LDS; triangular factors of
+//                 blocks of 16 reflectors beside them
 //   k_dc_prep, k_dc_secular, k_dc_zhat, k_dc_norm, k_dc_gemm
 //                 the merges above that (Cuppen's rank-one update; deflation
 //                 and the recomputed vector z of M. Gu and S. Eisenstat, SIAM J.
 //                 Matrix Anal. Appl. 16, 172 (1995)), products on MFMA
-//   k_eig_back    the reflectors of the tridiagonal form applied to 16
-//                 eigenvectors in registers, then C = L^-T Z in LDS
+//   k_eig_back    the blocks of reflectors of the tridiagonal form applied to
+//                 16 eigenvectors in registers, then C = L^-T Z in LDS
 //
 // Matrices are column-major n x n at EigMol::w0 of the workspace buffers,
 // vectors at the molecule's first orbital a0.
@@ -960,16 +961,74 @@ struct LeafShared {
     Rot rot[LN];
 };
 
+// Triangular factor M of block g of 16 reflectors (k_eig_back), column c from
+// reflector c on, into the part of V above the reflector (column kmax - c, which
+// holds nothing else).  Workgroups of the leaves' launch, which is longer: as a
+// launch of its own 5 us for 26 orbitals, 10 for 768.
+constexpr int WB = 16;
+__device__ void wy_block(const EigMol &M, double *V, const double *tau, int g,
+                         double (*red)[WB][WB + 1])
+{
+    const int n = M.n, kmax = n - 3 - WB * g;
+    if (kmax < 0) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    double *Vm = V + M.w0;
+    const int k = kmax - li;
+    const double *col = Vm + (long long)max(k, 0) * n;
+    dbl4 acc = dbl4{0.0, 0.0, 0.0, 0.0};
+    for (int r0 = (max(kmax - WB + 2, 0) & ~15) + 16 * wv; r0 < n; r0 += 64) {
+        double v[4];
+        const double *src = col + min(r0 + 4 * lk, n - 1);  // at most 3 past the column: in V
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = src[r];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int row = r0 + 4 * lk + r;
+            v[r] = (k >= 0 && row > k && row < n) ? v[r] : 0.0;
+            acc = mfma(v[r], v[r], acc);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wv][lk + 4 * r][li] = acc[r];
+    __syncthreads();
+    const int i = threadIdx.x >> 4, j = threadIdx.x & 15;
+    red[0][i][j] += red[1][i][j] + red[2][i][j] + red[3][i][j];
+    __syncthreads();
+    if (threadIdx.x >= WB) return;
+    const int c = threadIdx.x, m = min(WB, kmax + 1);  // column of M; reflectors
+    double t[WB], s[WB];
+#pragma unroll
+    for (int q = 0; q < WB; ++q) t[q] = tau[M.a0 + max(kmax - q, 0)];
+#pragma unroll
+    for (int q = 0; q < WB; ++q) {
+        double x = q == c ? 1.0 : 0.0;
+#pragma unroll
+        for (int e = 0; e < q; ++e) x -= red[0][q][e] * s[e];
+        s[q] = q < m ? t[q] * x : 0.0;
+    }
+    if (c < m) {
+        double *out = Vm + (long long)(kmax - c) * n;
+#pragma unroll
+        for (int q = 0; q < WB; ++q)
+            if (q >= c && q < m) out[q - c] = s[q];
+    }
+}
+
 __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const double *dg,
                                                  const double *eg, double *dout, double *q0,
-                                                 double *q1, const double *anorm,
-                                                 const int *info)
+                                                 double *q1, const double *anorm, int leaves,
+                                                 double *V, const double *tau, const int *info)
 {
     extern __shared__ double sh[];
     LeafShared &W = *reinterpret_cast<LeafShared *>(sh);
     const EigMol M = mols[blockIdx.y];
     const int n = M.n;
     if (info[M.mol] != 0) return;
+    if ((int)blockIdx.x >= leaves) {
+        wy_block(M, V, tau, (int)blockIdx.x - leaves,
+                 reinterpret_cast<double (*)[WB][WB + 1]>(sh));
+        return;
+    }
     const int L = dc_levels(n);
     if ((int)blockIdx.x >= (1 << L)) return;
     const int g0 = seg_at(n, L, blockIdx.x), g1 = seg_at(n, L, blockIdx.x + 1), N = g1 - g0;
@@ -1554,24 +1613,31 @@ __global__ void __launch_bounds__(256) k_dc_gemm(const EigMol *mols, DcPtr D, in
 }
 
 // ---------------------------------------------------------------------------
-// back-transformation of 16 eigenvectors per workgroup: each wavefront holds
-// four of them in registers (rows lane + 64 r) and applies the reflectors from
-// the last to the first, panels of eight staged in LDS (the next panel loaded
-// meanwhile, in the space the strip takes later); then the strip is solved with
-// L^T in LDS.  768 orbitals: 556 us, of which the solve takes 107 (1081 us with
-// each reflector read from L2 by every wavefront and four separate sums).
-constexpr int BP = 8;
+// Back-transformation of 16 eigenvectors per workgroup, by blocks of 16 reflectors
+// from the last to the first: H_15 .. H_0 = I - V M V^T with M the transpose of the
+// triangular factor of the compact WY form (R. Schreiber and C. Van Loan, SIAM J.
+// Sci. Stat. Comput. 10, 53 (1989)), H_0 the block's last column.  Each wavefront
+// holds a quarter of the rows, in tiles of 16 dealt in turn, as accumulators of
+// the matrix instruction, whose registers are also the right operand of V^T Z;
+// V comes from global memory in the layout of that product (the next block
+// meanwhile: two ahead are no faster) and goes through LDS to the layout of the
+// update.  Then the strip is solved with L^T in LDS.  768 orbitals, us: 556 with
+// the reflectors applied one by one (a sum across the wavefront each; 535 four at
+// a time), 412 now, of which the solve is 160, reads of V not hidden 90; 26
+// orbitals 20 and 11.
+constexpr int WP = 18;   // row length of a staged tile of V (doubles; banks)
+
 template <int R>
 __global__ void __launch_bounds__(256) k_eig_back(const EigMol *mols, const double *Z,
-                                                  const double *V, const double *tau,
-                                                  const double *L, const double *eval,
-                                                  double *C, double *ev, const int *info)
+                                                  const double *V, const double *L,
+                                                  const double *eval, double *C, double *ev,
+                                                  const int *info)
 {
     extern __shared__ double X[];
     const EigMol M = mols[blockIdx.y];
     const int n = M.n, c0 = 16 * blockIdx.x;
     if (c0 >= n || info[M.mol] == 1) return;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, lk = lane >> 4;
     if (info[M.mol] != 0) {  // non-finite input
         const double nan = __longlong_as_double(0x7ff8000000000000LL);
         for (int c = 0; c < 16 && c0 + c < n; ++c)
@@ -1580,82 +1646,100 @@ __global__ void __launch_bounds__(256) k_eig_back(const EigMol *mols, const doub
         return;
     }
     if (tid < 16 && c0 + tid < n) ev[M.a0 + c0 + tid] = eval[M.a0 + c0 + tid];
-    const double *Zm = Z + M.w0, *Vm = V + M.w0, *tm = tau + M.a0;
+    const double *Zm = Z + M.w0, *Vm = V + M.w0;
     const int rows = (n + NB - 1) / NB * NB;  // <= 64 R
-    double z[4][R];
+    // tile t: rows 64 t + 16 wv ..; register r of lane (lk, li): row 4 lk + r, column li
+    const int row0 = 16 * wv + 4 * lk;
+    dbl4 z[R];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int t = 0; t < R; ++t)
 #pragma unroll
-        for (int r = 0; r < R; ++r) z[c][r] = ldg(Zm, n, lane + 64 * r, c0 + 4 * wv + c);
-    // panel q: reflectors n - 3 - BP q - b, b = 0 .. BP - 1 (two per wavefront)
-    constexpr int RS = R < 4 ? R : 4;
-    double px[BP / 4][R], ptau = 0.0;
-    __shared__ double pt[2][BP];
-    auto fetch = [&](int q) {
+        for (int r = 0; r < 4; ++r) z[t][r] = ldg(Zm, n, row0 + 64 * t + r, c0 + li);
+    double *stage = X + wv * (R * WB * WP), *red = X + 4 * (R * WB * WP);
+    double px[R][4], pm[4];
+    // block g: V of reflector kmax - li in the tile's rows, -M[li][4 s + lk]
+    auto fetch = [&](int g) {
+        const int kmax = n - 3 - WB * g, k = kmax - li;
+        const double *col = Vm + (long long)max(k, 0) * n;
 #pragma unroll
-        for (int b = 0; b < BP / 4; ++b) {
-            const int k = n - 3 - BP * q - (wv + 4 * b);
+        for (int t = 0; t < R; ++t)
+            if (64 * t + 64 > kmax - WB + 2) {  // uniform: V is zero in the rows above
+                const double *src = col + min(row0 + 64 * t, n - 1);  // at most 3 past: in V
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int row = lane + 64 * r;
-                px[b][r] = (k >= 0 && row > k && row < n) ? Vm[row + (long long)k * n] : 0.0;
+                for (int r = 0; r < 4; ++r) px[t][r] = src[r];
             }
+        const int m = min(WB, kmax + 1);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int c = 4 * s + lk;
+            const double x = Vm[max(li - c, 0) + (long long)max(kmax - c, 0) * n];
+            pm[s] = (li >= c && li < m) ? -x : 0.0;
         }
-        const int k = n - 3 - BP * q - tid;
-        if (tid < BP && k >= 0) ptau = tm[k];
     };
-    const int npan = n > 2 ? (n - 2 + BP - 1) / BP : 0;
-    if (npan > 0) fetch(0);
-    for (int q = 0; q < npan; ++q) {
-        double *P = X + (q & 1) * BP * 64 * R;
+    const int nblk = n > 2 ? (n - 2 + WB - 1) / WB : 0;
+    if (nblk > 0) fetch(0);
+    for (int g = 0; g < nblk; ++g) {
+        const int kmax = n - 3 - WB * g, k = kmax - li, low = kmax - WB + 2;
+        dbl4 w0 = dbl4{0.0, 0.0, 0.0, 0.0}, w1 = w0;
 #pragma unroll
-        for (int b = 0; b < BP / 4; ++b)
+        for (int t = 0; t < R; ++t)
+            if (64 * t + 64 > low) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) P[(wv + 4 * b) * 64 * R + lane + 64 * r] = px[b][r];
-        if (tid < BP) pt[q & 1][tid] = ptau;
-        __syncthreads();  // also: the panel before this one is done with
-        if (q + 1 < npan) fetch(q + 1);
-        for (int b = 0; b < BP; ++b) {
-            const int k = n - 3 - BP * q - b;
-            if (k < 0) break;
-            const double tk = pt[q & 1][b];
-            const double *pv = P + b * 64 * R + lane;
-            // v is zero above row k: blocks of RS registers of rows there are left out
-            double v[R], s[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-            for (int g = 0; g < R; g += RS)
-                if (64 * (g + RS) > k) {  // uniform
-#pragma unroll
-                    for (int r = g; r < g + RS; ++r) v[r] = pv[64 * r];
-#pragma unroll
-                    for (int r = g; r < g + RS; ++r)
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) s[c] += v[r] * z[c][r];
+                for (int r = 0; r < 4; ++r) {
+                    const int row = row0 + 64 * t + r;
+                    px[t][r] = (k >= 0 && row > k && row < n) ? px[t][r] : 0.0;
                 }
-            wsum4(s);
+                double2 *st = reinterpret_cast<double2 *>(stage + (t * WB + li) * WP + 4 * lk);
+                st[0] = make_double2(px[t][0], px[t][1]);
+                st[1] = make_double2(px[t][2], px[t][3]);
+                w0 = mfma(px[t][0], z[t][0], w0);
+                w1 = mfma(px[t][1], z[t][1], w1);
+                w0 = mfma(px[t][2], z[t][2], w0);
+                w1 = mfma(px[t][3], z[t][3], w1);
+            }
+        double a[4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) s[c] *= tk;
+        for (int s = 0; s < 4; ++s) a[s] = pm[s];
+        if (g + 1 < nblk) fetch(g + 1);
 #pragma unroll
-            for (int g = 0; g < R; g += RS)
-                if (64 * (g + RS) > k) {
+        for (int r = 0; r < 4; ++r) red[(wv * 4 + r) * 64 + lane] = w0[r] + w1[r];
+        __syncthreads();
+        dbl4 w, y = dbl4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-                    for (int r = g; r < g + RS; ++r)
+        for (int r = 0; r < 4; ++r)
+            w[r] = red[r * 64 + lane] + red[(4 + r) * 64 + lane] + red[(8 + r) * 64 + lane] +
+                   red[(12 + r) * 64 + lane];
+        __syncthreads();  // red is read before the next block's
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) z[c][r] -= s[c] * v[r];
-                }
-        }
+        for (int s = 0; s < 4; ++s) y = mfma(a[s], w[s], y);
+        // rows of the update's accumulators are 4 lk + r: row of operand lane li
+        const double *sv = stage + lk * WP + 4 * (li & 3) + (li >> 2);
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+            if (64 * t + 64 > low) {
+#pragma unroll
+                for (int s = 0; s < 4; ++s) z[t] = mfma(sv[(t * WB + 4 * s) * WP], y[s], z[t]);
+            }
     }
     __syncthreads();
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
+    for (int t = 0; t < R; ++t)
 #pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (lane + 64 * r < rows) X[(lane + 64 * r) * XS + 4 * wv + c] = z[c][r];
+        for (int r = 0; r < 4; ++r)
+            if (row0 + 64 * t + r < rows) X[(row0 + 64 * t + r) * XS + li] = z[t][r];
     __syncthreads();
     strip_solve<false>(L + M.w0, n, X);
     for (int c = 0; c < 16 && c0 + c < n; ++c)
         for (int r = tid; r < n; r += 256) C[M.d0 + r + (long long)(c0 + c) * n] = X[r * XS + c];
 }
+
+// LDS of k_eig_back<R>: the strip (64 R rows), or the block of reflectors and the
+// partial products before it
+constexpr size_t back_lds(size_t R)
+{
+    return sizeof(double) * std::max(XS * 64 * R, 4 * R * WB * WP + 16 * 64);
+}
+static_assert(back_lds(TBX_EIG_MAXN / 64) <= 160 * 1024, "LDS of a CU");
 
 template <class F>
 hipError_t allow_lds(F f, size_t bytes)
@@ -1683,9 +1767,10 @@ extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, in
     hipError_t e = hipSuccess;
     if ((e = allow_lds(k_eig_trsm<false>, lds_max)) || (e = allow_lds(k_eig_trsm<true>, lds_max)) ||
         (e = allow_lds(k_dc_leaf, lds_leaf)) ||
-        (e = allow_lds(k_dc_prep, prep_max)) || (e = allow_lds(k_eig_back<2>, lds_max)) ||
-        (e = allow_lds(k_eig_back<4>, lds_max)) || (e = allow_lds(k_eig_back<8>, lds_max)) ||
-        (e = allow_lds(k_eig_back<12>, lds_max)) || (e = allow_lds(k_eig_back<16>, lds_max)))
+        (e = allow_lds(k_dc_prep, prep_max)) || (e = allow_lds(k_eig_back<2>, back_lds(2))) ||
+        (e = allow_lds(k_eig_back<4>, back_lds(4))) || (e = allow_lds(k_eig_back<8>, back_lds(8))) ||
+        (e = allow_lds(k_eig_back<12>, back_lds(12))) ||
+        (e = allow_lds(k_eig_back<16>, back_lds(16))))
         return e;
     (void)hipGetLastError();
     double *B0 = wk->m[0], *B1 = wk->m[1], *B2 = wk->m[2], *B3 = wk->m[3];
@@ -1722,8 +1807,9 @@ extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, in
     // eigenvectors by parity in B2, B3
     int levels = 0;
     while (((nmax + (1 << levels) - 1) >> levels) > TBX_DC_LEAF) ++levels;
-    hipLaunchKernelGGL(k_dc_leaf, dim3(1 << levels, nm), dim3(256), lds_leaf, s, mols, wk->d,
-                       wk->e, wk->ev, B2, B3, wk->anorm, info);
+    const int leaves = 1 << levels, wy = nmax > 2 ? (nmax - 2 + WB - 1) / WB : 0;
+    hipLaunchKernelGGL(k_dc_leaf, dim3(leaves + wy, nm), dim3(256), lds_leaf, s, mols, wk->d,
+                       wk->e, wk->ev, B2, B3, wk->anorm, leaves, B0, wk->tau, info);
     DcPtr D{};
     D.q[0] = B2;
     D.q[1] = B3;
@@ -1764,16 +1850,14 @@ extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, in
         if (m1 <= m0) continue;
         const int nx = n_host[m0];
         const dim3 grid((nx + 15) / 16, m1 - m0);
-        // the strip, or two panels of reflectors before it
-        const size_t lds = sizeof(double) * std::max(XS * ((nx + NB - 1) / NB * NB),
-                                                     2 * BP * 64 * cap[q]);
+        const size_t lds = back_lds(cap[q]);
         const EigMol *mm = mols + m0;
         switch (cap[q]) {
-        case 16: hipLaunchKernelGGL(k_eig_back<16>, grid, dim3(256), lds, s, mm, B2, B0, wk->tau, B1, wk->ev, H, ev, info); break;
-        case 12: hipLaunchKernelGGL(k_eig_back<12>, grid, dim3(256), lds, s, mm, B2, B0, wk->tau, B1, wk->ev, H, ev, info); break;
-        case 8: hipLaunchKernelGGL(k_eig_back<8>, grid, dim3(256), lds, s, mm, B2, B0, wk->tau, B1, wk->ev, H, ev, info); break;
-        case 4: hipLaunchKernelGGL(k_eig_back<4>, grid, dim3(256), lds, s, mm, B2, B0, wk->tau, B1, wk->ev, H, ev, info); break;
-        default: hipLaunchKernelGGL(k_eig_back<2>, grid, dim3(256), lds, s, mm, B2, B0, wk->tau, B1, wk->ev, H, ev, info); break;
+        case 16: hipLaunchKernelGGL(k_eig_back<16>, grid, dim3(256), lds, s, mm, B2, B0, B1, wk->ev, H, ev, info); break;
+        case 12: hipLaunchKernelGGL(k_eig_back<12>, grid, dim3(256), lds, s, mm, B2, B0, B1, wk->ev, H, ev, info); break;
+        case 8: hipLaunchKernelGGL(k_eig_back<8>, grid, dim3(256), lds, s, mm, B2, B0, B1, wk->ev, H, ev, info); break;
+        case 4: hipLaunchKernelGGL(k_eig_back<4>, grid, dim3(256), lds, s, mm, B2, B0, B1, wk->ev, H, ev, info); break;
+        default: hipLaunchKernelGGL(k_eig_back<2>, grid, dim3(256), lds, s, mm, B2, B0, B1, wk->ev, H, ev, info); break;
         }
         m0 = m1;
     }
