@@ -417,7 +417,7 @@ def main():
     # Fermi filling, the density products (FP64 MFMA; P is symmetric, so the
     # algorithmic FLOP is that of a symmetric rank-nao product, nao^2 (nao + 1)
     # per molecule and matrix), and the generalized eigensolver on a sample
-    # (one rocSOLVER dsygvd call per molecule)
+    # (molecules of up to 1024 orbitals in the same launches)
     def ev_ms(fn, reps=5):
         fn()
         torch.cuda.synchronize()

@@ -358,12 +358,15 @@ int tbx_batch_last_scf_timing(const tbx_batch *b, double *ms);
  * energies and occupations [nao] at ao_off[m].  One spin channel per call
  * (the reference loops over spins, scf/diag.f90:62-108). */
 /* sygvd (lapack/sygvd.f90, scf/diag.f90:84): H C = S C diag(eval) for every
- * molecule through rocSOLVER's dsygvd; d_H is overwritten with the
+ * molecule, those of up to 1024 orbitals together and larger ones through
+ * rocSOLVER's dsygvd one by one; d_H is overwritten with the
  * S-orthonormal eigenvectors C, d_eval [nao] with the ascending eigenvalues;
  * d_S is left unchanged (solved on a copy the batch holds).  Synchronises
  * the stream; TBX_ERR_ARG names a molecule whose S is not positive
- * definite.  rocSOLVER's own workspace is allocated by rocBLAS and is not
- * counted against tbx_context_set_memory_limit. */
+ * definite.  The workspace (four n x n matrices per molecule solved
+ * together, at most 2^24 elements each) shrinks under
+ * tbx_context_set_memory_limit; rocSOLVER's own is allocated by rocBLAS and
+ * is not counted. */
 int tbx_batch_sygvd(tbx_batch *b, double *d_H, const double *d_S, double *d_eval, void *stream);
 /* get_fermi_filling (wavefunction/fermi.f90:31-117) for every molecule:
  * d_nel [nmol] electrons of this spin channel, kt (hartree), d_emo [nao]
