@@ -17,9 +17,11 @@
 // about once per molecule and re-read from L2.  Zero padding covers rows and
 // k beyond nao.  Orbitals with an occupation of exactly zero are left out of
 // the products.  256 molecules of 8..256 atoms, 53 % of the orbitals occupied:
-// 361 us with each load waiting for the one before it, 282 us without, 222 us
-// without the empty orbitals; the matrix cores alone would need 70 us, the
-// look at the empty orbitals takes 37, the stores 17 (panels of 32 columns: 249).
+// 361 us with each load waiting for the one before it, 282 us without, 220 us
+// without the empty orbitals, 196 us with the look at these (the high words
+// alone) beside the products instead of after them; the matrix cores alone would
+// need 70 us, the stores take 17 (panels of 32 columns: 249 against 222; 3
+// workgroups a CU instead of 4: 204).
 #include <hip/hip_runtime.h>
 
 #include "tbx_tables.h"
@@ -58,7 +60,7 @@ __device__ void poison_rows(const TbxMols &mt, int m, const double *Cm, const do
 // four wavefronts compute its 32 x 32 quarters from panels of C staged in LDS
 // (64 rows x KB columns for each factor, the left one scaled by f_k), each
 // panel loaded by the whole workgroup while the products run on the previous one.
-__global__ void __launch_bounds__(256) k_density(TbxMols mt, const double *__restrict__ C,
+__global__ void __launch_bounds__(256, 4) k_density(TbxMols mt, const double *__restrict__ C,
                                                  const double *__restrict__ focc,
                                                  const double *__restrict__ eval,
                                                  double *__restrict__ P)
@@ -94,7 +96,7 @@ __global__ void __launch_bounds__(256) k_density(TbxMols mt, const double *__res
         ia[q] = min(R0 + rr + 16 * q, n - 1);
         ib[q] = min(C0 + rr + 16 * q, n - 1);
     }
-    double pois = 0.0;  // NaN once a skipped element is not finite
+    int worst = 0;  // largest magnitude (high word) of a skipped element
     for (int kc = 0; kc < n; kc += 256) {
         const int kt = kc + tid;
         double ft = 0.0;
@@ -136,6 +138,21 @@ __global__ void __launch_bounds__(256) k_density(TbxMols mt, const double *__res
                 pb[q] = col[ib[q]];
             }
         };
+        // skipped columns: the high words alone, a panel of them beside each panel
+        // of the product, read while that is multiplied
+        int cw[8], u0 = 0;
+        auto peek = [&](int u) {
+            const int *col = reinterpret_cast<const int *>(Cm + (long long)sl[min(u + kk, ns - 1)] * n) + 1;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                cw[q] = col[2 * ia[q]];
+                cw[4 + q] = col[2 * ib[q]];
+            }
+        };
+        auto note = [&]() {
+#pragma unroll
+            for (int q = 0; q < 8; ++q) worst = max(worst, cw[q] & 0x7fffffff);
+        };
         if (nk > 0) load(0);
         for (int k0 = 0; k0 < nk; k0 += KB) {
             __syncthreads();  // the products of the previous panel are done
@@ -148,6 +165,8 @@ __global__ void __launch_bounds__(256) k_density(TbxMols mt, const double *__res
             }
             __syncthreads();
             if (k0 + KB < nk) load(k0 + KB);
+            const bool look = u0 < ns;
+            if (look) peek(u0);
 #pragma unroll
             for (int ks = 0; ks < KB; ks += 4) {
                 double a[2], b[2];
@@ -163,15 +182,18 @@ __global__ void __launch_bounds__(256) k_density(TbxMols mt, const double *__res
                         acc[s][u] =
                             __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], b[u], acc[s][u], 0, 0, 0);
             }
+            if (look) {
+                note();
+                u0 += KB;
+            }
         }
 #pragma unroll 2
-        for (int u0 = 0; u0 < ns; u0 += KB) {
-            const double *col = Cm + (long long)sl[min(u0 + kk, ns - 1)] * n;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) pois += 0.0 * col[ia[q]] + 0.0 * col[ib[q]];
+        for (; u0 < ns; u0 += KB) {
+            peek(u0);
+            note();
         }
     }
-    if (__syncthreads_or(pois != 0.0)) poison_rows(mt, m, Cm, focc, eval, R0, C0, acc, sr, sc);
+    if (__syncthreads_or(worst >= 0x7ff00000)) poison_rows(mt, m, Cm, focc, eval, R0, C0, acc, sr, sc);
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
