@@ -11,10 +11,10 @@
 // without forming either array:
 //   dE/dR_i  += sum_{j,T} (dEdcn_i + dEdcn_j) f'(r) v / r,   v = R_i - R_j - T
 //   sigma_m  += sum_{i in m} dEdcn_i sum_{j,T} f'(r) v v^T / r.
-// One or four wavefronts per atom i; their lanes walk the atoms j of i's
+// One, two or four wavefronts per atom i; their lanes walk the atoms j of i's
 // molecule and the molecule's translations.  Every sum over j is a reduction
 // within the workgroup, so cn and dE/dR need no atomics; sigma is summed per
-// molecule with FP64 atomics (nine per atom).
+// molecule with FP64 atomics (nine per workgroup and molecule).
 #include <hip/hip_runtime.h>
 
 #include "tbx_tables.h"
@@ -61,7 +61,8 @@ __device__ __forceinline__ void dexp_count(const CnPar &c, double r2, double r0,
 // wavefronts.  One wavefront per atom and a loop over the translations left
 // the lanes beyond the cell's atoms idle and ran the exponentials for each
 // translation: 6 crystals of 6..96 atoms 127 us (cn) and 145 us (gradient), now
-// 13 and 15; 1536 atoms 21 and 43 us, now 15 and 29.  W = 4 where an atom has enough pairs to share (tbx_launch_ncoord).
+// 13 and 15; 1536 atoms 21 and 43 us, now 15 and 22.  W > 1 where an atom has
+// enough pairs to share (tbx_launch_ncoord).
 constexpr int QN = 128;  // queue entries per wavefront
 struct Queue {
     double v[3][QN];
@@ -152,69 +153,70 @@ __device__ __forceinline__ void atom_sums(const TbxMols &mt, const CnPar &c, con
     if (lane < nq) add(q.v[0][lane], q.v[1][lane], q.v[2][lane], q.j[lane]);
 }
 
-// Sums over the wavefront, then over the W wavefronts of the atom; on lane 0
-// of its first one.
-template <int W, int N>
-__device__ __forceinline__ void reduce(double (&sum)[N], int wv, double (*part)[9])
-{
-#pragma unroll
-    for (int k = 0; k < N; ++k) sum[k] = wave_sum(sum[k]);
-    if (W == 1) return;
-    if ((threadIdx.x & 63) == 0) {
-#pragma unroll
-        for (int k = 0; k < N; ++k) part[wv][k] = sum[k];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < N; ++k) {
-        sum[k] = 0.0;
-#pragma unroll
-        for (int w = 0; w < W; ++w) sum[k] += part[w][k];
-    }
-}
-
 template <int W>
 __global__ void __launch_bounds__(256) k_ncoord(TbxMols mt, CnPar c, const double *xyz,
                                                 double *cn)
 {
     __shared__ Queue q[4];
-    __shared__ double part[4][9];
+    __shared__ double part[4];
     const int i = W == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
     const int wv = W == 1 ? 0 : threadIdx.x >> 6;
     if (i >= mt.nat) return;  // whole atoms leave together
     double sum[1] = {0.0};
     atom_sums<false, W>(mt, c, xyz, nullptr, i, wv, q[threadIdx.x >> 6], sum);
-    reduce<W>(sum, wv, part);
+    sum[0] = wave_sum(sum[0]);
+    if (W > 1) {
+        if ((threadIdx.x & 63) == 0) part[wv] = sum[0];
+        __syncthreads();
+        sum[0] = (part[0] + part[1]) + (part[2] + part[3]);
+    }
     if ((threadIdx.x & 63) == 0 && wv == 0) cn[i] = sum[0];
 }
 
 // dE/dR (accumulated into grad) and sigma (accumulated, per molecule) from
-// dE/dcn
-template <int W>
-__global__ void __launch_bounds__(256) k_ncoord_grad(TbxMols mt, CnPar c, const double *xyz,
-                                                     const double *dEdcn, double *grad,
-                                                     double *sigma)
+// dE/dcn, A atoms of W wavefronts a workgroup.  The workgroup's atoms of one
+// molecule add to its sigma together: nine atomics an atom to the same nine
+// addresses were 10 of 29 us for 1536 atoms of one molecule, 11 of 25 us for 8
+// clusters of 200 to 500 (now 14.6).
+template <int W, int A>
+__global__ void __launch_bounds__(64 * W * A) k_ncoord_grad(TbxMols mt, CnPar c, const double *xyz,
+                                                            const double *dEdcn, double *grad,
+                                                            double *sigma)
 {
-    __shared__ Queue q[4];
-    __shared__ double part[4][9];
-    const int i = W == 1 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x;
-    const int wv = W == 1 ? 0 : threadIdx.x >> 6, lane = threadIdx.x & 63;
-    if (i >= mt.nat) return;
+    __shared__ Queue q[W * A];
+    __shared__ double part[W * A][9];
+    __shared__ int mol[A];
+    const int wave = threadIdx.x >> 6, slot = wave / W, i0 = blockIdx.x * A, i = i0 + slot;
     double sum[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    atom_sums<true, W>(mt, c, xyz, dEdcn, i, wv, q[threadIdx.x >> 6], sum);
-    reduce<W>(sum, wv, part);
-    if (wv != 0) return;
-    if (lane == 0) {
+    if (i < mt.nat) atom_sums<true, W>(mt, c, xyz, dEdcn, i, wave - slot * W, q[wave], sum);
 #pragma unroll
-        for (int k = 0; k < 3; ++k) grad[3 * i + k] += sum[k];
+    for (int k = 0; k < 9; ++k) sum[k] = wave_sum(sum[k]);
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) part[wave][k] = sum[k];
+        if (wave == slot * W) mol[slot] = i < mt.nat ? mt.at_mol[i] : -1;
     }
-    // sigma (3, 3) column-major from the packed symmetric sums
-    if (lane < 9) {
-        static constexpr int kPack[9] = {0, 1, 3, 1, 2, 4, 3, 4, 5};
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < 3 * A && i0 + t / 3 < mt.nat) {
         double v = 0.0;
 #pragma unroll
-        for (int k = 0; k < 9; ++k) v = (lane == k) ? sum[3 + kPack[k]] : v;
-        if (v != 0.0) unsafeAtomicAdd(&sigma[9 * mt.at_mol[i] + lane], v);
+        for (int w = 0; w < W; ++w) v += part[t / 3 * W + w][t % 3];
+        grad[3 * i0 + t] += v;
+    }
+    // sigma (3, 3) column-major from the packed symmetric sums, by the first
+    // atom of each molecule
+    if (t >= 64 && t < 64 + 9 * A) {
+        const int a = (t - 64) / 9, e = (t - 64) % 9, m = mol[a];
+        if (m >= 0 && (a == 0 || mol[a - 1] != m)) {
+            const int r = e % 3, col = e / 3, lo = min(r, col), hi = max(r, col);
+            const int k = 3 + hi * (hi + 1) / 2 + lo;  // xx xy yy xz yz zz
+            double v = 0.0;
+            for (int b = a; b < A && mol[b] == m; ++b)
+#pragma unroll
+                for (int w = 0; w < W; ++w) v += part[b * W + w][k];
+            if (v != 0.0) unsafeAtomicAdd(&sigma[9 * m + e], v);
+        }
     }
 }
 
@@ -248,11 +250,19 @@ extern "C" hipError_t tbx_launch_ncoord_grad(const TbxMols *mol, const double *r
     if (mol->nat <= 0) return hipSuccess;
     const CnPar c{rcov, ka, kb, rshift, cutoff * cutoff};
     (void)hipGetLastError();
-    if (share_atoms(mol))
-        hipLaunchKernelGGL(k_ncoord_grad<4>, dim3(mol->nat), dim3(256), 0, stream, *mol, c, xyz,
-                           dEdcn, grad, sigma);
-    else
-        hipLaunchKernelGGL(k_ncoord_grad<1>, dim3((mol->nat + 3) / 4), dim3(256), 0, stream, *mol,
+    // From 1024 atoms with many pairs two atoms of two wavefronts fill the chip and
+    // halve the atomics: 1536 atoms 21.8 us, one atom of four wavefronts 29.0, two
+    // 22.7, four 28.5.  Below, one atom of four: 6 crystals of 6 to 96 atoms 15.1 us
+    // (four atoms a workgroup 26).
+    const unsigned nat = mol->nat;
+    if (!share_atoms(mol))
+        hipLaunchKernelGGL((k_ncoord_grad<1, 4>), dim3((nat + 3) / 4), dim3(256), 0, stream, *mol,
                            c, xyz, dEdcn, grad, sigma);
+    else if (nat >= 1024)
+        hipLaunchKernelGGL((k_ncoord_grad<2, 2>), dim3((nat + 1) / 2), dim3(256), 0, stream, *mol,
+                           c, xyz, dEdcn, grad, sigma);
+    else
+        hipLaunchKernelGGL((k_ncoord_grad<4, 1>), dim3(nat), dim3(256), 0, stream, *mol, c, xyz,
+                           dEdcn, grad, sigma);
     return hipGetLastError();
 }
