@@ -1233,19 +1233,31 @@ __global__ void __launch_bounds__(256) k_dc_leaf(const EigMol *mols, const doubl
             // the entries of the columns' segments, which are also their rows
             const int klo = W.lo[sc], khi = W.hi[min(sc + 31, N - 1)];
             const int kend = sr < khi && sr + 32 > klo ? khi : klo;
-            for (int ks = klo & ~3; ks < kend; ks += 4) {
-                const int kk = ks + lk;
-                const double *qc = Q + (kk < N ? W.idx[kk] : 0) * LQ;
-                double x[2], y[2];
+            // sixteen entries at a time, their columns' indices, then their
+            // operands under way together (U is zero outside the segment): 39
+            // against 59 thousand cycles over the six merges of 50 rows with an
+            // index, its operands and its products at a time
+            for (int ks = klo & ~15; ks < kend; ks += 16) {
+                int col[4];
+                double x[4][2], y[4][2];
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    x[u] = qc[sr + 16 * u + li];
-                    y[u] = W.U[(sc + 16 * u + li) * LQ + kk];  // zero for kk >= N
+                for (int p = 0; p < 4; ++p) {
+                    const int kk = ks + 4 * p + lk;
+                    col[p] = W.idx[min(kk, N - 1)];
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) y[p][u] = W.U[(sc + 16 * u + li) * LQ + kk];
                 }
 #pragma unroll
-                for (int u = 0; u < 2; ++u)
+                for (int p = 0; p < 4; ++p)
 #pragma unroll
-                    for (int q = 0; q < 2; ++q) acc[u][q] = mfma(x[u], y[q], acc[u][q]);
+                    for (int u = 0; u < 2; ++u) x[p][u] = Q[col[p] * LQ + sr + 16 * u + li];
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+#pragma unroll
+                    for (int u = 0; u < 2; ++u)
+#pragma unroll
+                        for (int q = 0; q < 2; ++q)
+                            acc[u][q] = mfma(x[p][u], y[p][q], acc[u][q]);
             }
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
