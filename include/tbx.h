@@ -420,6 +420,17 @@ int tbx_batch_get_tiles(const tbx_batch *b, tbx_tiles *tiles);
  * order.  Rebuilds the units (host) and waits for the whole device (every
  * stream) before it replaces them. */
 int tbx_batch_order_pairs(tbx_batch *b, const double *xyz, double skin);
+/* The same where it pays: a batch of few work units (up to 768 of either
+ * kind), all of which the device runs at once, keeps its present order, since
+ * checking the hint would cost more than the skipped units.  xyz and skin are
+ * checked either way. */
+int tbx_batch_order_pairs_if_large(tbx_batch *b, const double *xyz, double skin);
+/* Work units of the present order: those holding a pair within cutoff + skin
+ * at the hint (all units without a hint), and the others. */
+typedef struct {
+    long long fwd_near, fwd_far, grad_near, grad_far;
+} tbx_unit_counts;
+int tbx_batch_unit_counts(const tbx_batch *b, tbx_unit_counts *n);
 
 /* Work-unit plans of a batch description, built on the host only (no
  * context, no device) with `tiles` (NULL: the defaults), and checked against

@@ -103,7 +103,8 @@ class Batch:
     """Batched GFN2 S/D/Q/H0 + gradient for a list of ``(numbers, xyz_bohr)``.
 
     ``order_pairs``: order the atom pairs of the work units near-first by the
-    given geometry (``order_pairs()``); it changes the speed, not the results.
+    given geometry (``order_pairs()``) where the batch has enough units for it
+    to pay; it changes the speed, not the results.
     ``lattices``: optional, one entry per structure, ``None`` for a molecule
     or ``(periodic[3], lattice)`` with the lattice vectors as the rows of
     ``lattice`` (bohr); each periodic structure then sums over its lattice
@@ -163,7 +164,7 @@ class Batch:
         self.rcov = np.array([params.covalent_rad(int(z)) for z in self.nums])
         self.set_ncoord(self.rcov)
         if order_pairs:
-            self.order_pairs(self.xyz0, skin)
+            self._order_pairs(L.lib().tbx_batch_order_pairs_if_large, self.xyz0, skin)
 
     def _shell_tables(self):
         spec = self.spec
@@ -411,14 +412,24 @@ class Batch:
         kernels skip while their pairs stay beyond the cutoff.  Every pair is
         still screened on the device, so any geometry gives the same results;
         ``xyz=None`` restores the geometry-independent order."""
+        self._order_pairs(L.lib().tbx_batch_order_pairs, xyz, skin)
+
+    def _order_pairs(self, entry, xyz, skin):
         x = None
         if xyz is not None:
             if isinstance(xyz, torch.Tensor):
                 xyz = xyz.detach().cpu().numpy()
             x = np.ascontiguousarray(np.asarray(xyz, dtype=np.float64).reshape(-1))
             assert x.size == 3 * self.nat
-        L.check(L.lib().tbx_batch_order_pairs(
-            self.handle, None if x is None else x.ctypes.data_as(ct.c_void_p), float(skin)))
+        L.check(entry(self.handle, None if x is None else x.ctypes.data_as(ct.c_void_p),
+                      float(skin)))
+
+    def unit_counts(self) -> dict:
+        """Work units of the present pair order, forward and gradient: those with
+        a pair within cutoff + skin at the hint, and the others."""
+        n = L.UnitCounts()
+        L.check(L.lib().tbx_batch_unit_counts(self.handle, ct.byref(n)))
+        return {f: getattr(n, f) for f, _ in L.UnitCounts._fields_}
 
     def tiles(self) -> dict:
         """Current tile shapes (work-unit caps and chunk lengths) of the kernels."""

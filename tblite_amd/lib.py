@@ -66,6 +66,10 @@ class Tiles(ct.Structure):
                 ("grad_chunk", ct.c_int), ("fwd_band", ct.c_int), ("grad_band", ct.c_int)]
 
 
+class UnitCounts(ct.Structure):
+    _fields_ = [(n, ct.c_longlong) for n in ("fwd_near", "fwd_far", "grad_near", "grad_far")]
+
+
 class PlanStats(ct.Structure):
     _fields_ = [(n, ct.c_longlong) for n in (
         "nunit_fwd", "nunit_grad", "npair_fwd", "npair_grad", "ntask_fwd", "ntask_grad",
@@ -124,6 +128,8 @@ _SIGS = {
     "tbx_batch_plan_stats": (ct.c_int, [ct.POINTER(BatchDesc), ct.POINTER(Tiles), _P,
                                         ct.c_double, ct.POINTER(PlanStats)]),
     "tbx_batch_order_pairs": (ct.c_int, [_P, _P, ct.c_double]),
+    "tbx_batch_order_pairs_if_large": (ct.c_int, [_P, _P, ct.c_double]),
+    "tbx_batch_unit_counts": (ct.c_int, [_P, ct.POINTER(UnitCounts)]),
     "tbx_batch_sygvd": (ct.c_int, [_P, _P, _P, _P, _P]),
     "tbx_batch_fermi_filling": (ct.c_int, [_P, _P, ct.c_double, _P, _P, _P, _P]),
     "tbx_batch_get_density_matrix": (ct.c_int, [_P, _P, _P, _P, _P]),
