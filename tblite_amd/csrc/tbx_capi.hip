@@ -625,7 +625,7 @@ static bool build_plans(const HostSpecies &hs, const HostMols &hm, const std::ve
 // pairs, the zero units of their elements, molecule by molecule and in equal
 // shares along each, so that stores and arithmetic run side by side on every CU
 // and both touch a molecule's columns at about the same time.  Outputs with
-// lattice images are zeroed before the launch and need no zero units.
+// several translations are zeroed before the launch and need no zero units.
 static void build_forward_launch(const HostSpecies &hs, HostMols &hm,
                                  const std::vector<TbxUnitHead> &near)
 {
@@ -645,6 +645,8 @@ static void build_forward_launch(const HostSpecies &hs, HostMols &hm,
             x[c].resize(n);
             for (int j = 0; j < n; ++j) x[c][j] = hm.hint_xyz[3 * (a0 + j) + c];
         }
+        const int itr = hm.mol_tr[m].x;  // the structure's one translation
+        const double T[3] = {hm.trans[3 * itr], hm.trans[3 * itr + 1], hm.trans[3 * itr + 2]};
         far.assign(n + 1, 0);  // ends with a pair that is not far
         zero.clear();
         int elems = TBX_ZERO_ELEMS;
@@ -670,12 +672,24 @@ static void build_forward_launch(const HostSpecies &hs, HostMols &hm,
         };
         for (int i = 0; i < n; ++i) {
             const double p[3] = {x[0][i], x[1][i], x[2][i]};
-            for (int j = 0; j < n; ++j) {
+            // the pairs of the half list: (i, j) below i, (j, i) above
+            for (int j = 0; j < i; ++j) {
                 double r2 = 0.0;
-                for (int c = 0; c < 3; ++c) r2 += (p[c] - x[c][j]) * (p[c] - x[c][j]);
+                for (int c = 0; c < 3; ++c) {
+                    const double d = p[c] - x[c][j] - T[c];
+                    r2 += d * d;
+                }
                 far[j] = !(r2 <= hm.near2);
             }
-            far[i] = !pair_near(hm, a0 + i, a0 + i, hm.mol_tr[m].x);
+            for (int j = i + 1; j < n; ++j) {
+                double r2 = 0.0;
+                for (int c = 0; c < 3; ++c) {
+                    const double d = x[c][j] - p[c] - T[c];
+                    r2 += d * d;
+                }
+                far[j] = !(r2 <= hm.near2);
+            }
+            far[i] = !pair_near(hm, a0 + i, a0 + i, itr);
             for (int j = 0, j0 = -1; j <= n; ++j) {
                 if (far[j] && j0 < 0) j0 = j;
                 if (!far[j] && j0 >= 0) {

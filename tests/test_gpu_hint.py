@@ -146,3 +146,29 @@ def test_start_order_of_a_batch():
         x[0, 0] = x[0, 0] if bad is None else bad
         with pytest.raises(L.TbxError):
             Batch([(z, x)], skin=skin)
+
+
+def test_one_structure_with_one_nonzero_translation(monkeypatch):
+    """The distance that decides whether a pair is distant is that of its one
+    image: the clusters are 60 bohr apart and the translation brings one onto
+    the other, so pairs of one cluster are distant and pairs of both are near."""
+    from tblite_amd import structure
+    from tblite_amd.batch import Batch
+    monkeypatch.setattr(structure, "get_lattice_points",
+                        lambda *a, **k: np.array([[60.0, 0.5, 0.0]]))
+    z, x = synthetic.water_cluster(14, seed=8)
+    z2, x2 = synthetic.random_molecule(11, np.random.default_rng(6))
+    one = (np.concatenate([z, z2]), np.concatenate([x, x2 + np.array([63.0, 1.0, 2.0])]))
+    b = Batch([one], lattices=[([True] * 3, np.eye(3) * 60.0)])
+    xyz = b.tensor_xyz()
+    se = b.selfenergy(b.ncoord(xyz))[0].contiguous()
+    b.order_pairs(None)
+    ref = b.forward(xyz, se)
+    b.order_pairs(b.xyz0)
+    print(f"[gpu] one translation: {b.unit_counts()}", flush=True)
+    assert b.unit_counts()["fwd_far"] > 0 and ref[0].abs().max() > 1e-3
+    out = tuple(torch.full_like(r, float("nan")) for r in ref)
+    b.forward(xyz, se, out=out)
+    for k, (r, g) in enumerate(zip(ref, out)):
+        assert torch.isfinite(g).all(), k
+        assert torch.abs(r - g).max().item() <= 1e-12, k
