@@ -500,6 +500,57 @@ __device__ __forceinline__ void pair_vec(const TbxMols &mt, const double *xyz, c
     for (int c = 0; c < 3; ++c) v[c] = xyz[3 * pr.i + c] - xyz[3 * pr.j + c] - mt.trans[3 * itr + c];
 }
 
+// Far units, for a hint that no longer holds: most still have no pair within the
+// cutoff.  A wavefront looks at the pairs of FAR_LOOK units (their atoms alone,
+// straight from the plan), a workgroup at FAR_UNITS, dealt to the workgroups in
+// turn, and `run` takes those that may have one (the margin is rounding's: a unit
+// screens its pairs itself).  Units next to each other in one workgroup leave
+// the living ones to a few: the adjoint of 8 clusters of 200 to 500 atoms, all
+// displaced by 0.5 bohr, 211 against 181 us.
+constexpr int FAR_LOOK = 4, FAR_UNITS = 4 * FAR_LOOK;  // four wavefronts
+
+__device__ __forceinline__ bool unit_lives(const TbxMols &mt, const TbxUnitHead &H,
+                                           const int *plan, const double *xyz, double cutoff2)
+{
+    const int npair = H.counts & 255;
+    const int *w = plan + 4 * (long long)H.plan, *ext = w + 4 * ((10 * npair + 3) >> 2);
+    bool live = false;
+    for (int p0 = 0; p0 < npair; p0 += 64) {
+        const int p = min(p0 + (int)(threadIdx.x & 63), npair - 1);
+        PairInfo pr;
+        pr.i = w[10 * p];
+        pr.j = w[10 * p + 1];
+        double v[3];
+        pair_vec(mt, xyz, pr, ext[p], v);
+        live = live || v[0] * v[0] + v[1] * v[1] + v[2] * v[2] <= cutoff2 * (1.0 + 1e-12);
+    }
+    return __any(live);
+}
+
+template <class F>
+__device__ __forceinline__ void far_units(const TbxMols &mt, const TbxUnitHead *units, int n,
+                                          const int *plan, const double *xyz, double cutoff2,
+                                          const F &run)
+{
+    __shared__ int lives[FAR_UNITS];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), step = gridDim.x;
+    for (int u0 = blockIdx.x; u0 < n; u0 += FAR_UNITS * step) {
+#pragma unroll
+        for (int k = 0; k < FAR_LOOK; ++k) {
+            const int q = FAR_LOOK * wv + k, u = u0 + q * step;
+            const bool live = u < n && unit_lives(mt, units[u], plan, xyz, cutoff2);
+            if ((threadIdx.x & 63) == 0) lives[q] = live;
+        }
+        __syncthreads();
+        for (int q = 0; q < FAR_UNITS; ++q)
+            if (lives[q]) {
+                run(u0 + q * step);
+                __syncthreads();  // its LDS is read until its last phase
+            }
+        __syncthreads();  // the answers are read before the next ones
+    }
+}
+
 // Decode task tid of a staged unit: shell pair index, type and Cartesian pair.
 template <class US>
 __device__ __forceinline__ int4 decode_task(const US &U, int task, int &spx)
@@ -929,7 +980,7 @@ __device__ __forceinline__ void diat_block(const double (*acc)[10], const double
 // mirror (rows i, column j: operator shifted to j, xtb/h0.f90:704-747) --
 // every element of the molecule's matrices is written exactly once.  DIAT:
 // off-site H0 blocks from the diatomic-frame scaled overlap (sp.kdiat).
-template <bool DIAT>
+template <bool DIAT, bool FAR>
 __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead &H)
 {
     __shared__ FwdStage U;
@@ -969,7 +1020,8 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
     double v[3];
     const int pl = tid < npair ? tid : 0;
     pair_vec(mt, A.xyz, U.pinf[pl], U.pext[pl], v);
-    const ShellLoad sl = shell_load(sp, U, A.se, tid < nspair ? tid : 0);
+    ShellLoad sl;
+    if (!FAR) sl = shell_load(sp, U, A.se, tid < nspair ? tid : 0);
     if (tid < npair) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) U.pv[tid][c] = v[c];
@@ -988,10 +1040,12 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
         }
     }
     if (!__syncthreads_or(live)) {
-        // outputs with lattice images are zero-filled before the launch
-        if (!accum) far_zero_unit(A, H, U, eoff);
+        // outputs with lattice images are zero-filled before the launch, a far
+        // unit's elements by the zero units
+        if (!FAR && !accum) far_zero_unit(A, H, U, eoff);
         return;
     }
+    if (FAR) sl = shell_load(sp, U, A.se, tid < nspair ? tid : 0);
     // shell pairs: screening counts and H0 factors (one lane per shell pair)
     if (tid < nspair) {
         const int k = tid;
@@ -1194,24 +1248,29 @@ template <bool DIAT>
 __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
 {
     const TbxUnitHead H = A.mol.funit[xcd_unit(blockIdx.x, gridDim.x)];
-    if (H.nel & TBX_UNIT_ZERO) {  // unless the far units run (k_forward_far)
-        if (!__syncthreads_or((int)threadIdx.x < A.nstale ? A.stale[threadIdx.x] : 0))
-            zero_unit(A, H);
+    if (H.nel & TBX_UNIT_ZERO) {
+        zero_unit(A, H);
         return;
     }
-    forward_unit<DIAT>(A, H);
+    forward_unit<DIAT, false>(A, H);
 }
 
 // The forward units of the pairs beyond cutoff + skin at the hint, when an
-// atom has left it (as k_gradient_far).
+// atom has left it (as k_gradient_far).  Their elements are zero by the zero
+// units of k_forward; a unit with a pair within the cutoff writes them anew.
+// Forward of 640 molecules of 8 to 256 atoms with one atom moved by 1 bohr 1593
+// us, all displaced by 0.5 bohr 1662 (hint valid: 1550); with every far unit
+// staged here and its zeros written by it 2142 and 2140; with a hint stretched
+// threefold, most units alive, 2911 and 2622.  (H2O)512, one atom: 211 and 347.
+// The loop keeps the unit's constants in registers, 178 without a bound (236 with
+// DIAT, 40 spilled to fit three wavefronts): at three wavefronts 2911, two 3224.
 template <bool DIAT>
-__global__ void __launch_bounds__(NTHREADS, 2) k_forward_far(FwdArgs A)
+__global__ void __launch_bounds__(NTHREADS, DIAT ? 2 : 3) k_forward_far(FwdArgs A)
 {
+    static_assert(NTHREADS == 256, "four wavefronts");
     if (!__syncthreads_or((int)threadIdx.x < A.nstale ? A.stale[threadIdx.x] : 0)) return;
-    for (int u = blockIdx.x; u < A.mol.nfunit_far; u += gridDim.x) {
-        __syncthreads();  // the previous unit's LDS is read until its last phase
-        forward_unit<DIAT>(A, A.mol.ffunit[u]);
-    }
+    far_units(A.mol, A.mol.ffunit, A.mol.nfunit_far, A.mol.fplan, A.xyz, A.sp.cutoff2,
+              [&](int u) { forward_unit<DIAT, true>(A, A.mol.ffunit[u]); });
 }
 
 // The explicit pair-vector terms of one spherical element (mu on atom j, nu
@@ -2020,16 +2079,18 @@ __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient(GradArgs A)
 // The far gradient units (no pair within cutoff + skin at the pair-order
 // hint): nothing to do while every atom is within skin/2 of its hint
 // position (every answer of k_begin 0), since then every such pair is
-// still beyond the cutoff.  Otherwise the workgroups walk them.
+// still beyond the cutoff.  Otherwise the workgroups look through them: 640
+// molecules of 8 to 256 atoms with one atom moved by 1 bohr, adjoint given S and
+// D 1635 us, 1769 with every far unit staged (hint valid: 1575).
 template <int MODE, bool EX>
 __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient_far(GradArgs A,
                                                                      const int *stale, int nstale)
 {
+    static_assert(GTHREADS == 256, "four wavefronts");
     if (!__syncthreads_or((int)threadIdx.x < nstale ? stale[threadIdx.x] : 0)) return;
-    for (int u = A.mol.nunit_near + blockIdx.x; u < A.mol.nunit; u += gridDim.x) {
-        __syncthreads();  // the previous unit's LDS is read until its last phase
-        gradient_unit<MODE, EX>(A, u);
-    }
+    const int near = A.mol.nunit_near;
+    far_units(A.mol, A.mol.unit + near, A.mol.nunit - near, A.mol.plan, A.xyz, A.sp.cutoff2,
+              [&](int u) { gradient_unit<MODE, EX>(A, near + u); });
 }
 
 // What a launch needs before its main kernel, in one launch (a small molecule's
