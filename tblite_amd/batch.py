@@ -200,9 +200,11 @@ class Batch:
         ent = self._se_tables.get(device)
         if ent is None or not all(np.array_equal(a, b) for a, b in zip(ent[0], src)):
             stream = torch.cuda.current_stream(device) if device.type == "cuda" else None
-            # torch.tensor copies: a CPU tensor must not share the caller's arrays
-            ent = (tuple(np.array(a) for a in src),
-                   tuple(torch.tensor(a, device=device) for a in src), stream)
+            # torch.tensor copies: a CPU tensor must not share the caller's arrays.
+            # Made under inference mode they could never be saved for a backward.
+            with torch.inference_mode(False):
+                ent = (tuple(np.array(a) for a in src),
+                       tuple(torch.tensor(a, device=device) for a in src), stream)
             self._se_tables[device] = ent
         elif ent[2] is not None:
             cur = torch.cuda.current_stream(device)
