@@ -395,7 +395,9 @@ int tbx_batch_last_timing(const tbx_batch *b, double *ms_forward, double *ms_pai
  * (1..64) per work item.  The pairs go into units in bands of *_band
  * consecutive row atoms (1..16), walked column by column, so that a unit
  * covers a few rows i and a run of columns j.  Defaults: forward 256, 128,
- * chunk 3, band 1; gradient 256, 128, chunk 1, band 4.
+ * chunk 3, band 1; gradient 256, 128, chunk 1, band 4, the tasks fewer for a
+ * batch of fewer than 512 such units (down to the largest atom pair), so that
+ * it fills the device; tbx_batch_get_tiles returns what the batch runs.
  * tbx_batch_set_tiles rebuilds the units (host) and waits for the whole
  * device (every stream) before it replaces them, so no launch still reads
  * the old units; tblite_amd/tune.py chooses them by timing the kernels.  A
@@ -433,7 +435,7 @@ typedef struct {
 int tbx_batch_unit_counts(const tbx_batch *b, tbx_unit_counts *n);
 
 /* Work-unit plans of a batch description, built on the host only (no
- * context, no device) with `tiles` (NULL: the defaults), and checked against
+ * context, no device) with `tiles` (NULL: those the batch would start with), and checked against
  * what the kernels assume; no counterpart in the reference (an inspection
  * entry for tests and tooling).  Checked: every atom pair (i, j <= i) of every
  * molecule is in exactly one forward unit and every (i, j < i) in exactly one

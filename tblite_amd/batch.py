@@ -80,7 +80,7 @@ def plan_stats(molecules, tiles: dict | None = None, hint: bool = False,
     on the host (no device): unit, pair, task and element counts, plan bytes,
     and the number of violations of what the kernels assume (``bad_pairs``,
     ``bad_elems``, ``bad_units``; all zero for a correct planner).  ``tiles``
-    as in ``Batch.set_tiles`` (None: the library defaults); ``hint``: order
+    as in ``Batch.set_tiles`` (None: those a ``Batch`` starts with); ``hint``: order
     the pairs near-first by the molecules' own geometry (``Batch.order_pairs``)
     and count the gradient units with a pair inside the cutoff there
     (``nunit_grad_live``)."""

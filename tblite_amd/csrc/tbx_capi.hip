@@ -710,9 +710,9 @@ static void build_forward_launch(const HostSpecies &hs, HostMols &hm,
     }
 }
 
-// Smaller units where the default ones would leave the chip idle: with fewer
-// than TBX_FULL_UNITS units (two workgroups per CU) the task caps shrink until
-// there are that many, down to the largest atom pair.
+// Tiles a batch starts with: smaller units where the default ones would leave the
+// chip idle.  With fewer than TBX_FULL_UNITS units (two workgroups per CU) the
+// task caps shrink until there are that many, down to the largest atom pair.
 #define TBX_FULL_UNITS 512
 static tbx_tiles fill_chip(const HostSpecies &hs, const HostMols &hm, tbx_tiles t)
 {
@@ -727,11 +727,8 @@ static tbx_tiles fill_chip(const HostSpecies &hs, const HostMols &hm, tbx_tiles 
     return t;
 }
 
-// fill: shrink the units of small batches (the tile shapes are the defaults,
-// not a caller's choice)
-static int build_units(const HostSpecies &hs, HostMols &hm, tbx_tiles t, bool fill)
+static int build_units(const HostSpecies &hs, HostMols &hm, const tbx_tiles &t)
 {
-    if (fill) t = fill_chip(hs, hm, t);
     std::vector<char> far, ffar;
     build_units_list(hs, hm, false, t.grad_unit_tasks, t.grad_unit_pairs, t.grad_band, hm.useg,
                      hm.unit_seg, &far);
@@ -1098,7 +1095,6 @@ struct tbx_batch {
     HostSpecies hs;
     HostMols hm;
     tbx_tiles tiles = kDefaultTiles;
-    bool tiles_set = false;  // chosen by the caller (tbx_batch_set_tiles)
     double cutoff = 0.0;  // neighbour cutoff (bohr)
     DevTables tab;
     DevBuf flag, dse_tmp;
@@ -1317,7 +1313,7 @@ static int prepare_single(tbx_context *ctx, const tbx_geom *geom, const tbx_list
     if (!reuse_mols) {
         hm_new.trans.assign(geom->trans, geom->trans + 3 * geom->ntrans);
         hm_new.mol_tr.assign(1, make_int2(0, geom->ntrans));
-        if ((st = build_units(ctx->hs, hm_new, kDefaultTiles, true))) return st;
+        if ((st = build_units(ctx->hs, hm_new, fill_chip(ctx->hs, hm_new, kDefaultTiles)))) return st;
         HIP_TRY(hipStreamSynchronize(s));
         HIP_TRY(upload_mols(ctx->tab, hm_new, s));
         ctx->hm = std::move(hm_new);
@@ -1591,7 +1587,8 @@ static int batch_create(tbx_context *ctx, const tbx_batch_desc *desc, const int 
     }
     hipError_t e = hipSetDevice(ctx->device);
     if (e == hipSuccess) e = upload_species(b->tab, b->hs, desc->cutoff, ctx->stream);
-    if ((st = build_units(b->hs, b->hm, b->tiles, !b->tiles_set))) {
+    b->tiles = fill_chip(b->hs, b->hm, kDefaultTiles);
+    if ((st = build_units(b->hs, b->hm, b->tiles))) {
         tbx_batch_delete(b);
         return st;
     }
@@ -1631,12 +1628,11 @@ extern "C" int tbx_batch_set_tiles(tbx_batch *b, const tbx_tiles *tiles)
 {
     if (!b || !tiles) return fail(TBX_ERR_ARG, "null argument");
     if (int st = check_tiles(b->hs, tiles)) return st;
-    if (int st = build_units(b->hs, b->hm, *tiles, false)) {
-        (void)build_units(b->hs, b->hm, b->tiles, !b->tiles_set);  // keep the host copy of the current units
+    if (int st = build_units(b->hs, b->hm, *tiles)) {
+        (void)build_units(b->hs, b->hm, b->tiles);  // keep the host copy of the current units
         return st;
     }
     b->tiles = *tiles;
-    b->tiles_set = true;
     HIP_TRY(hipSetDevice(b->ctx->device));
     // The batch's kernels run on the callers' streams: wait for every stream
     // of the device, so that no launch still reads the units replaced here.
@@ -1676,10 +1672,10 @@ extern "C" int tbx_batch_order_pairs(tbx_batch *b, const double *xyz, double ski
     const std::vector<double> old_xyz = b->hm.hint_xyz;
     const double old_near2 = b->hm.near2;
     if (int st = set_hint(b->hm, xyz, skin, b->cutoff)) return st;
-    if (int st = build_units(b->hs, b->hm, b->tiles, !b->tiles_set)) {
+    if (int st = build_units(b->hs, b->hm, b->tiles)) {
         b->hm.hint_xyz = old_xyz;  // keep the host copy of the current units
         b->hm.near2 = old_near2;
-        (void)build_units(b->hs, b->hm, b->tiles, !b->tiles_set);
+        (void)build_units(b->hs, b->hm, b->tiles);
         return st;
     }
     HIP_TRY(hipSetDevice(b->ctx->device));
@@ -1762,9 +1758,9 @@ extern "C" int tbx_batch_plan_stats(const tbx_batch_desc *desc, const tbx_tiles 
     if (!st) st = build_mols(hs, desc->nmol, desc->mol_nat, desc->id, hm);
     if (!st) st = set_hint(hm, xyz, skin, desc->cutoff);
     if (st) return st;
-    const tbx_tiles t = tiles ? *tiles : kDefaultTiles;
+    const tbx_tiles t = tiles ? *tiles : fill_chip(hs, hm, kDefaultTiles);
     if ((st = check_tiles(hs, &t))) return st;
-    if ((st = build_units(hs, hm, t, false))) return st;
+    if ((st = build_units(hs, hm, t))) return st;
     tbx_plan_stats s = {};
     s.ndense = hm.ndense;
     s.nunit_fwd = (long long)hm.fhead.size();

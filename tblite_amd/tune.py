@@ -52,7 +52,8 @@ def tune(b, xyz, se, adjoints, plain=None, reps: int = 2, fwd_unit_tasks=FWD_UNI
 
     ``adjoints`` = (Sb, Db, Qb, Hb) times the adjoint kernel; ``plain`` =
     (dsedcn, P, W, vao, vdp, vqp) additionally times the plain gradient
-    kernel (the gradient tile is then chosen on the sum of both).  Returns
+    kernel (the gradient tile is then chosen on the sum of both).  The default
+    task caps are searched together with the batch's own.  Returns
     ``{"tiles": {...}, "table": [...]}`` and leaves the best tiles applied."""
     key = batch_key(b)
     if cache is not None and Path(cache).exists():
@@ -60,6 +61,12 @@ def tune(b, xyz, se, adjoints, plain=None, reps: int = 2, fwd_unit_tasks=FWD_UNI
         if key in known:
             b.set_tiles(**known[key]["tiles"])
             return known[key]
+    # a batch that does not fill the device starts with smaller units than these
+    own = b.tiles()
+    if fwd_unit_tasks is FWD_UNIT_TASKS:
+        fwd_unit_tasks = sorted({own["fwd_unit_tasks"], *FWD_UNIT_TASKS})
+    if grad_unit_tasks is GRAD_UNIT_TASKS:
+        grad_unit_tasks = sorted({own["grad_unit_tasks"], *GRAD_UNIT_TASKS})
     min_tasks = int(max(sum((c.ang + 1) * (c.ang + 2) // 2 for c in sh)
                         for sh in b.spec.basis_cgto)) ** 2
     fwd = [t for t in fwd_unit_tasks if t >= min_tasks]
