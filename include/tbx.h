@@ -363,7 +363,9 @@ int tbx_batch_last_scf_timing(const tbx_batch *b, double *ms);
  * S-orthonormal eigenvectors C, d_eval [nao] with the ascending eigenvalues;
  * d_S is left unchanged (solved on a copy the batch holds).  Synchronises
  * the stream; TBX_ERR_ARG names a molecule whose S is not positive
- * definite.  The workspace (four n x n matrices per molecule solved
+ * definite.  Only the upper triangles are read; an infinity or NaN in a
+ * molecule's H gives NaN for all its eigenvalues and vectors, and TBX_OK.
+ * The workspace (four n x n matrices per molecule solved
  * together, at most 2^24 elements each) shrinks under
  * tbx_context_set_memory_limit; rocSOLVER's own is allocated by rocBLAS and
  * is not counted. */

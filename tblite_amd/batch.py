@@ -331,7 +331,9 @@ class Batch:
     # -- density matrices (scf/diag.f90:62-166, wavefunction/fermi.f90) -----
     def sygvd(self, H, S, eval_out=None):
         """Generalized eigenproblem H C = S C diag(eval) of every molecule:
-        ``H`` (dense, packed) is overwritten with C; returns ``eval`` [nao]."""
+        ``H`` (dense, packed) is overwritten with C; returns ``eval`` [nao].
+        A molecule with an infinity or NaN in H gets NaN results; one whose S
+        is not positive definite is an error."""
         if eval_out is None:
             eval_out = torch.empty(self.nao, dtype=torch.float64, device=self.torch_device)
         L.check(L.lib().tbx_batch_sygvd(self.handle, _ptr(H), _ptr(S), _ptr(eval_out),

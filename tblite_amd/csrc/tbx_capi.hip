@@ -66,6 +66,8 @@ extern "C" hipError_t tbx_launch_fermi(const TbxMols *mol, const double *nel, do
 extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, int nmol,
                                        const EigWork *wk, double *H, const double *S, double *ev,
                                        int *info, hipStream_t s);
+extern "C" hipError_t tbx_launch_eigen_finite(int n, const double *H, int *info, hipStream_t s);
+extern "C" hipError_t tbx_launch_eigen_set(int n, double *H, double *ev, double v, hipStream_t s);
 extern "C" hipError_t tbx_launch_ncoord(const TbxMols *mol, const double *rcov, double ka,
                                         double kb, double rshift, double cutoff,
                                         const double *xyz, double *cn, hipStream_t stream);
@@ -2190,7 +2192,9 @@ extern "C" int tbx_batch_ncoord_gradient(tbx_batch *b, const double *d_xyz,
 }
 
 // The eigenproblem of molecules that the batched kernels do not take, one
-// rocSOLVER call each (S is overwritten by its Cholesky factor: on a copy).
+// rocSOLVER call each (S is overwritten by its Cholesky factor: on a copy).  An
+// infinity or NaN in H is not given to the library: with zeros in its place the
+// library looks at S, and the results are NaN, as the batched kernels'.
 static int sygvd_library(tbx_batch *b, const std::vector<int> &which, double *d_H,
                          const double *d_S, double *d_eval, hipStream_t s)
 {
@@ -2202,18 +2206,27 @@ static int sygvd_library(tbx_batch *b, const std::vector<int> &which, double *d_
     for (int m : which) nn = std::max(nn, (size_t)b->hm.mol_nao[m] * b->hm.mol_nao[m]);
     HIP_TRY(b->sy_b.reserve(sizeof(double) * nn));
     HIP_TRY(b->sy_e.reserve(sizeof(double) * (size_t)std::max(1, b->hm.nao)));
+    for (int m : which)
+        HIP_TRY(tbx_launch_eigen_finite(b->hm.mol_nao[m], d_H + b->hm.mol_dense[m],
+                                        b->sy_info.as<int>() + m, s));
+    std::vector<int> info(b->hm.nmol);
+    HIP_TRY(hipMemcpyAsync(info.data(), b->sy_info.p, sizeof(int) * info.size(),
+                           hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipStreamSynchronize(s));
     for (int m : which) {
         const int n = b->hm.mol_nao[m];
-        const long long d0 = b->hm.mol_dense[m];
-        const int a0 = b->hm.mol_ao[m];
-        HIP_TRY(hipMemcpyAsync(b->sy_b.p, d_S + d0, sizeof(double) * (size_t)n * n,
+        double *H = d_H + b->hm.mol_dense[m], *ev = d_eval + b->hm.mol_ao[m];
+        const bool finite = info[m] == 0;
+        if (!finite) HIP_TRY(tbx_launch_eigen_set(n, H, ev, 0.0, s));
+        HIP_TRY(hipMemcpyAsync(b->sy_b.p, d_S + b->hm.mol_dense[m], sizeof(double) * (size_t)n * n,
                                hipMemcpyDeviceToDevice, s));
         const rocblas_status st = rocsolver_dsygvd(
-            b->solver, rocblas_eform_ax, rocblas_evect_original, rocblas_fill_upper, n, d_H + d0,
-            n, b->sy_b.as<double>(), n, d_eval + a0, b->sy_e.as<double>() + a0,
+            b->solver, rocblas_eform_ax, rocblas_evect_original, rocblas_fill_upper, n, H, n,
+            b->sy_b.as<double>(), n, ev, b->sy_e.as<double>() + b->hm.mol_ao[m],
             b->sy_info.as<rocblas_int>() + m);
         if (st != rocblas_status_success)
             return fail(TBX_ERR_DEVICE, "rocsolver_dsygvd (molecule %d): status %d", m, (int)st);
+        if (!finite) HIP_TRY(tbx_launch_eigen_set(n, H, ev, std::nan(""), s));
     }
     return TBX_OK;
 }

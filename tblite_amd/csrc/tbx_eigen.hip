@@ -1760,7 +1760,45 @@ hipError_t allow_lds(F f, size_t bytes)
                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
+// Molecules of the library route: info = TBX_EIG_NONFINITE for an infinity or
+// NaN in the upper triangle of H, a wavefront per column
+__global__ void __launch_bounds__(256) k_eig_finite(int n, const double *H, int *info)
+{
+    const int c = 4 * blockIdx.x + (threadIdx.x >> 6);
+    if (c >= n) return;
+    bool bad = false;
+    for (int r = threadIdx.x & 63; r <= c; r += 64) {
+        const int hi = __double2hiint(H[r + (long long)c * n]) & 0x7fffffff;
+        bad = bad || hi >= 0x7ff00000;
+    }
+    if (__any(bad) && (threadIdx.x & 63) == 0) *info = TBX_EIG_NONFINITE;
+}
+
+__global__ void __launch_bounds__(256) k_eig_set(int n, double *H, double *ev, double v)
+{
+    for (int r = threadIdx.x; r < n; r += 256) H[r + (long long)blockIdx.x * n] = v;
+    if (threadIdx.x == 0) ev[blockIdx.x] = v;
+}
+
 } // namespace
+
+// info[0] <- TBX_EIG_NONFINITE for an infinity or NaN in the upper triangle of H, else 0
+extern "C" hipError_t tbx_launch_eigen_finite(int n, const double *H, int *info, hipStream_t s)
+{
+    const hipError_t e = hipMemsetAsync(info, 0, sizeof(int), s);  // the solver waits: no capture
+    if (e != hipSuccess) return e;
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_eig_finite, dim3((n + 3) / 4), dim3(256), 0, s, n, H, info);
+    return hipGetLastError();
+}
+
+// every element of H [n * n] and ev [n] <- v
+extern "C" hipError_t tbx_launch_eigen_set(int n, double *H, double *ev, double v, hipStream_t s)
+{
+    (void)hipGetLastError();
+    hipLaunchKernelGGL(k_eig_set, dim3(n), dim3(256), 0, s, n, H, ev, v);
+    return hipGetLastError();
+}
 
 // The molecules mols[0 .. nmol) (device; nmax .. nmin orbitals, descending):
 // H and S are the batch's dense arrays, wb the workspace (EigWork).
