@@ -313,6 +313,9 @@ __device__ bool factor_inverse(double (*T)[PR], double (*buf)[2 * NB], double *p
 // factor and inverse, so a block column is one launch.  kb = -1: the first
 // diagonal block only.  768 orbitals: 33 us a launch, about half of it the
 // chain of 64 eliminations (60 us with loads one at a time and unmasked rows).
+// A molecule whose S has failed goes on, into values that nobody reads: one
+// workgroup of the launch writes its info, so a look at it here could send the
+// wavefronts of another to different sides of a barrier.
 __global__ void __launch_bounds__(256) k_eig_chol(const EigMol *mols, double *A, double *L,
                                                   int kb, int *info)
 {
@@ -324,7 +327,6 @@ __global__ void __launch_bounds__(256) k_eig_chol(const EigMol *mols, double *A,
     int tj = 0, rest = blockIdx.x;  // tile column tj: left - tj tiles
     while (tj < left && rest >= left - tj) rest -= left - tj++;
     if (tj >= left || (kb < 0 && blockIdx.x > 0)) return;
-    if (info[M.mol] != 0) return;
     const int bj = kb + 1 + tj, bi = bj + rest;
     double *Am = A + M.w0, *Lm = L + M.w0;
     const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
