@@ -1691,7 +1691,7 @@ extern "C" int tbx_batch_order_pairs(tbx_batch *b, const double *xyz, double ski
 }
 
 // Up to TBX_HINT_UNITS units a hint is not worth its launches: every unit fits
-// the chip at once (three workgroups per CU), so the distant ones cost nothing
+// the chip at once (three or four workgroups per CU), so the distant ones cost nothing
 // (they end after their pair vectors), and the check of the hint and the launch
 // of the far units would be most of the overhead.  Forward and adjoint without
 // and with a hint: n-octane (86 units) 45 and 55 us, 96 waters (663) 74 and 80,

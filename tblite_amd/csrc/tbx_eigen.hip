@@ -949,7 +949,7 @@ __device__ __forceinline__ void sibling_zero(double *Q, int n, int lev, int s, i
 // Leaves: one workgroup solves a segment of at most 64 rows by merges from
 // single rows, everything in LDS.  Four lanes per entry; at each level all
 // merges of the segment run together.  Bound by the chain of its phases, the
-// roots first: 98 us for 50 rows (222 us with a serial deflation pass and the
+// roots first: 91 us for 50 rows (222 us with a serial deflation pass and the
 // vectors' products on the vector unit).
 constexpr int LN = TBX_DC_LEAF;
 constexpr int LQ = LN + 1;
@@ -1803,7 +1803,7 @@ extern "C" hipError_t tbx_launch_eigen_set(int n, double *H, double *ev, double 
 }
 
 // The molecules mols[0 .. nmol) (device; nmax .. nmin orbitals, descending):
-// H and S are the batch's dense arrays, wb the workspace (EigWork).
+// H, S and ev are the batch's dense and orbital arrays, wk the workspace.
 extern "C" hipError_t tbx_launch_eigen(const EigMol *mols, const int *n_host, int nmol,
                                        const EigWork *wk, double *H, const double *S, double *ev,
                                        int *info, hipStream_t s)

@@ -47,14 +47,14 @@ def _batch(kind):
     if kind == "crystals":
         mols, lats = _crystals()
         return Batch(mols, lattices=lats)
-    if kind == "rounds":  # more far units than a launch looks at in one round (2048 x 16)
+    if kind == "passes":  # more far units than a launch looks at in one pass (2048 x 16)
         b = Batch([synthetic.water_cluster(256, seed=5)])
         b.set_tiles(fwd_unit_pairs=4, grad_unit_pairs=4)
         return b
     return Batch(_structures(), diat_scale=_ones if kind == "diatomic" else None)
 
 
-@pytest.mark.parametrize("kind", ["molecules", "crystals", "diatomic", "rounds"])
+@pytest.mark.parametrize("kind", ["molecules", "crystals", "diatomic", "passes"])
 @pytest.mark.parametrize("stale", [False, True])
 def test_hint_in_effect(kind, stale):
     b = _batch(kind)
@@ -81,11 +81,11 @@ def test_hint_in_effect(kind, stale):
     ref = [r.clone() for r in run()]
     hint = b.xyz0.copy()
     if stale:
-        hint[: 1 if kind != "rounds" else b.nat // 2] += 30.0  # near pairs end up in far units
+        hint[: 1 if kind != "passes" else b.nat // 2] += 30.0  # near pairs end up in far units
     b.order_pairs(hint, skin=0.5)
     n = b.unit_counts()
     print(f"[gpu] hint {kind} stale {stale}: {n}", flush=True)
-    least = 2048 * 16 if kind == "rounds" else 0
+    least = 2048 * 16 if kind == "passes" else 0
     assert n["fwd_far"] > least and n["grad_far"] > least
     for _ in range(2):
         for k, (r, g) in enumerate(zip(ref, run())):
