@@ -501,13 +501,13 @@ __device__ __forceinline__ void pair_vec(const TbxMols &mt, const double *xyz, c
 }
 
 // Far units, for a hint that no longer holds: most still have no pair within the
-// cutoff.  A wavefront looks at the pairs of FAR_LOOK units (their atoms alone,
-// straight from the plan), a workgroup at FAR_UNITS, dealt to the workgroups in
-// turn, and `run` takes those that may have one (the margin is rounding's: a unit
-// screens its pairs itself).  Units next to each other in one workgroup leave
-// the living ones to a few: the adjoint of 8 clusters of 200 to 500 atoms, all
-// displaced by 0.5 bohr, 211 against 181 us.
-constexpr int FAR_LOOK = 4, FAR_UNITS = 4 * FAR_LOOK;  // four wavefronts
+// cutoff.  A wavefront looks at the pairs of one unit (their atoms alone, straight
+// from the plan), a workgroup at FAR_UNITS, dealt to the workgroups in turn, and
+// `run` takes those that may have one (the margin is rounding's: a unit screens
+// its pairs itself).  Four units a wavefront instead of one leave more living ones
+// to a workgroup: the gradient of 8 clusters of 200 to 500 atoms, all displaced
+// by 0.5 bohr, 195 against 186 us; 16 neighbours of the list 213.
+constexpr int FAR_UNITS = 4;  // wavefronts
 
 __device__ __forceinline__ bool unit_lives(const TbxMols &mt, const TbxUnitHead &H,
                                            const int *plan, const double *xyz, double cutoff2)
@@ -535,12 +535,9 @@ __device__ __forceinline__ void far_units(const TbxMols &mt, const TbxUnitHead *
     __shared__ int lives[FAR_UNITS];
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), step = gridDim.x;
     for (int u0 = blockIdx.x; u0 < n; u0 += FAR_UNITS * step) {
-#pragma unroll
-        for (int k = 0; k < FAR_LOOK; ++k) {
-            const int q = FAR_LOOK * wv + k, u = u0 + q * step;
-            const bool live = u < n && unit_lives(mt, units[u], plan, xyz, cutoff2);
-            if ((threadIdx.x & 63) == 0) lives[q] = live;
-        }
+        const int mine = u0 + wv * step;
+        const bool live = mine < n && unit_lives(mt, units[mine], plan, xyz, cutoff2);
+        if ((threadIdx.x & 63) == 0) lives[wv] = live;
         __syncthreads();
         for (int q = 0; q < FAR_UNITS; ++q)
             if (lives[q]) {
@@ -1020,8 +1017,7 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
     double v[3];
     const int pl = tid < npair ? tid : 0;
     pair_vec(mt, A.xyz, U.pinf[pl], U.pext[pl], v);
-    ShellLoad sl;
-    if (!FAR) sl = shell_load(sp, U, A.se, tid < nspair ? tid : 0);
+    const ShellLoad sl = shell_load(sp, U, A.se, tid < nspair ? tid : 0);
     if (tid < npair) {
 #pragma unroll
         for (int c = 0; c < 3; ++c) U.pv[tid][c] = v[c];
@@ -1045,7 +1041,6 @@ __device__ __forceinline__ void forward_unit(const FwdArgs &A, const TbxUnitHead
         if (!FAR && !accum) far_zero_unit(A, H, U, eoff);
         return;
     }
-    if (FAR) sl = shell_load(sp, U, A.se, tid < nspair ? tid : 0);
     // shell pairs: screening counts and H0 factors (one lane per shell pair)
     if (tid < nspair) {
         const int k = tid;
@@ -1262,12 +1257,13 @@ __global__ void __launch_bounds__(NTHREADS, 2) k_forward(FwdArgs A)
 // The forward units of the pairs beyond cutoff + skin at the hint, when an
 // atom has left it (as k_gradient_far).  Their elements are zero by the zero
 // units of k_forward; a unit with a pair within the cutoff writes them anew.
-// Forward of 640 molecules of 8 to 256 atoms with one atom moved by 1 bohr 1593
-// us, all displaced by 0.5 bohr 1662 (hint valid: 1550); with every far unit
-// staged here and its zeros written by it 2142 and 2140; with a hint stretched
-// threefold, most units alive, 2911 and 2622.  (H2O)512, one atom: 211 and 347.
-// The loop keeps the unit's constants in registers, 178 without a bound (236 with
-// DIAT, 40 spilled to fit three wavefronts): at three wavefronts 2911, two 3224.
+// Forward of 640 molecules of 8 to 256 atoms with one atom moved by 1 bohr 1894
+// us, all displaced by 0.5 bohr 1972 (hint valid: 1861); with every far unit
+// staged here and its zeros written by it 2445 and 2442; with a hint stretched
+// threefold, most units alive, 3400 and 2730: zeros are written over.  (H2O)512,
+// one atom: 268 and 476.  The loop keeps the unit's constants in registers, more
+// than 168 without a bound (243 with DIAT, spilled under one): the threefold hint
+// 2911 at three wavefronts and 3224 at two (valid: 1550, on another placement).
 template <bool DIAT>
 __global__ void __launch_bounds__(NTHREADS, DIAT ? 2 : 3) k_forward_far(FwdArgs A)
 {
@@ -2085,7 +2081,7 @@ __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient(GradArgs A)
 // position (every answer of k_begin 0), since then every such pair is
 // still beyond the cutoff.  Otherwise the workgroups look through them: 640
 // molecules of 8 to 256 atoms with one atom moved by 1 bohr, adjoint given S and
-// D 1635 us, 1769 with every far unit staged (hint valid: 1575).
+// D 1636 us, 1772 with every far unit staged (hint valid: 1582).
 template <int MODE, bool EX>
 __global__ void __launch_bounds__(GTHREADS, EX ? 2 : 3) k_gradient_far(GradArgs A,
                                                                      const int *stale, int nstale)

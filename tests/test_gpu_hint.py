@@ -47,7 +47,7 @@ def _batch(kind):
     if kind == "crystals":
         mols, lats = _crystals()
         return Batch(mols, lattices=lats)
-    if kind == "passes":  # more far units than a launch looks at in one pass (2048 x 16)
+    if kind == "passes":  # more far units than a launch looks at in one pass (2048 x 4)
         b = Batch([synthetic.water_cluster(256, seed=5)])
         b.set_tiles(fwd_unit_pairs=4, grad_unit_pairs=4)
         return b
@@ -85,7 +85,7 @@ def test_hint_in_effect(kind, stale):
     b.order_pairs(hint, skin=0.5)
     n = b.unit_counts()
     print(f"[gpu] hint {kind} stale {stale}: {n}", flush=True)
-    least = 2048 * 16 if kind == "passes" else 0
+    least = 2048 * 4 if kind == "passes" else 0
     assert n["fwd_far"] > least and n["grad_far"] > least
     for _ in range(2):
         for k, (r, g) in enumerate(zip(ref, run())):
